@@ -126,6 +126,14 @@ typedef struct {
     float eps;
 } qw_linear_desc;
 int qw_gpu_linear(h3_gpu *gpu, const qw_linear_desc *desc);
+/* The SwiGLU MLP's first linear and its activation in one launch: weight
+ * [2F, k] = [gate | up] rows, cols = 2F (a multiple of 16), out [rows, F] at
+ * stride ldc >= F: bf16(bf16(silu(g)) * u) with g, u the linear's bf16
+ * results, as qw_gpu_linear followed by qw_gpu_swiglu_bf16 (8 rows or fewer
+ * run as those two, into a whole [rows, F] output at offset 0). epilogue must
+ * be QW_LINEAR_STORE. No counterpart in the reference, which runs two
+ * kernels. */
+int qw_gpu_linear_swiglu(h3_gpu *gpu, const qw_linear_desc *desc);
 /* No counterpart in the reference. For callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc): qw_gpu_linear with every workspace in

@@ -25,13 +25,13 @@
 enum {
     K_LN_MOD, K_RMS_ONE, K_QK_NORM_ROPE, K_GATE, K_ACT, K_SWIGLU, K_CAST,
     K_REORDER, K_FILL, K_QUANT, K_DEQUANT, K_COPY2D, K_ATTN,
-    /* GEMM kernels in QW_LINEAR_* epilogue order (store, gelu, gate, qknorm) */
-    K_GEMM_BF16_STORE_Q, K_GEMM_BF16_GELU_Q, K_GEMM_BF16_GATE_Q, K_GEMM_BF16_QKN_Q,
+    /* GEMM kernels in QW_EPI_* order (store, gelu, gate, qknorm, swiglu) */
+    K_GEMM_BF16_STORE_Q, K_GEMM_BF16_GELU_Q, K_GEMM_BF16_GATE_Q, K_GEMM_BF16_QKN_Q, K_GEMM_BF16_SWIGLU_Q,
     K_WIDEN, K_LN_MOD_WIDE, K_EULER, K_LORA,
     K_GEMV_BF16_STORE, K_GEMV_BF16_GELU, K_GEMV_I8_STORE, K_GEMV_I8_GELU, K_ZERO,
-    K_GEMM_W8_STORE_Q, K_GEMM_W8_GELU_Q, K_GEMM_W8_GATE_Q, K_GEMM_W8_QKN_Q,
-    K_GEMM_BF16_STORE_T224, K_GEMM_BF16_GELU_T224, K_GEMM_BF16_GATE_T224, K_GEMM_BF16_QKN_T224,
-    K_GEMM_BF16_STORE_H3, K_GEMM_BF16_GELU_H3, K_GEMM_BF16_GATE_H3, K_GEMM_BF16_QKN_H3,
+    K_GEMM_W8_STORE_Q, K_GEMM_W8_GELU_Q, K_GEMM_W8_GATE_Q, K_GEMM_W8_QKN_Q, K_GEMM_W8_SWIGLU_Q,
+    K_GEMM_BF16_STORE_T224, K_GEMM_BF16_GELU_T224, K_GEMM_BF16_GATE_T224, K_GEMM_BF16_QKN_T224, K_GEMM_BF16_SWIGLU_T224,
+    K_GEMM_BF16_STORE_H3, K_GEMM_BF16_GELU_H3, K_GEMM_BF16_GATE_H3, K_GEMM_BF16_QKN_H3, K_GEMM_BF16_SWIGLU_H3,
     K_ATTN_W4,
     K_COUNT
 };
@@ -40,16 +40,16 @@ static const char *k_names[K_COUNT] = {
     "qw_gate_bf16", "qw_act_bf16", "qw_swiglu_bf16", "qw_cast_f32_bf16",
     "qw_modulation_reorder_bf16", "qw_fill_normal_bf16", "qw_quantize_int8_rows",
     "qw_dequant_int8_f32", "qw_copy2d", "qw_attention_bf16",
-    "qw_gemm_bf16_store_q", "qw_gemm_bf16_gelu_q", "qw_gemm_bf16_gate_q", "qw_gemm_bf16_qkn_q",
+    "qw_gemm_bf16_store_q", "qw_gemm_bf16_gelu_q", "qw_gemm_bf16_gate_q", "qw_gemm_bf16_qkn_q", "qw_gemm_bf16_swiglu_q",
     "qw_widen_i8_bf16",
     "qw_layer_norm_mod_wide_bf16", "qw_cfg_euler_f32", "qw_lora_fuse_bf16",
     "qw_gemv_bf16_store", "qw_gemv_bf16_gelu", "qw_gemv_i8_store", "qw_gemv_i8_gelu",
     "qw_zero_u32",
-    "qw_gemm_w8_store_q", "qw_gemm_w8_gelu_q", "qw_gemm_w8_gate_q", "qw_gemm_w8_qkn_q",
+    "qw_gemm_w8_store_q", "qw_gemm_w8_gelu_q", "qw_gemm_w8_gate_q", "qw_gemm_w8_qkn_q", "qw_gemm_w8_swiglu_q",
     "qw_gemm_bf16_store_t224", "qw_gemm_bf16_gelu_t224", "qw_gemm_bf16_gate_t224",
-    "qw_gemm_bf16_qkn_t224",
+    "qw_gemm_bf16_qkn_t224", "qw_gemm_bf16_swiglu_t224",
     "qw_gemm_bf16_store_h3", "qw_gemm_bf16_gelu_h3", "qw_gemm_bf16_gate_h3",
-    "qw_gemm_bf16_qkn_h3", "qw_attention_w4_bf16"};
+    "qw_gemm_bf16_qkn_h3", "qw_gemm_bf16_swiglu_h3", "qw_attention_w4_bf16"};
 
 /* How int8 linears run (QW_INT8_ROUTE, a measurement switch): AUTO (the
  * default) widens the weight to a bf16 copy and runs the bf16 kernels when
@@ -1024,13 +1024,15 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc) {
     if (d->lda % 8 || d->in_offset % 8 || d->lda < d->k)
         return fail(g, "linear: input rows must be 16-byte aligned (lda %u, offset %zu)", d->lda,
                     d->in_offset);
-    if (d->ldc < d->cols) return fail(g, "linear: ldc < cols");
-    if (d->cols % 8 || d->ldc % 4 || d->out_offset % 4)
+    const int glu = d->epilogue == QW_EPI_SWIGLU; /* cols = 2 F, output [rows, F] */
+    const uint32_t out_cols = glu ? d->cols / 2 : d->cols;
+    if (d->ldc < out_cols) return fail(g, "linear: ldc < cols");
+    if (out_cols % 8 || (glu && d->cols % 16) || d->ldc % 4 || d->out_offset % 4)
         return fail(g, "linear: cols (%u) must be a multiple of 8 and output rows 8-byte aligned",
                     d->cols);
     if (!fits(d->in, d->in_offset, (size_t)(d->rows - 1) * d->lda + d->k))
         return fail(g, "linear: input too small");
-    if (!fits(d->out, d->out_offset, (size_t)(d->rows - 1) * d->ldc + d->cols))
+    if (!fits(d->out, d->out_offset, (size_t)(d->rows - 1) * d->ldc + out_cols))
         return fail(g, "linear: output too small");
     if (!fits(d->weight, 0, (size_t)d->cols * d->k)) return fail(g, "linear: weight too small");
     if ((uint64_t)d->cols * d->k >= (1ull << 32) || (uint64_t)d->rows * d->lda >= (1ull << 32))
@@ -1069,7 +1071,7 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc) {
         if (((uintptr_t)d->norm_q->ptr | (uintptr_t)d->norm_k->ptr | (uintptr_t)d->rope_cos->ptr |
              (uintptr_t)d->rope_sin->ptr | (uintptr_t)d->out->ptr) % 16)
             return fail(g, "linear qk: tensors must be 16-byte aligned");
-    } else if (d->epilogue != QW_LINEAR_STORE && d->epilogue != QW_LINEAR_GELU) {
+    } else if (d->epilogue != QW_LINEAR_STORE && d->epilogue != QW_LINEAR_GELU && !glu) {
         return fail(g, "linear: unknown epilogue %d", d->epilogue);
     }
     if (d->epilogue == QW_LINEAR_QKNORM && d->rope_rows < 128) {
@@ -1176,7 +1178,7 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc) {
     {
         const uint64_t ab = ((uint64_t)(d->rows - 1) * d->lda + d->k) * 2;
         const uint64_t wb = (uint64_t)d->cols * d->k * (int8 && !widen ? 1 : 2);
-        const uint64_t ob = ((uint64_t)(d->rows - 1) * d->ldc + d->cols) * 2;
+        const uint64_t ob = ((uint64_t)(d->rows - 1) * d->ldc + out_cols) * 2;
         if (ab >= (1ull << 31) || wb >= (1ull << 31) || ob >= (1ull << 31))
             return fail(g, "linear: operand exceeds 2 GiB buffer range");
         a.a_bytes = (uint32_t)ab;
@@ -1327,11 +1329,44 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc) {
     return launch(g, kid, dim3(grid), dim3(threads), a);
 }
 
-extern "C" int qw_gpu_linear(h3_gpu *g, const qw_linear_desc *d) { return linear_impl(g, d, 0); }
+static int check_epilogue(h3_gpu *g, const qw_linear_desc *d) {
+    if (d && (d->epilogue < QW_LINEAR_STORE || d->epilogue > QW_LINEAR_QKNORM))
+        return fail(g, "linear: unknown epilogue %d", d->epilogue);
+    return 1;
+}
+
+extern "C" int qw_gpu_linear(h3_gpu *g, const qw_linear_desc *d) {
+    return check_epilogue(g, d) ? linear_impl(g, d, 0) : 0;
+}
+
+/* The tile kernels from 9 rows on; fewer rows keep the streaming linear and
+ * the separate pass over its few rows, in the runtime's scratch buffer. */
+static void *scratch(h3_gpu *g, size_t bytes);
+extern "C" int qw_gpu_linear_swiglu(h3_gpu *g, const qw_linear_desc *d) {
+    if (!g || !d) return 0;
+    if (!check_epilogue(g, d)) return 0;
+    if (d->epilogue != QW_LINEAR_STORE) return fail(g, "linear_swiglu: epilogue must be STORE");
+    qw_linear_desc t = *d;
+    if (d->rows > 8) {
+        t.epilogue = QW_EPI_SWIGLU;
+        return linear_impl(g, &t, 0);
+    }
+    if (!d->rows || !d->cols) return 1;
+    if (d->cols % 16 || d->ldc != d->cols / 2 || d->out_offset)
+        return fail(g, "linear_swiglu: at most 8 rows go to a whole [rows, cols / 2] output");
+    const size_t wide = (size_t)d->rows * d->cols;
+    void *s = scratch(g, wide * 2);
+    if (!s) return fail(g, "linear_swiglu: scratch allocation failed");
+    h3_gpu_tensor tw = {g, (unsigned char *)s, wide, H3_GPU_BF16, 0};
+    t.out = &tw;
+    t.ldc = d->cols;
+    return linear_impl(g, &t, 0) && qw_gpu_swiglu_bf16(g, d->out, &tw, d->rows, d->cols / 2);
+}
 
 extern "C" int qw_gpu_linear_static(h3_gpu *g, const qw_linear_desc *d) {
     if (!g) return 0;
     if (!g->static_scratch) return fail(g, "linear_static: no static workspace");
+    if (!check_epilogue(g, d)) return 0;
     /* every context on this device shares the workspace: this call's
      * kernels wait for the last call that used it, from any stream */
     hipError_t e = (hipError_t)qw_static_scratch_acquire(g->device, g->stream);
@@ -1394,6 +1429,16 @@ extern "C" int h3_gpu_mlp_bf16(h3_gpu *g, h3_gpu_tensor *out, const h3_gpu_tenso
                                uint32_t rows, uint32_t in_dim, uint32_t hidden,
                                uint32_t out_dim) {
     size_t wide = (size_t)rows * hidden * 2, act_n = (size_t)rows * hidden;
+    if (rows > 8 && hidden % 8 == 0) { /* one launch for fc1 and the activation */
+        unsigned char *s = (unsigned char *)scratch(g, act_n * 2);
+        if (!s) return fail(g, "mlp: scratch allocation failed");
+        if (!fc1 || fc1->dtype != H3_GPU_BF16) return fail(g, "linear_bf16: weight must be bf16");
+        h3_gpu_tensor ta = {g, s, act_n, H3_GPU_BF16, 0};
+        qw_linear_desc d = plain_linear(&ta, in, fc1, NULL, rows, in_dim, 2 * hidden);
+        d.ldc = hidden;
+        return qw_gpu_linear_swiglu(g, &d) &&
+               h3_gpu_linear_bf16(g, out, &ta, fc2, NULL, rows, hidden, out_dim);
+    }
     unsigned char *s = (unsigned char *)scratch(g, (wide + act_n) * 2 + 512);
     if (!s) return fail(g, "mlp: scratch allocation failed");
     h3_gpu_tensor tw = {g, s, wide, H3_GPU_BF16, 0};

@@ -401,6 +401,111 @@ __device__ __forceinline__ void gemm_epilogue_mode(const qw_gemm_args &a, SlabWr
     }
 }
 
+/* SwiGLU (EPI_SWIGLU): the wave's 128 columns are the gate rows f0..f0 + 63
+ * of W, then the up rows F + f0..F + f0 + 63 (qg_wrow), so one lane finds a
+ * gate and its up value 64 staged columns apart: 8 lanes per output row, 8
+ * output columns (one 16-byte store) per lane, 8 rows per pass. The same
+ * rounding points as the linear followed by qw_swiglu_bf16: g and u to bf16,
+ * silu(g) to bf16, the product to bf16.
+ *
+ * Fused because the separate pass writes and re-reads the [M, 2F] linear
+ * output: at M = 4119, F = 12288 the pass took 120-123 us after a 625 us
+ * linear that also had twice the output to store.
+ *
+ * MODE 0: a finished tile; MODE 2: the last piece of a split tile, which
+ * adds all pieces' sums in piece order. read_half(lr, half, v): this lane's
+ * 8 sums of gate (half 0) or up (half 1) columns of staged row lr. */
+template <int INT8, int NSLAB, int SR, int MODE, class SlabWriter, class HalfReader>
+__device__ __forceinline__ void gemm_epilogue_swiglu(const qw_gemm_args &a, SlabWriter write_slab,
+                                                     HalfReader read_half, uint32_t row0,
+                                                     uint32_t f0, uint32_t lane,
+                                                     const float *pld, uint32_t npart,
+                                                     uint32_t own) {
+#pragma clang fp contract(off)
+    const bool scaled = INT8 || a.wscale != nullptr;
+    const __amdgpu_buffer_rsrc_t part_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)a.sk_part, (short)0, (int)0x7FFFFFF0, 0x00020000);
+    const __amdgpu_buffer_rsrc_t out_rsrc =
+        __builtin_amdgcn_make_buffer_rsrc((void *)a.out, (short)0, (int)a.out_bytes, 0x00020000);
+    const uint32_t F = a.n / 2, rr = lane >> 3, cc = lane & 7;
+    const uint32_t col = f0 + cc * 8;
+    const bool col_ok = col < F;             /* F % 8 == 0 */
+    const uint32_t colc = col_ok ? col : F - 8; /* in-range column for operand loads */
+    float sc[2][8], bias[2][8];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) sc[h][j] = 1.0f, bias[h][j] = 0.0f;
+        if (scaled) {
+            const floatx4 s0 = *(const floatx4 *)(a.wscale + h * F + colc);
+            const floatx4 s1 = *(const floatx4 *)(a.wscale + h * F + colc + 4);
+#pragma unroll
+            for (int j = 0; j < 4; j++) sc[h][j] = s0[j], sc[h][4 + j] = s1[j];
+        }
+        if (a.bias) {
+            const u32x4 bb = *(const u32x4 *)(a.bias + h * F + colc);
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                bias[h][2 * j] = lo_bf(bb[j]), bias[h][2 * j + 1] = hi_bf(bb[j]);
+        }
+    }
+#pragma unroll
+    for (int mi = 0; mi < NSLAB; mi++) {
+        write_slab(mi);
+#pragma unroll
+        for (int p = 0; p < SR / 8; p++) {
+            const uint32_t lr = 8 * p + rr, row = row0 + mi * SR + lr;
+            const uint32_t ooff = col_ok && row < a.m ? (row * a.ldc + col) * 2 : 0x80000000u;
+            float y[2][8];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                if (MODE == 0) {
+                    read_half(lr, h, y[h]);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 8; j++) y[h][j] = 0.0f;
+                    for (uint32_t pc = 0; pc < npart; pc++) {
+                        float v[8];
+                        if (pc == own) {
+                            read_half(lr, h, v);
+                        } else {
+                            const uint32_t poff = (mi * SR + lr) * 256 + h * 64 + cc * 8;
+                            const uint32_t bo =
+                                (uint32_t)((pld - a.sk_part) + pc * QW_SPLIT_PART + poff) * 4;
+                            const floatx4 q0 = __builtin_bit_cast(
+                                floatx4, __builtin_amdgcn_raw_buffer_load_b128(part_rsrc, bo, 0,
+                                                                               QW_CPOL_COHERENT));
+                            const floatx4 q1 = __builtin_bit_cast(
+                                floatx4, __builtin_amdgcn_raw_buffer_load_b128(
+                                             part_rsrc, bo + 16, 0, QW_CPOL_COHERENT));
+#pragma unroll
+                            for (int j = 0; j < 4; j++) v[j] = q0[j], v[4 + j] = q1[j];
+                        }
+#pragma unroll
+                        for (int j = 0; j < 8; j++) y[h][j] += v[j];
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < 8; j += 2) {
+                    const float t0 = y[h][j] * sc[h][j], t1 = y[h][j + 1] * sc[h][j + 1];
+                    const uint32_t w = pack_bf(t0 + bias[h][j], t1 + bias[h][j + 1]);
+                    y[h][j] = lo_bf(w);
+                    y[h][j + 1] = hi_bf(w);
+                }
+            }
+            uint32_t pk[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t g =
+                    pack_bf(silu_fast_f(y[0][2 * j]), silu_fast_f(y[0][2 * j + 1]));
+                pk[j] = pack_bf(lo_bf(g) * y[1][2 * j], hi_bf(g) * y[1][2 * j + 1]);
+            }
+            __builtin_amdgcn_raw_buffer_store_b128(u32x4{pk[0], pk[1], pk[2], pk[3]}, out_rsrc,
+                                                   ooff, 0, QW_CPOL_NT);
+        }
+    }
+}
+
 template <int EPI, int INT8, int NSLAB, int SR, int RP, class SlabWriter, class SlabReader>
 __device__ __forceinline__ void gemm_epilogue_lds(const qw_gemm_args &a, SlabWriter write_slab,
                                                   SlabReader read_row, uint32_t row0,

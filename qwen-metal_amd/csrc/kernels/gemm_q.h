@@ -75,6 +75,17 @@ __device__ __forceinline__ void qg_ready(const bf16x8 (&f)[8]) {
                      "v"(f[6]));
 }
 
+/* Row of W that row r of the tile's 256-row W stage holds (columns n0 + r of
+ * the output, clamped). GLU (EPI_SWIGLU, W = [gate | up], n = 2F): the tile
+ * covers 128 output columns from n0 / 2; each wave column's 128 stage rows
+ * are 64 gate rows, then the up rows of the same 64 output columns. */
+template <bool GLU>
+__device__ __forceinline__ uint32_t qg_wrow(const qw_gemm_args &a, uint32_t n0, uint32_t r) {
+    if (!GLU) return min(n0 + r, a.n - 1);
+    const uint32_t F = a.n / 2;
+    return min(n0 / 2 + (r >> 7) * 64 + (r & 63u), F - 1) + ((r >> 6) & 1u) * F;
+}
+
 /* fragment j of a sub-step, in the order its MFMAs consume them (W block 0,
  * A blocks 0..MB-1, W blocks 1-7) */
 template <int MB = 8, int AB = QG_A_BYTES>
@@ -154,7 +165,7 @@ __device__ __forceinline__ void qg_slice(const QgCtx &c, floatx4 (&acc)[8][8], b
 /* Sums of tile (tm, tn) over k-steps [kb, ke) into acc; ends with the LDS
  * stages free (after a barrier). MB = 8: 256-row tiles; MB = 7: 224-row
  * tiles (each wave's 112 rows; the A stage's last 32 rows unused). */
-template <int MB = 8>
+template <int MB = 8, bool GLU = false>
 __device__ __forceinline__ void qg_mainloop(const qw_gemm_args &a, unsigned char *lds,
                                             unsigned char *lds_b, uint32_t tm, uint32_t tn,
                                             uint32_t kb, uint32_t ke, floatx4 (&acc)[8][8]) {
@@ -170,7 +181,7 @@ __device__ __forceinline__ void qg_mainloop(const qw_gemm_args &a, unsigned char
         const uint32_t ra = wave * (MB * 8) + j * 8 + lrow; /* A row: 8 MB rows per wave */
         if (j < MB)
             c.a_dvoff[j] = (min(m0 + ra, a.m - 1) * a.lda + (lp ^ ((ra >> 1) & 7u)) * 8) * 2;
-        c.w_dvoff[j] = (min(n0 + r, a.n - 1) * a.k + (lp ^ ((r >> 1) & 7u)) * 8) * 2;
+        c.w_dvoff[j] = (qg_wrow<GLU>(a, n0, r) * a.k + (lp ^ ((r >> 1) & 7u)) * 8) * 2;
     }
     c.a_rs4 = gemm_rs4(a.a, a.a_bytes);
     c.w_rs4 = gemm_rs4(a.w, a.w_bytes);
@@ -230,6 +241,7 @@ __device__ __forceinline__ void qg_mainloop(const qw_gemm_args &a, unsigned char
 #define QG3_AB (4 * 32 * 128)         /* A bytes per stage: 128 rows x 64 bf16 */
 #define QG3_STAGE (QG3_AB + 256 * 128) /* + W: 256 rows x 64 bf16 */
 #define QG3_WAIT_NEWEST() asm volatile("s_waitcnt vmcnt(12) lgkmcnt(0)\n\ts_barrier" ::: "memory")
+template <bool GLU>
 __device__ __forceinline__ void qg_mainloop3(const qw_gemm_args &a, unsigned char *lds,
                                              uint32_t th, uint32_t tn, uint32_t kb, uint32_t ke,
                                              floatx4 (&acc)[8][8]) {
@@ -246,7 +258,7 @@ __device__ __forceinline__ void qg_mainloop3(const qw_gemm_args &a, unsigned cha
         const uint32_t ra = wave * (MB * 8) + j * 8 + lrow;
         if (j < MB)
             c.a_dvoff[j] = (min(m0 + ra, a.m - 1) * a.lda + (lp ^ ((ra >> 1) & 7u)) * 8) * 2;
-        c.w_dvoff[j] = (min(n0 + r, a.n - 1) * a.k + (lp ^ ((r >> 1) & 7u)) * 8) * 2;
+        c.w_dvoff[j] = (qg_wrow<GLU>(a, n0, r) * a.k + (lp ^ ((r >> 1) & 7u)) * 8) * 2;
     }
     c.a_rs4 = gemm_rs4(a.a, a.a_bytes);
     c.w_rs4 = gemm_rs4(a.w, a.w_bytes);
@@ -489,6 +501,7 @@ __device__ __forceinline__ void qw8_slice(const QgCtx &c, Qw8 &w, floatx4 (&acc)
 
 /* Sums of tile (tm, tn) over k-steps [kb, ke), int8 W widened per
  * workgroup; ends with the LDS stages free and no load in flight. */
+template <bool GLU>
 __device__ __forceinline__ void qw8_mainloop(const qw_gemm_args &a, unsigned char *lds,
                                              unsigned char *lds_b, uint32_t tm, uint32_t tn,
                                              uint32_t kb, uint32_t ke, floatx4 (&acc)[8][8]) {
@@ -507,7 +520,7 @@ __device__ __forceinline__ void qw8_mainloop(const qw_gemm_args &a, unsigned cha
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const uint32_t r = wave * 64 + i * 16 + (lane >> 2), q = lane & 3;
-        w.voff[i] = min(n0 + r, a.n - 1) * a.k + q * 16;
+        w.voff[i] = qg_wrow<GLU>(a, n0, r) * a.k + q * 16;
 #pragma unroll
         for (int h = 0; h < 2; h++)
             w.wdst[i][h] = QG_A_BYTES + r * 128 + (((2 * q + h) ^ ((r >> 1) & 7u)) << 4);
@@ -629,6 +642,7 @@ __device__ __forceinline__ void qh_slice(const QgCtx &c, floatx4 (&acc)[8][8], b
 
 /* Sums of the half tile at rows [m0, m0 + 128), columns [n0, n0 + 256) over
  * all of K into acc[0..3][*]; ends with the LDS stages free. */
+template <bool GLU>
 __device__ __forceinline__ void qh_mainloop(const qw_gemm_args &a, unsigned char *lds,
                                             unsigned char *lds_b, uint32_t m0, uint32_t n0,
                                             floatx4 (&acc)[8][8]) {
@@ -645,7 +659,7 @@ __device__ __forceinline__ void qh_mainloop(const qw_gemm_args &a, unsigned char
 #pragma unroll
     for (int j = 0; j < 8; j++) {
         const uint32_t r = wave * 64 + j * 8 + lrow;
-        c.w_dvoff[j] = (min(n0 + r, a.n - 1) * a.k + (lp ^ ((r >> 1) & 7u)) * 8) * 2;
+        c.w_dvoff[j] = (qg_wrow<GLU>(a, n0, r) * a.k + (lp ^ ((r >> 1) & 7u)) * 8) * 2;
     }
     c.a_rs4 = gemm_rs4(a.a, a.a_bytes);
     c.w_rs4 = gemm_rs4(a.w, a.w_bytes);
@@ -689,14 +703,14 @@ __device__ __forceinline__ void qh_mainloop(const qw_gemm_args &a, unsigned char
 }
 
 /* INT8: 0 bf16 W, 1 int8 W widened once per workgroup */
-template <int INT8>
+template <int INT8, bool GLU>
 __device__ __forceinline__ void qg_mainloop_any(const qw_gemm_args &a, unsigned char *lds,
                                                 unsigned char *lds_b, uint32_t tm, uint32_t tn,
                                                 uint32_t kb, uint32_t ke, floatx4 (&acc)[8][8]) {
     if constexpr (INT8)
-        qw8_mainloop(a, lds, lds_b, tm, tn, kb, ke, acc);
+        qw8_mainloop<GLU>(a, lds, lds_b, tm, tn, kb, ke, acc);
     else
-        qg_mainloop(a, lds, lds_b, tm, tn, kb, ke, acc);
+        qg_mainloop<8, GLU>(a, lds, lds_b, tm, tn, kb, ke, acc);
 }
 
 /* The epilogue of the tile (MB = 8), 224-row tile (MB = 7) or half tile
@@ -748,6 +762,28 @@ __device__ __forceinline__ void qg_finish_at(const qw_gemm_args &a, unsigned cha
             v[4 + j] = v1[j];
         }
     };
+    if constexpr (EPI == QW_EPI_SWIGLU) {
+        if (!pst) { /* a split piece's sums are stored as any other's, below */
+            auto read_half = [&](uint32_t lr, int h, float (&v)[8]) __attribute__((always_inline)) {
+                const float *p = region + lr * LDF + 64 * h + (lane & 7) * 8;
+                const floatx4 v0 = *(const floatx4 *)(p + 4 * h);
+                const floatx4 v1 = *(const floatx4 *)(p + 4 * (h ^ 1));
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[j] = v0[j], v[4 + j] = v1[j];
+            };
+            const uint32_t f0 = n0 / 2 + wn * 64;
+            if (pld)
+                gemm_epilogue_swiglu<INT8, MB / SB, 16 * SB, 2>(a, write_slab, read_half, row0, f0,
+                                                                lane, pld + poff, npart, own);
+            else
+                gemm_epilogue_swiglu<INT8, MB / SB, 16 * SB, 0>(a, write_slab, read_half, row0, f0,
+                                                                lane, nullptr, 0, 0);
+        } else {
+            gemm_epilogue_mode<QW_EPI_STORE, INT8, MB / SB, 16 * SB, 4 * SB, 1>(
+                a, write_slab, read_row, row0, col0, lane, pst + poff, nullptr, 0, 0);
+        }
+        return;
+    } else
     gemm_epilogue_lds<EPI, INT8, MB / SB, 16 * SB, 4 * SB>(a, write_slab, read_row, row0, col0, lane,
                                             pst ? pst + poff : nullptr,
                                             pld ? pld + poff : nullptr, npart, own);
@@ -765,6 +801,7 @@ __device__ __forceinline__ void qg_finish(const qw_gemm_args &a, unsigned char *
 template <int EPI, int INT8>
 __device__ __forceinline__ void qg_impl(const qw_gemm_args &a, unsigned char *lds,
                                         unsigned char *lds_b) {
+    constexpr bool GLU = EPI == QW_EPI_SWIGLU;
     const uint32_t KT = a.k / GBK;
     const uint32_t nt = a.tiles_m * a.tiles_n;
     const bool split = a.split > 1;
@@ -787,7 +824,7 @@ __device__ __forceinline__ void qg_impl(const qw_gemm_args &a, unsigned char *ld
                     uint32_t q = id;
                     if ((F & 7u) == 0) q = (q & 7u) * (F >> 3) + (q >> 3);
                     gemm_tile_at(a, q, tm, tn);
-                    qg_mainloop_any<INT8>(a, lds, lds_b, tm, tn, 0, KT, acc);
+                    qg_mainloop_any<INT8, GLU>(a, lds, lds_b, tm, tn, 0, KT, acc);
                     qg_finish<EPI, INT8>(a, lds, lds_b, tm, tn, acc);
                 } else if (!INT8) {
                     uint32_t hq = id - F;
@@ -795,9 +832,9 @@ __device__ __forceinline__ void qg_impl(const qw_gemm_args &a, unsigned char *ld
                     gemm_tile_at(a, F + (hq >> 1), tm, tn);
                     const uint32_t m0 = tm * 256 + (hq & 1) * 128;
                     if (a.half3)
-                        qg_mainloop3(a, lds, m0 / 128, tn, 0, KT, acc);
+                        qg_mainloop3<GLU>(a, lds, m0 / 128, tn, 0, KT, acc);
                     else
-                        qh_mainloop(a, lds, lds_b, m0, tn * 256, acc);
+                        qh_mainloop<GLU>(a, lds, lds_b, m0, tn * 256, acc);
                     qg_finish_at<EPI, INT8, 4>(a, lds, lds_b, m0, tn * 256, acc);
                 }
                 asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -806,7 +843,7 @@ __device__ __forceinline__ void qg_impl(const qw_gemm_args &a, unsigned char *ld
         }
         if ((ndp & 7u) == 0) pid = (pid & 7u) * (ndp >> 3) + (pid >> 3);
         gemm_tile_at(a, pid, tm, tn);
-        qg_mainloop_any<INT8>(a, lds, lds_b, tm, tn, 0, KT, acc);
+        qg_mainloop_any<INT8, GLU>(a, lds, lds_b, tm, tn, 0, KT, acc);
         qg_finish<EPI, INT8>(a, lds, lds_b, tm, tn, acc);
         return;
     }
@@ -825,13 +862,13 @@ __device__ __forceinline__ void qg_impl(const qw_gemm_args &a, unsigned char *ld
     float *slots = a.sk_part + (size_t)r * S * QW_SPLIT_PART;
     if constexpr (!INT8) {
         if (hs) {
-            qg_mainloop<4>(a, lds, lds_b, th, tn, kb, ke, acc);
+            qg_mainloop<4, GLU>(a, lds, lds_b, th, tn, kb, ke, acc);
             qg_finish_at<EPI, INT8, 4>(a, lds, lds_b, th * 128, tn * 256, acc,
                                        slots + (size_t)piece * QW_SPLIT_PART);
         }
     }
     if (!hs) {
-        qg_mainloop_any<INT8>(a, lds, lds_b, tm, tn, kb, ke, acc);
+        qg_mainloop_any<INT8, GLU>(a, lds, lds_b, tm, tn, kb, ke, acc);
         qg_finish<EPI, INT8>(a, lds, lds_b, tm, tn, acc, slots + (size_t)piece * QW_SPLIT_PART);
     }
     __builtin_amdgcn_s_waitcnt(0x0F70); /* vmcnt(0): the partial's stores are done */
@@ -869,7 +906,7 @@ __device__ __forceinline__ void qg_impl_t224(const qw_gemm_args &a, unsigned cha
         uint32_t q = id;
         if ((nt & 7u) == 0) q = (q & 7u) * (nt >> 3) + (q >> 3);
         gemm_tile_at(a, q, tm, tn);
-        qg_mainloop<7>(a, lds, lds_b, tm, tn, 0, KT, acc);
+        qg_mainloop<7, EPI == QW_EPI_SWIGLU>(a, lds, lds_b, tm, tn, 0, KT, acc);
         qg_finish_at<EPI, 0, 7>(a, lds, lds_b, tm * 224, tn * 256, acc);
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
@@ -893,7 +930,7 @@ __device__ __forceinline__ void qg_impl_h3(const qw_gemm_args &a, unsigned char 
     gemm_tile_at(a, r >> 1, tm, tn);
     const uint32_t th = tm * 2 + (r & 1);
     floatx4 acc[8][8];
-    qg_mainloop3(a, lds, th, tn, kb, ke, acc);
+    qg_mainloop3<EPI == QW_EPI_SWIGLU>(a, lds, th, tn, kb, ke, acc);
     unsigned char *lds_b = lds + QG_STAGE;
     if (S == 1) {
         qg_finish_at<EPI, 0, 4>(a, lds, lds_b, th * 128, tn * 256, acc);
@@ -932,12 +969,14 @@ QG_ENTRY(qw_gemm_bf16_store_q, QW_EPI_STORE, 0)
 QG_ENTRY(qw_gemm_bf16_gelu_q, QW_EPI_GELU, 0)
 QG_ENTRY(qw_gemm_bf16_gate_q, QW_EPI_GATE, 0)
 QG_ENTRY(qw_gemm_bf16_qkn_q, QW_EPI_QKNORM, 0)
+QG_ENTRY(qw_gemm_bf16_swiglu_q, QW_EPI_SWIGLU, 0)
 /* int8 weights (per-row scale in the epilogue), widened once per workgroup
  * into the bf16 W stage */
 QG_ENTRY(qw_gemm_w8_store_q, QW_EPI_STORE, 1)
 QG_ENTRY(qw_gemm_w8_gelu_q, QW_EPI_GELU, 1)
 QG_ENTRY(qw_gemm_w8_gate_q, QW_EPI_GATE, 1)
 QG_ENTRY(qw_gemm_w8_qkn_q, QW_EPI_QKNORM, 1)
+QG_ENTRY(qw_gemm_w8_swiglu_q, QW_EPI_SWIGLU, 1)
 /* bf16 W, 224-row tiles */
 #define QG_ENTRY_T224(name, EPI)                                                               \
     QW_KERNEL void __launch_bounds__(256, 1) name(qw_gemm_args a) {                            \
@@ -948,6 +987,7 @@ QG_ENTRY_T224(qw_gemm_bf16_store_t224, QW_EPI_STORE)
 QG_ENTRY_T224(qw_gemm_bf16_gelu_t224, QW_EPI_GELU)
 QG_ENTRY_T224(qw_gemm_bf16_gate_t224, QW_EPI_GATE)
 QG_ENTRY_T224(qw_gemm_bf16_qkn_t224, QW_EPI_QKNORM)
+QG_ENTRY_T224(qw_gemm_bf16_swiglu_t224, QW_EPI_SWIGLU)
 /* bf16 W, small launches: half tiles on three stages */
 #define QG_ENTRY_H3(name, EPI)                                                                 \
     QW_KERNEL void __launch_bounds__(256, 1) name(qw_gemm_args a) {                            \
@@ -958,3 +998,4 @@ QG_ENTRY_H3(qw_gemm_bf16_store_h3, QW_EPI_STORE)
 QG_ENTRY_H3(qw_gemm_bf16_gelu_h3, QW_EPI_GELU)
 QG_ENTRY_H3(qw_gemm_bf16_gate_h3, QW_EPI_GATE)
 QG_ENTRY_H3(qw_gemm_bf16_qkn_h3, QW_EPI_QKNORM)
+QG_ENTRY_H3(qw_gemm_bf16_swiglu_h3, QW_EPI_SWIGLU)

@@ -13,9 +13,11 @@ enum {
     QW_EPI_STORE = 0, /* store y */
     QW_EPI_GELU = 1,  /* store bf16(gelu_tanh(y)) */
     QW_EPI_GATE = 2,  /* out = bf16(out + y * gate[row_map[r]][n]) in place */
-    QW_EPI_QKNORM = 3 /* store y; columns below qk_cols (q then k heads of 128)
-                       * first get the per-head RMS norm and the RoPE rotation
-                       * of qw_qk_norm_rope_bf16, with its rounding points */
+    QW_EPI_QKNORM = 3, /* store y; columns below qk_cols (q then k heads of 128)
+                        * first get the per-head RMS norm and the RoPE rotation
+                        * of qw_qk_norm_rope_bf16, with its rounding points */
+    QW_EPI_SWIGLU = 4  /* w = [gate | up] rows, n = 2F: store bf16(bf16(silu(y
+                        * of gate row f)) * y of up row F + f) in column f */
 };
 
 typedef struct {

@@ -49,7 +49,7 @@ struct qw_dit {
     h3_gpu_tensor *txt_norm;
     /* activation workspaces, sized for ws_rows rows */
     uint32_t ws_rows;
-    h3_gpu_tensor *ws_mod, *ws_qkv, *ws_attn, *ws_wide, *ws_act;
+    h3_gpu_tensor *ws_mod, *ws_qkv, *ws_attn, *ws_wide;
     uint32_t ws_text_rows;
     h3_gpu_tensor *ws_tnorm, *ws_twide;
     /* conditioning (2 modulation rows) */
@@ -728,7 +728,7 @@ void qw_dit_free(qw_dit *d) {
     lin_free(&d->mod);
     lin_free(&d->norm_out);
     lin_free(&d->proj_out);
-    h3_gpu_tensor *t[] = {d->txt_norm, d->ws_mod, d->ws_qkv, d->ws_attn, d->ws_wide, d->ws_act,
+    h3_gpu_tensor *t[] = {d->txt_norm, d->ws_mod, d->ws_qkv, d->ws_attn, d->ws_wide,
                           d->ws_tnorm, d->ws_twide, d->feat, d->feat_bf16, d->c_wide, d->c_silu,
                           d->temb, d->mod_raw, d->modulation, d->norm_out_mod, d->joint,
                           d->row_map};
@@ -843,8 +843,7 @@ static void free_ws(qw_dit *d) {
     h3_gpu_tensor_free(d->ws_qkv);
     h3_gpu_tensor_free(d->ws_attn);
     h3_gpu_tensor_free(d->ws_wide);
-    h3_gpu_tensor_free(d->ws_act);
-    d->ws_mod = d->ws_qkv = d->ws_attn = d->ws_wide = d->ws_act = NULL;
+    d->ws_mod = d->ws_qkv = d->ws_attn = d->ws_wide = NULL;
     d->ws_rows = 0;
 }
 
@@ -854,13 +853,11 @@ static int ensure_ws(qw_dit *d, uint32_t rows) {
     free_ws(d);
     h3_gpu *g = d->gpu;
     const size_t H = d->cfg.hidden, F = d->cfg.mlp_width;
-    const int swiglu = d->cfg.mlp_act == QW_MLP_SWIGLU;
     d->ws_mod = h3_gpu_tensor_new_bf16(g, rows * H);
     d->ws_qkv = h3_gpu_tensor_new_bf16(g, rows * 3 * H);
     d->ws_attn = h3_gpu_tensor_new_bf16(g, rows * H);
-    d->ws_wide = h3_gpu_tensor_new_bf16(g, rows * (swiglu ? 2 * F : F));
-    d->ws_act = swiglu ? h3_gpu_tensor_new_bf16(g, rows * F) : NULL;
-    if (!d->ws_mod || !d->ws_qkv || !d->ws_attn || !d->ws_wide || (swiglu && !d->ws_act)) {
+    d->ws_wide = h3_gpu_tensor_new_bf16(g, rows * F);
+    if (!d->ws_mod || !d->ws_qkv || !d->ws_attn || !d->ws_wide) {
         free_ws(d);
         return 0;
     }
@@ -1032,6 +1029,25 @@ static int qkv_linear(qw_dit *d, const qw_layer *L, uint32_t M, const h3_gpu_ten
     return qw_gpu_linear(d->gpu, &desc);
 }
 
+/* The fused gate|up projection and its SwiGLU in one launch:
+ * ws_wide [M, F] = silu(gate) * up of ws_mod. */
+static int swiglu_linear(qw_dit *d, const qw_layer *L, uint32_t M) {
+    qw_linear_desc desc;
+    memset(&desc, 0, sizeof(desc));
+    desc.out = d->ws_wide;
+    desc.ldc = d->cfg.mlp_width;
+    desc.in = d->ws_mod;
+    desc.lda = d->cfg.hidden;
+    desc.weight = L->fc1.w;
+    desc.wscale = L->fc1.scales;
+    desc.bias = L->fc1.bias;
+    desc.rows = M;
+    desc.k = d->cfg.hidden;
+    desc.cols = L->fc1.n;
+    desc.epilogue = QW_LINEAR_STORE;
+    return qw_gpu_linear_swiglu(d->gpu, &desc);
+}
+
 static int block_run(qw_dit *d, int li, h3_gpu_tensor *hidden, uint32_t batch, uint32_t rows,
                      uint32_t text_rows, const h3_gpu_tensor *modulation,
                      const h3_gpu_tensor *rope_cos, const h3_gpu_tensor *rope_sin,
@@ -1112,24 +1128,16 @@ static int block_run(qw_dit *d, int li, h3_gpu_tensor *hidden, uint32_t batch, u
     if (!ok) return 0;
 
     prof_begin(d);
-    if (d->cfg.mlp_act == QW_MLP_GELU_TANH) {
-        span_b(d, QW_SPAN_UP);
+    span_b(d, QW_SPAN_UP);
+    if (d->cfg.mlp_act == QW_MLP_GELU_TANH)
         ok = plain(d, &L->fc1, d->ws_wide, d->ws_mod, M, QW_LINEAR_GELU);
-        span_e(d);
-        span_b(d, QW_SPAN_DOWN);
-        ok = ok && linear(d, &L->fc2, hidden, 0, H, d->ws_wide, 0, F, M, QW_LINEAR_GATE,
-                          modulation, row_map, S, 3);
-        span_e(d);
-    } else {
-        span_b(d, QW_SPAN_UP);
-        ok = plain(d, &L->fc1, d->ws_wide, d->ws_mod, M, QW_LINEAR_STORE) &&
-             qw_gpu_swiglu_bf16(g, d->ws_act, d->ws_wide, M, F);
-        span_e(d);
-        span_b(d, QW_SPAN_DOWN);
-        ok = ok && linear(d, &L->fc2, hidden, 0, H, d->ws_act, 0, F, M, QW_LINEAR_GATE,
-                          modulation, row_map, S, 3);
-        span_e(d);
-    }
+    else
+        ok = swiglu_linear(d, L, M);
+    span_e(d);
+    span_b(d, QW_SPAN_DOWN);
+    ok = ok && linear(d, &L->fc2, hidden, 0, H, d->ws_wide, 0, F, M, QW_LINEAR_GATE, modulation,
+                      row_map, S, 3);
+    span_e(d);
     prof_end(d, P_MLP);
     return ok;
 }

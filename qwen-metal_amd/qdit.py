@@ -131,6 +131,7 @@ SIGNATURES = {
     "qw_gpu_layer_norm_mod_shift_bf16": (C.c_int, [vp, vp, vp, vp, vp, u32, u32, u32, u32,
                                                    C.c_int32, C.c_float]),
     "qw_gpu_linear": (C.c_int, [vp, C.POINTER(LinearDesc)]),
+    "qw_gpu_linear_swiglu": (C.c_int, [vp, C.POINTER(LinearDesc)]),
     "qw_gpu_linear_static": (C.c_int, [vp, C.POINTER(LinearDesc)]),
     "qw_gpu_qk_norm_rope_bf16": (C.c_int, [vp, vp, u32, u32, u32, u32, vp, vp, vp, vp, u32,
                                            C.c_float]),

@@ -1,0 +1,103 @@
+"""The fused SwiGLU linear (qw_gpu_linear_swiglu) against the linear followed
+by the separate SwiGLU pass, which have their own tests against the oracle.
+
+Both take the same sums in the same order, so g and u are the same bf16
+values. The fused form evaluates silu with the hardware exp and reciprocal
+(relative error about 2^-22, against a bf16 half-ulp of 2^-9): bf16(silu)
+flips where it lies that close to a rounding boundary, about one value in
+2^12, by one ulp, which the product passes on as at most two."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from conftest import ulp_diff
+
+pytestmark = pytest.mark.gpu
+
+
+def fused(gpu, qd, out, x, w, rows, k, F, ldc=None, **kw):
+    h = lambda t: t.h if t is not None else None  # noqa: E731
+    d = qd.LinearDesc(out.h, kw.get("out_offset", 0), ldc or F, x.h, 0, k, w.h,
+                      h(kw.get("wscale")), h(kw.get("bias")), rows, k, 2 * F,
+                      kw.get("epilogue", qd.LINEAR_STORE), *([None] * 2), 0, 0, *([None] * 4), 0,
+                      0.0)
+    return qd.lib().qw_gpu_linear_swiglu(gpu.h, C.byref(d))
+
+
+# rows, k, F: half tiles and ragged columns; split pieces of small launches;
+# the streaming rows; whole tiles with a split tail; 224-row tiles; the walk
+# with its half-tile tail
+CASES = [(9, 64, 64, False), (100, 128, 200, True), (300, 1024, 448, False), (130, 4096, 256, True),
+         (3, 256, 72, True), (8, 64, 128, False), (520, 2304, 4096, False), (2100, 64, 4224, True),
+         (4119, 64, 3072, False)]
+
+
+@pytest.mark.parametrize("route", ["bf16", "int8", "w8"])
+@pytest.mark.parametrize("rows,k,F,bias", CASES)
+def test_swiglu_linear_is_linear_then_swiglu(qd, oracle, monkeypatch, rows, k, F, bias, route):
+    if route == "w8":
+        monkeypatch.setenv("QW_INT8_ROUTE", "w8")
+    gpu = qd.Gpu()
+    try:
+        x = gpu.put(oracle.fill_normal_bf16(rows * k, 7, 1, 1.0))
+        w = gpu.put(oracle.fill_normal_bf16(2 * F * k, 7, 2, 1.5 / np.sqrt(k)))
+        b = gpu.put(oracle.fill_normal_bf16(2 * F, 7, 3, 0.2)) if bias else None
+        s = None
+        if route != "bf16":
+            q, s = gpu.new(2 * F * k, qd.I8), gpu.new(2 * F, qd.F32)
+            gpu.check(qd.lib().h3_gpu_quantize_weight_int8(gpu.h, q.h, s.h, w.h, 2 * F, k), "q")
+            w = q
+        wide, two = gpu.new(rows * 2 * F, qd.BF16), gpu.new(rows * F, qd.BF16)
+        gpu.linear(wide, x, w, rows, k, 2 * F, bias=b, wscale=s)
+        gpu.check(qd.lib().qw_gpu_swiglu_bf16(gpu.h, two.h, wide.h, rows, F), "swiglu")
+        pad = 0 if rows <= 8 else 8  # a strided output's gap stays untouched
+        one = gpu.put(np.full(rows * (F + pad), 0x1234, np.uint16))
+        gpu.check(fused(gpu, qd, one, x, w, rows, k, F, ldc=F + pad, bias=b, wscale=s), "fused")
+        gpu.submit()
+        got = one.read().reshape(rows, F + pad)
+        assert (got[:, F:] == 0x1234).all()
+        d = ulp_diff(np.ascontiguousarray(got[:, :F]).ravel(), two.read())
+        assert d.max() <= 2 and np.mean(d != 0) < 2e-3, (d.max(), np.mean(d != 0))
+    finally:
+        gpu.close()
+
+
+def test_swiglu_linear_gate_range(gpu, qd, oracle):
+    """Gates over the whole bf16 range (x = I picks single weights): no
+    overflow, and silu right to one bf16 ulp where the result is normal, up
+    to the gates where e^-g overflows."""
+    k = F = 64
+    mags = np.geomspace(1e-30, 3e38, k * F // 2)
+    g = np.concatenate([mags, -mags, ])
+    g[:200] = np.linspace(-89.5, -80.0, 200)
+    gb = oracle.f32_to_bf16(g.astype(np.float32)).reshape(F, k)
+    up = oracle.f32_to_bf16(np.ones((F, k), np.float32))
+    x = oracle.f32_to_bf16(np.eye(k, dtype=np.float32))
+    out = gpu.new(k * F, qd.BF16)
+    gpu.check(fused(gpu, qd, out, gpu.put(x), gpu.put(np.concatenate([gb, up])), k, k, F), "fused")
+    gpu.submit()
+    got = oracle.bf16_to_f32(out.read()).astype(np.float64).reshape(k, F).T
+    v = oracle.bf16_to_f32(gb.ravel()).astype(np.float64).reshape(F, k)
+    ref = np.where(v < -709, 0.0, v / (1.0 + np.exp(-np.maximum(v, -709))))
+    # where e^-g overflows fp32 (g < -88.7) silu comes out as 0, as the
+    # separate pass has it; one rounding to bf16 otherwise
+    assert np.isfinite(got).all()
+    live = v > -88.7
+    assert (np.abs(got - ref)[live] <= 2.0 ** -8 * np.abs(ref)[live] + 2.0 ** -133).all()
+    assert (np.abs(got)[~live] <= 1e-35).all()
+
+
+def test_swiglu_linear_refusals(gpu, qd):
+    F, k, rows = 64, 64, 16
+    x, w, out = gpu.new(rows * k, qd.BF16), gpu.new(2 * F * k, qd.BF16), gpu.new(rows * F, qd.BF16)
+    assert fused(gpu, qd, out, x, w, rows, k, F)
+    assert not fused(gpu, qd, out, x, w, rows, k, F, ldc=F - 8)
+    assert not fused(gpu, qd, out, x, w, rows + 1, k, F)
+    assert not fused(gpu, qd, out, x, w, rows, k, F, epilogue=qd.LINEAR_GELU)
+    assert not fused(gpu, qd, out, x, w, rows, k, F, epilogue=4)
+    assert not fused(gpu, qd, out, x, w, 4, k, F, ldc=F + 8)
+    d = qd.LinearDesc(out.h, 0, F, x.h, 0, k, w.h, None, None, rows, k, F, 4, None, None, 0, 0,
+                      None, None, None, None, 0, 0.0)
+    assert not qd.lib().qw_gpu_linear(gpu.h, C.byref(d))  # not an epilogue of qw_gpu_linear
+    gpu.submit()
