@@ -31,7 +31,9 @@ enum {
     K_GEMV_BF16_STORE, K_GEMV_BF16_GELU, K_GEMV_I8_STORE, K_GEMV_I8_GELU, K_ZERO,
     K_GEMM_W8_STORE_Q, K_GEMM_W8_GELU_Q, K_GEMM_W8_GATE_Q, K_GEMM_W8_QKN_Q, K_GEMM_W8_SWIGLU_Q,
     K_GEMM_BF16_STORE_T224, K_GEMM_BF16_GELU_T224, K_GEMM_BF16_GATE_T224, K_GEMM_BF16_QKN_T224, K_GEMM_BF16_SWIGLU_T224,
-    K_GEMM_BF16_STORE_H3, K_GEMM_BF16_GELU_H3, K_GEMM_BF16_GATE_H3, K_GEMM_BF16_QKN_H3, K_GEMM_BF16_SWIGLU_H3,
+    /* narrow tiles of 64, 128, 192 and 256 rows, each in the same order */
+    K_GEMM_N1, K_GEMM_N1_LAST = K_GEMM_N1 + 4, K_GEMM_N2, K_GEMM_N2_LAST = K_GEMM_N2 + 4,
+    K_GEMM_N3, K_GEMM_N3_LAST = K_GEMM_N3 + 4, K_GEMM_N4, K_GEMM_N4_LAST = K_GEMM_N4 + 4,
     K_ATTN_W4,
     K_COUNT
 };
@@ -48,8 +50,11 @@ static const char *k_names[K_COUNT] = {
     "qw_gemm_w8_store_q", "qw_gemm_w8_gelu_q", "qw_gemm_w8_gate_q", "qw_gemm_w8_qkn_q", "qw_gemm_w8_swiglu_q",
     "qw_gemm_bf16_store_t224", "qw_gemm_bf16_gelu_t224", "qw_gemm_bf16_gate_t224",
     "qw_gemm_bf16_qkn_t224", "qw_gemm_bf16_swiglu_t224",
-    "qw_gemm_bf16_store_h3", "qw_gemm_bf16_gelu_h3", "qw_gemm_bf16_gate_h3",
-    "qw_gemm_bf16_qkn_h3", "qw_gemm_bf16_swiglu_h3", "qw_attention_w4_bf16"};
+    "qw_gemm_bf16_store_n1", "qw_gemm_bf16_gelu_n1", "qw_gemm_bf16_gate_n1", "qw_gemm_bf16_qkn_n1", "qw_gemm_bf16_swiglu_n1",
+    "qw_gemm_bf16_store_n2", "qw_gemm_bf16_gelu_n2", "qw_gemm_bf16_gate_n2", "qw_gemm_bf16_qkn_n2", "qw_gemm_bf16_swiglu_n2",
+    "qw_gemm_bf16_store_n3", "qw_gemm_bf16_gelu_n3", "qw_gemm_bf16_gate_n3", "qw_gemm_bf16_qkn_n3", "qw_gemm_bf16_swiglu_n3",
+    "qw_gemm_bf16_store_n4", "qw_gemm_bf16_gelu_n4", "qw_gemm_bf16_gate_n4", "qw_gemm_bf16_qkn_n4", "qw_gemm_bf16_swiglu_n4",
+    "qw_attention_w4_bf16"};
 
 /* How int8 linears run (QW_INT8_ROUTE, a measurement switch): AUTO (the
  * default) widens the weight to a bf16 copy and runs the bf16 kernels when
@@ -61,7 +66,7 @@ enum { QW_INT8_AUTO = 0, QW_INT8_WIDEN = 1, QW_INT8_W8 = 2 };
 #define QW_SPAN_MAX 4096
 
 /* below this many rows an int8 linear widens inside its GEMM, unless the
- * launch is small enough for half tiles (linear_impl) */
+ * launch is small enough for narrow tiles (linear_impl) */
 #define QW_WIDEN_MIN_ROWS 512
 
 struct h3_gpu {
@@ -83,11 +88,9 @@ struct h3_gpu {
     int int8_route; /* QW_INT8_* : how int8 linears of many rows run */
     int t224;       /* 224-row tiles allowed (QW_GEMM_T224=0 turns them off, for measurement) */
     uint32_t split_min_steps, split_force; /* measurement: QW_SPLIT_MIN_STEPS, QW_SPLIT_FORCE */
-    uint32_t split_small_min; /* shortest piece of a small launch (QW_SPLIT_SMALL_MIN_STEPS) */
-    int half3;      /* small launches' half tiles on the three-stage kernels (QW_GEMM_HALF3=0: two) */
     uint32_t widen_min_rows; /* int8: fewest rows for the widening route (QW_WIDEN_MIN_ROWS) */
     int t224_over_split; /* 224-row tiles preferred to split tiles (QW_T224_OVER_SPLIT=0: off) */
-    int half_small; /* launches of at most cus / 2 tiles as half tiles (QW_GEMM_HALF_SMALL=0: off) */
+    int narrow;     /* narrow tiles allowed (QW_GEMM_HALF_SMALL=0: off) */
     /* qw_gpu_span_*: event pairs recorded on the stream, read after a sync */
     hipEvent_t *span_ev;
     int *span_tag;
@@ -204,18 +207,14 @@ extern "C" h3_gpu *h3_gpu_create(const char *code_object_path, char *error,
     if (const char *r = getenv("QW_GEMM_T224")) g->t224 = atoi(r) != 0;
     g->split_min_steps = 32;
     if (const char *r = getenv("QW_SPLIT_MIN_STEPS")) g->split_min_steps = (uint32_t)atoi(r);
-    g->split_small_min = 16;
-    if (const char *r = getenv("QW_SPLIT_SMALL_MIN_STEPS")) g->split_small_min = (uint32_t)atoi(r);
     g->split_force = 0;
     if (const char *r = getenv("QW_SPLIT_FORCE")) g->split_force = (uint32_t)atoi(r);
-    g->half3 = 1;
-    if (const char *r = getenv("QW_GEMM_HALF3")) g->half3 = atoi(r) != 0;
     g->widen_min_rows = QW_WIDEN_MIN_ROWS;
     if (const char *r = getenv("QW_WIDEN_MIN_ROWS")) g->widen_min_rows = (uint32_t)atoi(r);
     g->t224_over_split = 1;
     if (const char *r = getenv("QW_T224_OVER_SPLIT")) g->t224_over_split = atoi(r) != 0;
-    g->half_small = 1;
-    if (const char *r = getenv("QW_GEMM_HALF_SMALL")) g->half_small = atoi(r) != 0;
+    g->narrow = 1;
+    if (const char *r = getenv("QW_GEMM_HALF_SMALL")) g->narrow = atoi(r) != 0;
     g->cus = 0;
     g->sk_part = NULL;
     g->sk_flag = NULL;
@@ -955,9 +954,7 @@ extern "C" int qw_gpu_widen_int8_bf16(h3_gpu *g, h3_gpu_tensor *out, const h3_gp
  * 152 tail tiles in 3 pieces 557-588 us against 573-644 us for the
  * whole-tile walk, same boxes; 2, 4 or 5 pieces 595-660 us). Pieces stay at least 32 k-steps (2048 k) long: shorter
  * pieces lost more to their partials than they gained (K = 3072 linears
- * measured slower when split, K = 12288 ones faster); the half tiles of a
- * launch of at most cus / 2 tiles, whose pieces all run in one wave, go
- * down to 16. And
+ * measured slower when split, K = 12288 ones faster). And
  * R s <= QW_SPLIT_MAX_PIECES * cus bounds the partial workspace. */
 #define QW_SPLIT_MAX_PIECES 2
 static uint32_t split_choice(h3_gpu *g, uint32_t tiles, uint32_t ksteps,
@@ -984,29 +981,122 @@ static uint32_t split_choice(h3_gpu *g, uint32_t tiles, uint32_t ksteps,
     return best;
 }
 
-/* Pieces for the half tiles of a small launch (at most cus / 2 tiles), all
- * in one round of CUs: the s that minimises 0.72 ksteps / s + 12 + 0.04
- * units s microseconds -- a half tile's slice, then each piece's prologue,
- * partial sums and last-piece reduction, which grow with the pieces in
- * flight. Fitted to the three-stage kernels at K = 3072 (M = 320: 24, 48,
- * 64, 96, 128 half tiles in 3, 3, 3, 2, 2 pieces 26.0, 29.3, 32.4, 35.8,
- * 40.6 us against 34.7-35.6 unsplit; M = 1152: 120 in 2 pieces 38.8
- * against 35.5), within 1.2 us of each. */
-static uint32_t small_split_choice(h3_gpu *g, uint32_t units, uint32_t ksteps) {
-    if (g->split_force > 1 && (uint64_t)units * g->split_force <= g->cus &&
-        ksteps >= g->split_force)
-        return g->split_force;
-    uint32_t best = 1;
-    double best_t = 0.72 * ksteps;
-    for (uint32_t s = 2; s <= 8; s++) {
-        if ((uint64_t)units * s > g->cus || ksteps < g->split_small_min * s) break;
-        const double t = 0.72 * ksteps / s + 12.0 + 0.04 * units * s;
-        if (t < best_t) {
-            best_t = t;
-            best = s;
+/* 224-row tiles where they leave fewer (work-weighted) waves than 256-row
+ * tiles with their half-tile tail: a wave of 224-row tiles is 0.875 of one
+ * of 256-row tiles. Out projection, M = 8704: 2 waves of 0.875 (468 tiles)
+ * against 2 waves (408 tiles). */
+static int rule_224(const h3_gpu *g, uint32_t rows, uint32_t cols) {
+    if (!g->t224 || g->cus % 8) return 0;
+    const uint32_t C = g->cus, tn = (cols + 255) / 256, tiles = (rows + 255) / 256 * tn;
+    const uint32_t t224 = (rows + 223) / 224 * tn, R = tiles % C;
+    const double w256 = (double)(tiles / C) + (R ? (2 * R <= C ? 0.5 : 1.0) : 0.0);
+    return 0.875 * (double)((t224 + C - 1) / C) < 0.97 * w256;
+}
+
+/* Time models of a linear on bf16 W, in microseconds, that pick its tiles.
+ *
+ * Wide (gemm_q.h): a round of 256 x 256 tiles takes 1.3 us a k-step (64 k)
+ * and 12 us for prologue and epilogue (measured at M = 1152-8704: 75-88 us a
+ * round at K = 3072, 92-102 at 4096, 274 at 12288); a partly filled last
+ * round the length of split_choice's pieces and 8 + 0.055 R s^2 us for their
+ * partial sums (M = 4119 against 4096, K = 4096: 59, 65 and 79 us for 16, 48
+ * and 96 tail tiles in 2; K = 12288: 79 us for 16 in 6, 138 for 60 in 4), or
+ * half a round on half tiles. */
+static double wide_us(h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t ksteps) {
+    const uint32_t C = g->cus, tn = (cols + 255) / 256, tiles = (rows + 255) / 256 * tn;
+    const double round = 1.3 * ksteps + 12.0;
+    if (rule_224(g, rows, cols)) return 0.875 * round * (((rows + 223) / 224 * tn + C - 1) / C);
+    const uint32_t R = tiles % C, s = split_choice(g, tiles, ksteps);
+    double t = (double)(tiles / C) * round;
+    if (s > 1)
+        t += (double)((R * s + C - 1) / C) / s * round + 8.0 + 0.055 * R * s * s;
+    else if (R)
+        t += tiles > C && 2 * R <= C ? 0.5 * round : round;
+    return t;
+}
+
+/* Narrow (gemm_s.h), tiles of 64 mb rows x 128 columns in s k-range pieces:
+ * a k-step of a tile takes 0.30, 0.39, 0.56, 0.70 us (mb = 1-4), times 0.85
+ * to 1.2 from an idle to a full chip and 1.35 to 1 from K = 8192 on (an A
+ * panel no longer stays in L2 beside the weights), a round 5 us more, and s
+ * pieces 0.5 + s (0.5 + 0.45 mb) us for the partial sums. Fitted to M =
+ * 23-1152 at K = 3072, 4096 and 12288 within 15% (M = 320: 26, 14, 37, 42 us
+ * for QKV, out, up and down, against 45, 33, 46 and 62 on the 128 x 256 tiles
+ * that these replace; M = 100, K = 4096: 13 against 31). The weights cannot
+ * come faster than 5 TB/s. Returns the least time and its mb and s. */
+static double narrow_us(const h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t ksteps,
+                        uint32_t *mb_out, uint32_t *s_out) {
+    static const double step_us[4] = {0.30, 0.39, 0.56, 0.70}, long_k[4] = {1.35, 1.3, 1.15, 1.0};
+    const uint32_t C = g->cus, tn = (cols + 127) / 128;
+    const double hbm_us = (double)cols * ksteps * 128 / 5e6;
+    double best = 1e30;
+    for (uint32_t mb = 1; mb <= 4; mb++) {
+        const uint32_t R = (rows + 64 * mb - 1) / (64 * mb) * tn;
+        for (uint32_t s = 1; s <= 8; s++) {
+            /* pieces of at least 4 k-steps, all in one round, a counter each */
+            if (s > 1 && ((uint64_t)R * s > C || ksteps < 4 * s)) break;
+            const double rounds = (double)(((uint64_t)R * s + C - 1) / C);
+            if (rounds > 2) break; /* not fitted, and the wide tiles' ground */
+            const double fill = std::min(1.0, (double)R * s / C);
+            double t = rounds * ((ksteps + s - 1) / s * step_us[mb - 1] * (0.85 + 0.35 * fill) *
+                                     (ksteps >= 128 ? long_k[mb - 1] : 1.0) + 5.0);
+            if (s > 1) t += 0.5 + s * (0.5 + 0.45 * mb);
+            t = std::max(t, hbm_us + 3.0);
+            if (t < best) {
+                best = t;
+                *mb_out = mb;
+                *s_out = s;
+            }
         }
     }
     return best;
+}
+
+/* How the rows of a linear on bf16 W run: the first `wide` of them (a
+ * multiple of 256 when the rest are not none) on wide tiles, the rest on
+ * narrow ones. A last tile row of few rows costs a whole round of wide tiles
+ * wherever it opens one (M = 4119, K = 4096, N = 4096: 161 us against 102
+ * for M = 4096), and one or two us per column of narrow tiles. */
+struct linear_plan {
+    uint32_t wide, mb, s;
+};
+static linear_plan plan_linear(h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t ksteps) {
+    linear_plan p = {rows, 0, 1};
+    if (!g->narrow) return p;
+    uint32_t mb, s;
+    double best = wide_us(g, rows, cols, ksteps);
+    const double all = narrow_us(g, rows, cols, ksteps, &mb, &s);
+    if (all < 0.98 * best) {
+        best = all;
+        p = {0, mb, s};
+    }
+    const uint32_t rem = rows % 256;
+    if (rem && rows > 256) {
+        const double t = wide_us(g, rows - rem, cols, ksteps) +
+                         narrow_us(g, rem, cols, ksteps, &mb, &s);
+        if (t < 0.97 * best) p = {rows - rem, mb, s};
+    }
+    return p;
+}
+
+/* partial sums and piece counters of split tiles, from the first one on */
+static int split_workspace(h3_gpu *g) {
+    if (g->sk_part) return 1;
+    hipStreamSynchronize(g->stream);
+    const size_t n = (size_t)QW_SPLIT_MAX_PIECES * g->cus;
+    g->stats.allocated_bytes += n * 256 * 256 * 4 + (size_t)g->cus * 4;
+    if (hipMalloc((void **)&g->sk_part, n * 256 * 256 * 4) != hipSuccess) {
+        g->sk_part = NULL;
+        return fail(g, "linear: split-tile workspace allocation failed");
+    }
+    if (hipMalloc((void **)&g->sk_flag, (size_t)g->cus * 4) != hipSuccess ||
+        hipMemset(g->sk_flag, 0, (size_t)g->cus * 4) != hipSuccess) {
+        hipFree(g->sk_part);
+        g->sk_part = NULL;
+        g->sk_flag = NULL;
+        return fail(g, "linear: split-tile flag allocation failed");
+    }
+    return 1;
 }
 
 /* no_alloc: the workspace-free form behind qw_gpu_linear_static (int8
@@ -1121,15 +1211,7 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc) {
      * VALU work (1.5 instructions per weight per workgroup): the same
      * kernel with the conversion left out runs as fast as the widening
      * pass plus the bf16 kernel. */
-    /* the 224-row tile rule on this shape (whole tiles, bf16 kernels) */
-    const uint32_t tn_w = (d->cols + 255) / 256, tiles_w = ((d->rows + 255) / 256) * tn_w;
-    const uint32_t t224_w = ((d->rows + 223) / 224) * tn_w;
-    int rule224 = 0;
-    if (g->t224 && g->cus % 8 == 0) {
-        const uint32_t C = g->cus, R = tiles_w % C;
-        const double w256 = (double)(tiles_w / C) + (R ? (2 * R <= C ? 0.5 : 1.0) : 0.0);
-        rule224 = 0.875 * (double)((t224_w + C - 1) / C) < 0.97 * w256;
-    }
+    const int rule224 = rule_224(g, d->rows, d->cols); /* on whole tiles, bf16 kernels */
     /* K >= 8192 keeps the in-LDS widening, unless the widened weight's bf16
      * kernel takes 224-row tiles (the down projection at M = 8704: whole
      * steps 64.07 against 65.39 ms with the pass and 224-row tiles, medians
@@ -1137,14 +1219,19 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc) {
     int route = g->int8_route;
     if (route == QW_INT8_AUTO)
         route = d->k >= 8192 && !(rule224 && g->t224_over_split) ? QW_INT8_W8 : QW_INT8_WIDEN;
-    /* A launch of at most cus / 2 tiles widens by a pass at any row count
-     * and K: the bf16 kernels' half tiles beat the whole "_w8" tiles by more
-     * than the pass costs (M = 64-448, us, w8 / pass + half tiles: QKV
+    /* Where the bf16 kernels take narrow tiles, for all rows or for the last
+     * few, the weight is widened by a pass at any row count and K: they beat
+     * the whole "_w8" tiles by more than the pass costs (M = 64-448, us, w8 /
+     * pass + 128 x 256 half tiles, which narrow tiles beat in turn: QKV
      * 64-66 / 48-55, out 63 / 35-38, up 65-67 / 56-59, down 74-84 / 66-76). */
-    const int small_w = g->int8_route == QW_INT8_AUTO && g->half_small && 2 * tiles_w <= g->cus;
+    linear_plan plan = {d->rows, 0, 1};
+    if (!no_alloc && (!int8 || g->int8_route != QW_INT8_W8))
+        plan = plan_linear(g, d->rows, d->cols, d->k / 64);
+    const int small_w = g->int8_route == QW_INT8_AUTO && plan.mb != 0;
     if (small_w) route = QW_INT8_WIDEN;
     const int widen = int8 && !no_alloc && (d->rows >= g->widen_min_rows || small_w) &&
                       route == QW_INT8_WIDEN;
+    if (int8 && !widen) plan = {d->rows, 0, 1};
     const void *wptr = d->weight->ptr;
     if (widen) {
         const size_t n = (size_t)d->cols * d->k, bytes = n * 2;
@@ -1199,27 +1286,43 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc) {
     a.rope_rows = qkn ? d->rope_rows : 1;
     a.qk_cols = qkn ? d->cols / 3 * 2 : 0;
     a.eps = qkn ? d->eps : 0.0f;
-    a.tiles_m = (d->rows + bm - 1) / bm;
+    a.half_from = 0;
+    a.half_count = 0;
+    a.m_base = 0;
+    a.sk_part = NULL;
+    a.sk_flag = NULL;
+    if (plan.mb) { /* the rows past plan.wide on narrow tiles */
+        qw_gemm_args n = a;
+        n.m_base = plan.wide;
+        n.tiles_m = (d->rows - plan.wide + 64 * plan.mb - 1) / (64 * plan.mb);
+        n.tiles_n = (d->cols + 127) / 128;
+        n.dp_tiles = 0;
+        n.split = plan.s;
+        const uint64_t np = (uint64_t)n.tiles_m * n.tiles_n * plan.s;
+        if (np >= (1ull << 31)) return fail(g, "linear: grid too large");
+        if (plan.s > 1) {
+            /* narrow_us keeps the pieces within a round: checked, so that a
+             * change to it fails loudly */
+            if (np > g->cus) return fail(g, "linear: internal error: %llu pieces", (unsigned long long)np);
+            if (!split_workspace(g)) return 0;
+            n.sk_part = g->sk_part;
+            n.sk_flag = g->sk_flag;
+        }
+        static const int first[4] = {K_GEMM_N1, K_GEMM_N2, K_GEMM_N3, K_GEMM_N4};
+        if (!launch(g, first[plan.mb - 1] + d->epilogue, dim3((uint32_t)np), dim3(threads), n))
+            return 0;
+        if (!plan.wide) return 1;
+        a.m = plan.wide;
+    }
+    const uint32_t rows = plan.wide; /* on wide tiles */
+    a.tiles_m = (rows + bm - 1) / bm;
     a.tiles_n = (d->cols + bn - 1) / bn;
     const uint32_t tiles = a.tiles_m * a.tiles_n;
     a.dp_tiles = tiles;
     a.split = 1;
-    a.sk_part = NULL;
-    a.sk_flag = NULL;
     uint32_t grid = tiles;
-    int small = 0;
-    /* 224-row tiles where they leave fewer (work-weighted) waves than
-     * 256-row tiles with their half-tile tail: a wave of 224-row tiles is
-     * 0.875 of one of 256-row tiles. Out projection, M = 8704: 2 waves of
-     * 0.875 (468 tiles) against 2 waves (408 tiles). */
-    const uint32_t t224 = ((d->rows + 223) / 224) * a.tiles_n;
-    int use224 = 0;
-    if (!(int8 && !widen) && g->t224 && g->cus % 8 == 0) {
-        const uint32_t C = g->cus, R = tiles % C;
-        const double w256 = (double)(tiles / C) + (R ? (2 * R <= C ? 0.5 : 1.0) : 0.0);
-        const double w224 = 0.875 * (double)((t224 + C - 1) / C);
-        use224 = w224 < 0.97 * w256;
-    }
+    const uint32_t t224 = ((rows + 223) / 224) * a.tiles_n;
+    const int use224 = !(int8 && !widen) && rule_224(g, rows, d->cols);
     if (no_alloc) {
         const uint32_t s = split_choice(g, tiles, d->k / 64, QW_STATIC_PARTS);
         if (s > 1) {
@@ -1245,45 +1348,19 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc) {
             grid = a.dp_tiles + R * s;
         }
     } else {
-        /* a launch of at most half as many tiles as CUs (bf16-W kernels)
-         * runs as twice as many 128 x 256 half tiles, split in k-ranges
-         * where that pays (a half tile's split pieces also re-read half the
-         * partial bytes) */
-        small = !(int8 && !widen) && 2 * tiles <= g->cus && g->cus % 8 == 0 && g->half_small;
-        const uint32_t units = small ? 2 * tiles : tiles;
-        /* half tiles of a small launch: pieces of at least 16 k-steps, all
-         * in one round of CUs (a second round of short pieces costs more
-         * than it saves: M = 320, K = 3072, N = 10752, 168 half tiles in 3
-         * pieces 62.8 us against 37 unsplit) */
         /* where 224-row tiles fill the waves better they also beat split
          * tiles (down projection shape, bf16 W, M = 8704: 500 us unsplit on
          * 224-row tiles against 568 with 256-row tiles and a 3-piece tail) */
-        const uint32_t s = small ? small_split_choice(g, units, d->k / 64)
-                         : use224 && g->t224_over_split ? 1u
-                                                        : split_choice(g, units, d->k / 64);
+        const uint32_t s =
+            use224 && g->t224_over_split ? 1u : split_choice(g, tiles, d->k / 64);
         if (s > 1) {
-            if (!g->sk_part) {
-                hipStreamSynchronize(g->stream);
-                const size_t n = (size_t)QW_SPLIT_MAX_PIECES * g->cus;
-                g->stats.allocated_bytes += n * 256 * 256 * 4 + (size_t)g->cus * 4;
-                if (hipMalloc((void **)&g->sk_part, n * 256 * 256 * 4) != hipSuccess) {
-                    g->sk_part = NULL;
-                    return fail(g, "linear: split-tile workspace allocation failed");
-                }
-                if (hipMalloc((void **)&g->sk_flag, (size_t)g->cus * 4) != hipSuccess ||
-                    hipMemset(g->sk_flag, 0, (size_t)g->cus * 4) != hipSuccess) {
-                    hipFree(g->sk_part);
-                    g->sk_part = NULL;
-                    g->sk_flag = NULL;
-                    return fail(g, "linear: split-tile flag allocation failed");
-                }
-            }
-            const uint32_t R = units % g->cus;
+            if (!split_workspace(g)) return 0;
+            const uint32_t R = tiles % g->cus;
             /* the workspace holds QW_SPLIT_MAX_PIECES * cus partials and
              * cus counters; split_choice keeps within both */
             if ((uint64_t)R * s > (uint64_t)QW_SPLIT_MAX_PIECES * g->cus || R > g->cus)
                 return fail(g, "linear: %u x %u split pieces exceed the partial workspace", R, s);
-            a.dp_tiles = small ? 0 : tiles - R;
+            a.dp_tiles = tiles - R;
             a.split = s;
             a.sk_part = g->sk_part;
             a.sk_flag = g->sk_flag;
@@ -1294,23 +1371,8 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc) {
      * the tiles, so a tile's output stores drain under the next tile's first
      * loads (up 521 -> 514 us, QKV 365 -> 359 us against one workgroup per
      * tile) */
-    a.half_from = 0;
-    a.half_count = 0;
-    a.half3 = g->half3;
-    if (small) {
-        if (g->half3) /* one half tile (or piece of one) per workgroup, three stages */
-            return launch(g, K_GEMM_BF16_STORE_H3 + d->epilogue,
-                          dim3(2 * tiles * (a.split > 1 ? a.split : 1)), dim3(threads), a);
-        if (a.split > 1) {
-            a.half_count = 1; /* the split tiles run as half tiles */
-        } else {
-            a.half_count = 2 * tiles;
-            grid = 2 * tiles;
-        }
-        return launch(g, kid, dim3(grid), dim3(threads), a);
-    }
     if (a.split == 1 && use224) {
-        a.tiles_m = (d->rows + 223) / 224;
+        a.tiles_m = (rows + 223) / 224;
         return launch(g, K_GEMM_BF16_STORE_T224 + d->epilogue,
                       dim3(t224 < g->cus ? t224 : g->cus), dim3(threads), a);
     }

@@ -229,11 +229,12 @@ __device__ __forceinline__ void qg_mainloop(const qw_gemm_args &a, unsigned char
     asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
 }
 
-/* Half tiles (MB = 4) with three LDS stages of 48 KB (A 16 KB, then W
- * 32 KB), loads two slices ahead: for launches of at most half as many
- * tiles as CUs, whose slices are bound by the load latency rather than the
- * MFMAs (one slice ahead, a 128 x 256 slice takes most of a 256 x 256
- * slice's time). Slice j is computed from stage j % 3 while slice j + 2
+/* Half tiles (MB = 4): a tile walk whose last wave of tiles would leave at
+ * least half the CUs idle runs those tiles as twice as many 128 x 256 half
+ * tiles instead. Three LDS stages of 48 KB (A 16 KB, then W 32 KB), loads
+ * two slices ahead: a half tile's slices are bound by the load latency rather
+ * than the MFMAs (one slice ahead, a 128 x 256 slice takes most of a 256 x
+ * 256 slice's time). Slice j is computed from stage j % 3 while slice j + 2
  * streams into stage (j + 2) % 3, the stage slice j - 1 was computed from;
  * each slice ends waiting for all but the newest slice's loads. Slices past
  * ke - 1 reload ke - 1 so that every slice issues the same loads. Ends
@@ -583,125 +584,6 @@ __device__ __forceinline__ void qw8_mainloop(const qw_gemm_args &a, unsigned cha
     asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
 }
 
-/* Half tiles (128 x 256, bf16 W): a tile walk whose last wave of tiles
- * would leave at least half the CUs idle runs those tiles as twice as many
- * half tiles instead. Same 2 x 2 waves, each 64 x 128 (4 x 8 MFMA tiles);
- * the A stage holds 128 rows (4 direct loads per wave), the W stage is the
- * full tile's. Per 32-k sub-step: 32 MFMAs, 12 fragments (W block 0, A
- * blocks 0-3, W blocks 1-7), and under the held-back sub-step the 12 direct
- * loads of the next slice, one load and one read every 2 MFMAs. */
-template <bool PREV>
-__device__ __forceinline__ void qh_slice(const QgCtx &c, floatx4 (&acc)[8][8], bf16x8 (&pa)[8],
-                                         bf16x8 (&pw)[8], const unsigned char *__restrict__ cur,
-                                         unsigned char *__restrict__ nxt, uint32_t k_next) {
-    const uint32_t nl = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)nxt;
-    auto dma = [&](int j) __attribute__((always_inline)) {
-        if (j < 4)
-            gemm_dma16(c.a_rs4, nl + c.dst0 + j * 1024, c.a_dvoff[j], k_next * 2);
-        else
-            gemm_dma16(c.w_rs4, nl + QG_A_BYTES + c.wdst0 + (j - 4) * 1024, c.w_dvoff[j - 4],
-                       k_next * 2);
-    };
-    auto rd = [&](int ks, int j, bf16x8(&A)[8], bf16x8(&W)[8]) __attribute__((always_inline)) {
-        if (j == 0)
-            W[0] = *(const bf16x8 *)(cur + QG_A_BYTES + c.w_frag + c.ch[ks]);
-        else if (j <= 4)
-            A[j - 1] = *(const bf16x8 *)(cur + c.a_frag + (j - 1) * 2048 + c.ch[ks]);
-        else
-            W[j - 4] = *(const bf16x8 *)(cur + QG_A_BYTES + c.w_frag + (j - 4) * 2048 + c.ch[ks]);
-    };
-    bf16x8 af[8], bw[8], af1[8], bw1[8];
-    if (PREV) {
-        qg_ready(pw);
-        qg_ready(pa);
-#pragma unroll
-        for (int i = 0; i < 32; i++) {
-            QG_MFMA(acc[i & 3][i >> 2], pw[i >> 2], pa[i & 3]);
-            if ((i & 1) == 0 && (i >> 1) < 12) dma(i >> 1);
-            if ((i & 1) == 1 && (i >> 1) < 12) rd(0, i >> 1, af, bw);
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < 12; j++) dma(j);
-#pragma unroll
-        for (int j = 0; j < 12; j++) rd(0, j, af, bw);
-    }
-#pragma unroll
-    for (int i = 0; i < 32; i++) {
-        if (PREV)
-            QG_MFMA(acc[i & 3][i >> 2], bw[i >> 2], af[i & 3]);
-        else
-            QG_MFMA0(acc[i & 3][i >> 2], bw[i >> 2], af[i & 3]);
-        if ((i & 1) == 1 && (i >> 1) < 12) rd(1, i >> 1, af1, bw1);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++) pa[i] = af1[i];
-#pragma unroll
-    for (int i = 0; i < 8; i++) pw[i] = bw1[i];
-}
-
-/* Sums of the half tile at rows [m0, m0 + 128), columns [n0, n0 + 256) over
- * all of K into acc[0..3][*]; ends with the LDS stages free. */
-template <bool GLU>
-__device__ __forceinline__ void qh_mainloop(const qw_gemm_args &a, unsigned char *lds,
-                                            unsigned char *lds_b, uint32_t m0, uint32_t n0,
-                                            floatx4 (&acc)[8][8]) {
-    const uint32_t tid = threadIdx.x, lane = tid & 63;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t wm = wave >> 1, wn = wave & 1;
-    QgCtx c;
-    const uint32_t lrow = lane >> 3, lp = lane & 7;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const uint32_t r = wave * 32 + j * 8 + lrow;
-        c.a_dvoff[j] = (min(m0 + r, a.m - 1) * a.lda + (lp ^ ((r >> 1) & 7u)) * 8) * 2;
-    }
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const uint32_t r = wave * 64 + j * 8 + lrow;
-        c.w_dvoff[j] = (qg_wrow<GLU>(a, n0, r) * a.k + (lp ^ ((r >> 1) & 7u)) * 8) * 2;
-    }
-    c.a_rs4 = gemm_rs4(a.a, a.a_bytes);
-    c.w_rs4 = gemm_rs4(a.w, a.w_bytes);
-    c.dst0 = wave * 32 * 128;
-    c.wdst0 = wave * 64 * 128;
-    const uint32_t l16 = lane & 15, h = lane >> 4, swz = (l16 >> 1) & 7u;
-    c.a_frag = (wm * 64 + l16) * 128;
-    c.w_frag = (wn * 128 + l16) * 128;
-    c.ch[0] = ((0 + h) ^ swz) << 4;
-    c.ch[1] = ((4 + h) ^ swz) << 4;
-    const uint32_t KT = a.k / GBK;
-    {
-        const uint32_t nb =
-            (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds;
-#pragma unroll
-        for (int j = 0; j < 4; j++) gemm_dma16(c.a_rs4, nb + c.dst0 + j * 1024, c.a_dvoff[j], 0);
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-            gemm_dma16(c.w_rs4, nb + QG_A_BYTES + c.wdst0 + j * 1024, c.w_dvoff[j], 0);
-    }
-    QW_SLICE_END();
-    bf16x8 pa[8], pw[8];
-    qh_slice<false>(c, acc, pa, pw, lds, lds_b, (1 < KT ? 1 : 0) * GBK);
-    QW_SLICE_END();
-    uint32_t kt = 1;
-    for (; kt + 1 < KT; kt += 2) {
-        qh_slice<true>(c, acc, pa, pw, lds_b, lds, (kt + 1) * GBK);
-        QW_SLICE_END();
-        qh_slice<true>(c, acc, pa, pw, lds, lds_b, (kt + 2 < KT ? kt + 2 : kt + 1) * GBK);
-        QW_SLICE_END();
-    }
-    if (kt < KT) {
-        qh_slice<true>(c, acc, pa, pw, lds_b, lds, kt * GBK);
-        QW_SLICE_END();
-    }
-    qg_ready(pw);
-    qg_ready(pa);
-#pragma unroll
-    for (int i = 0; i < 32; i++) QG_MFMA(acc[i & 3][i >> 2], pw[i >> 2], pa[i & 3]);
-    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
-}
-
 /* INT8: 0 bf16 W, 1 int8 W widened once per workgroup */
 template <int INT8, bool GLU>
 __device__ __forceinline__ void qg_mainloop_any(const qw_gemm_args &a, unsigned char *lds,
@@ -713,24 +595,18 @@ __device__ __forceinline__ void qg_mainloop_any(const qw_gemm_args &a, unsigned 
         qg_mainloop<8, GLU>(a, lds, lds_b, tm, tn, kb, ke, acc);
 }
 
-/* The epilogue of the tile (MB = 8), 224-row tile (MB = 7) or half tile
- * (MB = 4) whose rows start at m0 and columns at n0: each wave's MB x 8
- * accumulator blocks. */
-template <int EPI, int INT8, int MB>
-__device__ __forceinline__ void qg_finish_at(const qw_gemm_args &a, unsigned char *lds,
-                                             unsigned char *lds_b, uint32_t m0, uint32_t n0,
-                                             floatx4 (&acc)[8][8], float *pst = nullptr,
-                                             const float *pld = nullptr, uint32_t npart = 0,
-                                             uint32_t own = 0) {
-    const uint32_t tid = threadIdx.x, lane = tid & 63;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t wm = wave >> 1, wn = wave & 1;
-    const uint32_t row0 = m0 + wm * (MB * 16), col0 = n0 + wn * 128;
-    constexpr uint32_t LDF = 128 + 4, REG = 32 * LDF * 4;
-    /* waves 0, 1 stage through `lds`, 2, 3 through `lds_b` (free after the
-     * loop's last barrier), one 32-row slab (16.5 KB) at a time */
-    float *region = (float *)((wave < 2 ? lds : lds_b) + (wave & 1) * REG);
-    const uint32_t poff = wm * 128 * 256 + wn * 128;
+/* The epilogue of one wave's MB x 8 accumulator blocks, whose rows start at
+ * row0 and columns at col0 (EPI_SWIGLU: output columns at f0), staged through
+ * the wave's LDS region. poff: the block's place in a split-tile partial. */
+#define QG_REGION (32 * (128 + 4) * 4) /* bytes of staging per wave */
+template <int EPI, int INT8, int MB, int AR>
+__device__ __forceinline__ void qg_finish_wave(const qw_gemm_args &a, float *region, uint32_t row0,
+                                               uint32_t col0, uint32_t f0, uint32_t poff,
+                                               floatx4 (&acc)[AR][8], float *pst = nullptr,
+                                               const float *pld = nullptr, uint32_t npart = 0,
+                                               uint32_t own = 0) {
+    const uint32_t lane = threadIdx.x & 63;
+    constexpr uint32_t LDF = 128 + 4;
     /* slab mi: rows SB 16 mi + 16 q + lane % 16 (tile mb = SB mi + q), columns
      * 32 ni + 16 p + 4 (lane / 16) + 0..3 (tile nb = 2 ni + p); SB = 2 blocks
      * of 16 rows per slab, 1 for an odd block count (224-row tiles). Columns
@@ -771,7 +647,6 @@ __device__ __forceinline__ void qg_finish_at(const qw_gemm_args &a, unsigned cha
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] = v0[j], v[4 + j] = v1[j];
             };
-            const uint32_t f0 = n0 / 2 + wn * 64;
             if (pld)
                 gemm_epilogue_swiglu<INT8, MB / SB, 16 * SB, 2>(a, write_slab, read_half, row0, f0,
                                                                 lane, pld + poff, npart, own);
@@ -784,9 +659,27 @@ __device__ __forceinline__ void qg_finish_at(const qw_gemm_args &a, unsigned cha
         }
         return;
     } else
-    gemm_epilogue_lds<EPI, INT8, MB / SB, 16 * SB, 4 * SB>(a, write_slab, read_row, row0, col0, lane,
-                                            pst ? pst + poff : nullptr,
-                                            pld ? pld + poff : nullptr, npart, own);
+        gemm_epilogue_lds<EPI, INT8, MB / SB, 16 * SB, 4 * SB>(
+            a, write_slab, read_row, row0, col0, lane, pst ? pst + poff : nullptr,
+            pld ? pld + poff : nullptr, npart, own);
+}
+
+/* The epilogue of the tile (MB = 8), 224-row tile (MB = 7) or half tile
+ * (MB = 4) whose rows start at m0 and columns at n0: each wave's MB x 8
+ * accumulator blocks. */
+template <int EPI, int INT8, int MB>
+__device__ __forceinline__ void qg_finish_at(const qw_gemm_args &a, unsigned char *lds,
+                                             unsigned char *lds_b, uint32_t m0, uint32_t n0,
+                                             floatx4 (&acc)[8][8], float *pst = nullptr,
+                                             const float *pld = nullptr, uint32_t npart = 0,
+                                             uint32_t own = 0) {
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wm = wave >> 1, wn = wave & 1;
+    /* waves 0, 1 stage through `lds`, 2, 3 through `lds_b` (free after the
+     * loop's last barrier), one 32-row slab (16.5 KB) at a time */
+    float *region = (float *)((wave < 2 ? lds : lds_b) + (wave & 1) * QG_REGION);
+    qg_finish_wave<EPI, INT8, MB>(a, region, m0 + wm * (MB * 16), n0 + wn * 128, n0 / 2 + wn * 64,
+                                  wm * 128 * 256 + wn * 128, acc, pst, pld, npart, own);
 }
 
 template <int EPI, int INT8>
@@ -831,10 +724,7 @@ __device__ __forceinline__ void qg_impl(const qw_gemm_args &a, unsigned char *ld
                     if ((H & 15u) == 0) hq = (hq & 7u) * (H >> 3) + (hq >> 3);
                     gemm_tile_at(a, F + (hq >> 1), tm, tn);
                     const uint32_t m0 = tm * 256 + (hq & 1) * 128;
-                    if (a.half3)
-                        qg_mainloop3<GLU>(a, lds, m0 / 128, tn, 0, KT, acc);
-                    else
-                        qh_mainloop<GLU>(a, lds, lds_b, m0, tn * 256, acc);
+                    qg_mainloop3<GLU>(a, lds, m0 / 128, tn, 0, KT, acc);
                     qg_finish_at<EPI, INT8, 4>(a, lds, lds_b, m0, tn * 256, acc);
                 }
                 asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -847,30 +737,17 @@ __device__ __forceinline__ void qg_impl(const qw_gemm_args &a, unsigned char *ld
         qg_finish<EPI, INT8>(a, lds, lds_b, tm, tn, acc);
         return;
     }
-    /* piece of a split tile (k-range-major numbering, as gemm.h); with
-     * half_count set (bf16 W, a launch of at most half as many tiles as
-     * CUs) the split tiles run as half tiles, r = 2 tile + half */
+    /* piece of a split tile (k-range-major numbering, as gemm.h) */
     uint32_t &ticket = *(uint32_t *)(lds_b + QG_STAGE); /* reserved by QG_ENTRY */
-    const bool hs = !INT8 && a.half_count;
-    const uint32_t R = (nt - ndp) << (hs ? 1 : 0), S = a.split, np = R * S;
+    const uint32_t R = nt - ndp, S = a.split, np = R * S;
     uint32_t q = pid - ndp;
     if ((np & 7u) == 0) q = (q & 7u) * (np >> 3) + (q >> 3);
     const uint32_t piece = q / R, r = q % R;
     const uint32_t kb = piece * KT / S, ke = (piece + 1) * KT / S;
-    gemm_tile_at(a, ndp + (hs ? r >> 1 : r), tm, tn);
-    const uint32_t th = tm * 2 + (r & 1); /* half tile row (128 rows) */
+    gemm_tile_at(a, ndp + r, tm, tn);
     float *slots = a.sk_part + (size_t)r * S * QW_SPLIT_PART;
-    if constexpr (!INT8) {
-        if (hs) {
-            qg_mainloop<4, GLU>(a, lds, lds_b, th, tn, kb, ke, acc);
-            qg_finish_at<EPI, INT8, 4>(a, lds, lds_b, th * 128, tn * 256, acc,
-                                       slots + (size_t)piece * QW_SPLIT_PART);
-        }
-    }
-    if (!hs) {
-        qg_mainloop_any<INT8, GLU>(a, lds, lds_b, tm, tn, kb, ke, acc);
-        qg_finish<EPI, INT8>(a, lds, lds_b, tm, tn, acc, slots + (size_t)piece * QW_SPLIT_PART);
-    }
+    qg_mainloop_any<INT8, GLU>(a, lds, lds_b, tm, tn, kb, ke, acc);
+    qg_finish<EPI, INT8>(a, lds, lds_b, tm, tn, acc, slots + (size_t)piece * QW_SPLIT_PART);
     __builtin_amdgcn_s_waitcnt(0x0F70); /* vmcnt(0): the partial's stores are done */
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __syncthreads();
@@ -880,12 +757,7 @@ __device__ __forceinline__ void qg_impl(const qw_gemm_args &a, unsigned char *ld
     __syncthreads();
     if (ticket != S - 1) return;
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    if constexpr (!INT8) {
-        if (hs)
-            qg_finish_at<EPI, INT8, 4>(a, lds, lds_b, th * 128, tn * 256, acc, nullptr, slots, S,
-                                       piece);
-    }
-    if (!hs) qg_finish<EPI, INT8>(a, lds, lds_b, tm, tn, acc, nullptr, slots, S, piece);
+    qg_finish<EPI, INT8>(a, lds, lds_b, tm, tn, acc, nullptr, slots, S, piece);
     if (threadIdx.x == 0)
         __hip_atomic_store(a.sk_flag + r, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -910,48 +782,6 @@ __device__ __forceinline__ void qg_impl_t224(const qw_gemm_args &a, unsigned cha
         qg_finish_at<EPI, 0, 7>(a, lds, lds_b, tm * 224, tn * 256, acc);
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
-}
-
-/* Small launches (at most cus / 2 tiles, bf16 W) as half tiles on the
- * three-stage loop, one half tile -- or one k-range piece of one, when
- * a.split > 1 -- per workgroup: grid = 2 tiles x split. Pieces meet as in
- * qg_impl (k-range-major numbering, the last one in adds them in piece
- * order and runs the epilogue). */
-template <int EPI>
-__device__ __forceinline__ void qg_impl_h3(const qw_gemm_args &a, unsigned char *lds) {
-    const uint32_t KT = a.k / GBK;
-    const uint32_t R = 2 * a.tiles_m * a.tiles_n, S = a.split > 1 ? a.split : 1, np = R * S;
-    uint32_t q = blockIdx.x;
-    if (q >= np) return;
-    if ((np & 7u) == 0) q = (q & 7u) * (np >> 3) + (q >> 3);
-    const uint32_t piece = q / R, r = q % R;
-    const uint32_t kb = piece * KT / S, ke = (piece + 1) * KT / S;
-    uint32_t tm, tn;
-    gemm_tile_at(a, r >> 1, tm, tn);
-    const uint32_t th = tm * 2 + (r & 1);
-    floatx4 acc[8][8];
-    qg_mainloop3<EPI == QW_EPI_SWIGLU>(a, lds, th, tn, kb, ke, acc);
-    unsigned char *lds_b = lds + QG_STAGE;
-    if (S == 1) {
-        qg_finish_at<EPI, 0, 4>(a, lds, lds_b, th * 128, tn * 256, acc);
-        return;
-    }
-    uint32_t &ticket = *(uint32_t *)(lds + 3 * QG3_STAGE); /* reserved by QG_ENTRY_H3 */
-    float *slots = a.sk_part + (size_t)r * S * QW_SPLIT_PART;
-    qg_finish_at<EPI, 0, 4>(a, lds, lds_b, th * 128, tn * 256, acc,
-                            slots + (size_t)piece * QW_SPLIT_PART);
-    __builtin_amdgcn_s_waitcnt(0x0F70); /* vmcnt(0): the partial's stores are done */
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __syncthreads();
-    if (threadIdx.x == 0)
-        ticket = __hip_atomic_fetch_add(a.sk_flag + r, 1u, __ATOMIC_RELAXED,
-                                        __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (ticket != S - 1) return;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    qg_finish_at<EPI, 0, 4>(a, lds, lds_b, th * 128, tn * 256, acc, nullptr, slots, S, piece);
-    if (threadIdx.x == 0)
-        __hip_atomic_store(a.sk_flag + r, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 /* One LDS array fixes the layout: the first stage at offset 0, the second
@@ -988,14 +818,4 @@ QG_ENTRY_T224(qw_gemm_bf16_gelu_t224, QW_EPI_GELU)
 QG_ENTRY_T224(qw_gemm_bf16_gate_t224, QW_EPI_GATE)
 QG_ENTRY_T224(qw_gemm_bf16_qkn_t224, QW_EPI_QKNORM)
 QG_ENTRY_T224(qw_gemm_bf16_swiglu_t224, QW_EPI_SWIGLU)
-/* bf16 W, small launches: half tiles on three stages */
-#define QG_ENTRY_H3(name, EPI)                                                                 \
-    QW_KERNEL void __launch_bounds__(256, 1) name(qw_gemm_args a) {                            \
-        __shared__ __attribute__((aligned(16))) unsigned char smem[3 * QG3_STAGE + 16];         \
-        qg_impl_h3<EPI>(a, smem);                                                              \
-    }
-QG_ENTRY_H3(qw_gemm_bf16_store_h3, QW_EPI_STORE)
-QG_ENTRY_H3(qw_gemm_bf16_gelu_h3, QW_EPI_GELU)
-QG_ENTRY_H3(qw_gemm_bf16_gate_h3, QW_EPI_GATE)
-QG_ENTRY_H3(qw_gemm_bf16_qkn_h3, QW_EPI_QKNORM)
-QG_ENTRY_H3(qw_gemm_bf16_swiglu_h3, QW_EPI_SWIGLU)
+#include "gemm_s.h"

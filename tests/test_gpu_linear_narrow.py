@@ -1,0 +1,112 @@
+"""Narrow tiles (64-256 rows x 128 columns, in k-range pieces where tiles are
+few) against the oracle, at the edges of their tiles, columns and k-ranges,
+and the wide tiles at shapes that narrow ones would otherwise take."""
+import numpy as np
+import pytest
+
+import test_gpu_kernels as K
+from test_gpu_kernels import assert_gelu_close, assert_linear_close, bf16_neighbours, synth, ulp_diff
+
+pytestmark = pytest.mark.gpu
+
+# rows, k, n: one k-slice; fewer slices than stages; ragged columns; a piece
+# per few slices; one and two rows past a tile; each tile height; each with a
+# last tile row on narrow tiles below wide ones (4119 and 2305 rows)
+SHAPES = [(9, 64, 8), (9, 4096, 8), (65, 128, 136), (63, 8192, 264), (257, 512, 1032),
+          (700, 64, 3072), (320, 1024, 12288), (640, 128, 9216), (700, 4096, 3072),
+          (1100, 2048, 1032), (300, 8192, 1544), (577, 320, 9216), (4119, 512, 4096),
+          (2305, 1024, 7176)]
+
+
+def _operands(gpu, oracle, rows, k, n, int8):
+    x, w = synth(oracle, rows * k, 71), synth(oracle, n * k, 72, 0.02)
+    b = synth(oracle, n, 73, 0.02)
+    if int8:
+        q, s = oracle.quantize_int8_rows(w, n, k)
+        lin = oracle.linear_i8(x, q, s, b, rows, k, n)
+        wt, st = gpu.put(q), gpu.put(s)
+    else:
+        lin, wt, st = oracle.linear(x, w, b, rows, k, n), gpu.put(w), None
+    mag = oracle.bf16_to_f32(oracle.linear(x & np.uint16(0x7FFF), w & np.uint16(0x7FFF), None,
+                                           rows, k, n)).ravel()
+    return gpu.put(x), wt, st, gpu.put(b), lin.ravel(), mag
+
+
+@pytest.mark.parametrize("rows,k,n", SHAPES)
+def test_narrow_tiles_store_gelu_gate(gpu, qd, oracle, rows, k, n):
+    int8 = (rows + n) % 3 == 0
+    xt, wt, st, bt, lin, mag = _operands(gpu, oracle, rows, k, n, int8)
+    pad = 8  # the gap between output rows and the rows past the last stay untouched
+    out = gpu.put(np.full((rows + 1) * (n + pad), 0x1234, np.uint16))
+    for _ in range(2):  # the pieces' counters are back at zero for a second call
+        gpu.linear(out, xt, wt, rows, k, n, bias=bt, wscale=st, ldc=n + pad)
+    gpu.submit()
+    got = out.read().reshape(rows + 1, n + pad)
+    assert (got[:, n:] == 0x1234).all() and (got[rows] == 0x1234).all()
+    assert_linear_close(oracle, np.ascontiguousarray(got[:rows, :n]).ravel(), lin, mag)
+    if rows <= 8 or n > 4096:
+        return
+    out = gpu.new(rows * n, qd.BF16)
+    gpu.linear(out, xt, wt, rows, k, n, bias=bt, wscale=st, epilogue=qd.LINEAR_GELU)
+    gpu.submit()
+    assert_gelu_close(oracle, out.read(), lin, mag)
+    mod, h0 = synth(oracle, 2 * 6 * n, 74, 0.5), synth(oracle, rows * n, 75)
+    rm = (np.arange(rows) % 3 == 1).astype(np.uint32)
+    out = gpu.put(h0)
+    gpu.linear(out, xt, wt, rows, k, n, bias=bt, wscale=st, epilogue=qd.LINEAR_GATE,
+               modulation=gpu.put(mod), row_map=gpu.put(rm), slots=6, gate_slot=2)
+    gpu.submit()
+    best = None  # the gate of y or of a bf16 neighbour of y, within one ulp
+    for yv in (lin,) + bf16_neighbours(lin):
+        want = np.empty(rows * n, np.uint16)
+        oracle.lib().qo_gate(want, h0, np.ascontiguousarray(yv), mod, rm, rows, n, 6, 2)
+        d = ulp_diff(out.read(), want)
+        best = d if best is None else np.minimum(best, d)
+    assert best.max() <= 1, best.max()
+
+
+@pytest.mark.parametrize("rows,k,heads", [(70, 512, 2), (320, 3072, 4), (640, 256, 24),
+                                          (4119, 512, 10)])
+def test_narrow_tiles_qknorm(gpu, qd, oracle, rows, k, heads):
+    """The q/k norm + RoPE epilogue bit for bit against the plain linear and
+    the standalone kernel (the same tiles, whatever the epilogue): rows past
+    a table's end wrap, and a last tile row's table rows start where it
+    does."""
+    n = 3 * heads * 128
+    xt, wt, _, bt, _, _ = _operands(gpu, oracle, rows, k, n, False)
+    rope_rows = 200
+    ang = np.random.default_rng(9).uniform(-3, 3, (rope_rows, 64)).astype(np.float32)
+    ct, st = gpu.put(np.cos(ang)), gpu.put(np.sin(ang))
+    nq, nk = gpu.put(synth(oracle, 128, 34, 0.1)), gpu.put(synth(oracle, 128, 35, 0.1))
+    fused, ref = gpu.new(rows * n, qd.BF16), gpu.new(rows * n, qd.BF16)
+    gpu.linear(fused, xt, wt, rows, k, n, bias=bt, epilogue=qd.LINEAR_QKNORM,
+               qknorm=(nq, nk, ct, st, rope_rows, 1e-6))
+    gpu.linear(ref, xt, wt, rows, k, n, bias=bt)
+    gpu.check(qd.lib().qw_gpu_qk_norm_rope_bf16(gpu.h, ref.h, rows, heads, n, n // 3, nq.h, nk.h,
+                                                 ct.h, st.h, rope_rows, 1e-6), "qk")
+    gpu.submit()
+    assert np.array_equal(fused.read(), ref.read())
+
+
+@pytest.mark.parametrize("n,int8", [(1800, False), (1784, True)])
+def test_wide_224_row_tiles(qd, oracle, monkeypatch, n, int8):
+    """The shapes of test_linear_224_row_tiles_ragged_cols with narrow tiles
+    off, so that the 224-row kernels run them."""
+    monkeypatch.setenv("QW_GEMM_HALF_SMALL", "0")
+    gpu = qd.Gpu()
+    try:
+        K.test_linear_224_row_tiles_ragged_cols(gpu, qd, oracle, n, int8)
+    finally:
+        gpu.close()
+
+
+@pytest.mark.parametrize("case", K.SPLIT_CASES)
+def test_wide_split_tiles(qd, oracle, monkeypatch, case):
+    """The shapes of test_linear_split_tiles with narrow tiles off, so that
+    the wide tiles' split pieces run them."""
+    monkeypatch.setenv("QW_GEMM_HALF_SMALL", "0")
+    gpu = qd.Gpu()
+    try:
+        K.test_linear_split_tiles(gpu, qd, oracle, *case)
+    finally:
+        gpu.close()
