@@ -34,7 +34,7 @@ enum {
     /* narrow tiles of 64, 128, 192 and 256 rows, each in the same order */
     K_GEMM_N1, K_GEMM_N1_LAST = K_GEMM_N1 + 4, K_GEMM_N2, K_GEMM_N2_LAST = K_GEMM_N2 + 4,
     K_GEMM_N3, K_GEMM_N3_LAST = K_GEMM_N3 + 4, K_GEMM_N4, K_GEMM_N4_LAST = K_GEMM_N4 + 4,
-    K_ATTN_W4,
+    K_ATTN_W4, K_ATTN_SPLIT, K_ATTN_W4_SPLIT,
     K_COUNT
 };
 static const char *k_names[K_COUNT] = {
@@ -54,7 +54,7 @@ static const char *k_names[K_COUNT] = {
     "qw_gemm_bf16_store_n2", "qw_gemm_bf16_gelu_n2", "qw_gemm_bf16_gate_n2", "qw_gemm_bf16_qkn_n2", "qw_gemm_bf16_swiglu_n2",
     "qw_gemm_bf16_store_n3", "qw_gemm_bf16_gelu_n3", "qw_gemm_bf16_gate_n3", "qw_gemm_bf16_qkn_n3", "qw_gemm_bf16_swiglu_n3",
     "qw_gemm_bf16_store_n4", "qw_gemm_bf16_gelu_n4", "qw_gemm_bf16_gate_n4", "qw_gemm_bf16_qkn_n4", "qw_gemm_bf16_swiglu_n4",
-    "qw_attention_w4_bf16"};
+    "qw_attention_w4_bf16", "qw_attention_split_bf16", "qw_attention_w4_split_bf16"};
 
 /* How int8 linears run (QW_INT8_ROUTE, a measurement switch): AUTO (the
  * default) widens the weight to a bf16 copy and runs the bf16 kernels when
@@ -99,7 +99,7 @@ struct h3_gpu {
     size_t widen_bytes;
     uint32_t cus;      /* compute units */
     float *sk_part;    /* split-tile partials: 256 x 256 fp32 each */
-    uint32_t *sk_flag; /* split-tile piece counters, 0 between launches */
+    uint32_t *sk_flag; /* split piece counters (QW_FLAGS a CU), 0 between launches */
     /* this device's copy of the static workspace (qw_static_scratch.hip):
      * partials, then QW_STATIC_FLAGS counters */
     unsigned char *static_scratch;
@@ -1025,14 +1025,14 @@ static double wide_us(h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t ksteps) 
  * that these replace; M = 100, K = 4096: 13 against 31). The weights cannot
  * come faster than 5 TB/s. Returns the least time and its mb and s. */
 static double narrow_us(const h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t ksteps,
-                        uint32_t *mb_out, uint32_t *s_out) {
+                        uint32_t max_s, uint32_t *mb_out, uint32_t *s_out) {
     static const double step_us[4] = {0.30, 0.39, 0.56, 0.70}, long_k[4] = {1.35, 1.3, 1.15, 1.0};
     const uint32_t C = g->cus, tn = (cols + 127) / 128;
     const double hbm_us = (double)cols * ksteps * 128 / 5e6;
     double best = 1e30;
     for (uint32_t mb = 1; mb <= 4; mb++) {
         const uint32_t R = (rows + 64 * mb - 1) / (64 * mb) * tn;
-        for (uint32_t s = 1; s <= 8; s++) {
+        for (uint32_t s = 1; s <= max_s; s++) {
             /* pieces of at least 4 k-steps, all in one round, a counter each */
             if (s > 1 && ((uint64_t)R * s > C || ksteps < 4 * s)) break;
             const double rounds = (double)(((uint64_t)R * s + C - 1) / C);
@@ -1052,6 +1052,14 @@ static double narrow_us(const h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t 
     return best;
 }
 
+/* Whether a launch may be split: the workspace is there, or can be made now
+ * (not while the stream is being captured into a graph). */
+static int can_split(h3_gpu *g) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return g->sk_part ||
+           (hipStreamIsCapturing(g->stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone);
+}
+
 /* How the rows of a linear on bf16 W run: the first `wide` of them (a
  * multiple of 256 when the rest are not none) on wide tiles, the rest on
  * narrow ones. A last tile row of few rows costs a whole round of wide tiles
@@ -1064,8 +1072,9 @@ static linear_plan plan_linear(h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t
     linear_plan p = {rows, 0, 1};
     if (!g->narrow) return p;
     uint32_t mb, s;
+    const uint32_t max_s = can_split(g) ? 8 : 1;
     double best = wide_us(g, rows, cols, ksteps);
-    const double all = narrow_us(g, rows, cols, ksteps, &mb, &s);
+    const double all = narrow_us(g, rows, cols, ksteps, max_s, &mb, &s);
     if (all < 0.98 * best) {
         best = all;
         p = {0, mb, s};
@@ -1073,24 +1082,26 @@ static linear_plan plan_linear(h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t
     const uint32_t rem = rows % 256;
     if (rem && rows > 256) {
         const double t = wide_us(g, rows - rem, cols, ksteps) +
-                         narrow_us(g, rem, cols, ksteps, &mb, &s);
+                         narrow_us(g, rem, cols, ksteps, max_s, &mb, &s);
         if (t < 0.97 * best) p = {rows - rem, mb, s};
     }
     return p;
 }
 
-/* partial sums and piece counters of split tiles, from the first one on */
+/* partial sums and piece counters of split tiles (and of split attention
+ * blocks), from the first one on */
+#define QW_FLAGS 4
 static int split_workspace(h3_gpu *g) {
     if (g->sk_part) return 1;
     hipStreamSynchronize(g->stream);
     const size_t n = (size_t)QW_SPLIT_MAX_PIECES * g->cus;
-    g->stats.allocated_bytes += n * 256 * 256 * 4 + (size_t)g->cus * 4;
+    g->stats.allocated_bytes += n * 256 * 256 * 4 + (size_t)g->cus * QW_FLAGS * 4;
     if (hipMalloc((void **)&g->sk_part, n * 256 * 256 * 4) != hipSuccess) {
         g->sk_part = NULL;
         return fail(g, "linear: split-tile workspace allocation failed");
     }
-    if (hipMalloc((void **)&g->sk_flag, (size_t)g->cus * 4) != hipSuccess ||
-        hipMemset(g->sk_flag, 0, (size_t)g->cus * 4) != hipSuccess) {
+    if (hipMalloc((void **)&g->sk_flag, (size_t)g->cus * QW_FLAGS * 4) != hipSuccess ||
+        hipMemset(g->sk_flag, 0, (size_t)g->cus * QW_FLAGS * 4) != hipSuccess) {
         hipFree(g->sk_part);
         g->sk_part = NULL;
         g->sk_flag = NULL;
@@ -1512,6 +1523,67 @@ extern "C" int h3_gpu_mlp_bf16(h3_gpu *g, h3_gpu_tensor *out, const h3_gpu_tenso
 
 /* ---- attention ----------------------------------------------------------- */
 
+/* How an attention launch fills the CUs. A block of 256 queries takes its
+ * CU 1.9 us a tile of 64 keys in full rounds (two waves per SIMD; 1.75 where
+ * part of the chip idles), a block of 128 queries 1.32 us alone on a CU and
+ * 2 us beside another; blocks that see few keys (text rows) fill in between.
+ * Rounds of blocks that leave a last one partly filled (or do not fill the
+ * first) are cut along the keys instead: the blocks past the full rounds
+ * (`dp`) in `split` pieces, each a share of the key tiles, that meet in
+ * memory (7 us, 1 to 1.5 more a piece, and the partials at 5 TB/s). 1 x 32
+ * heads x 4119 rows (544 blocks, 2.1 rounds) 344 -> 295 us; 24 heads, 4096
+ * queries of 8512 keys (1.5 rounds) 426 -> 373; 465 of 3323 72 -> 39. */
+#define QW_ATTN_PART(waves) ((size_t)(waves) * (16 * 1024 + 512)) /* bytes of a piece's partial */
+struct attn_plan {
+    int small; /* 128-query blocks */
+    uint32_t dp, split;
+};
+static attn_plan plan_attention(const h3_gpu *g, const qw_attention_desc *d) {
+    const uint32_t C = g->cus, pairs = d->heads * d->batch, T = (d->kv_rows + 63) / 64;
+    /* blocks of qb queries, and those of a (batch, head) pair that see few
+     * keys: the leading ones, all text */
+    auto blocks = [&](uint32_t qb) { return (d->q_rows + qb - 1) / qb; };
+    auto light = [&](uint32_t qb) {
+        return d->kv_limit || 2 * d->text_rows > d->kv_rows ? 0u : d->text_rows / qb;
+    };
+    const uint64_t nb8 = (uint64_t)blocks(256) * pairs;
+    if (nb8 >= C) {
+        const uint32_t per = blocks(256) - light(256);
+        const uint64_t heavy = (uint64_t)per * pairs, full = heavy / C, R = heavy % C;
+        attn_plan p = {0, 0, 1};
+        if (!R) return p;
+        /* whole blocks: the rounds and the partly filled one */
+        double best = 0.97 * 1.75 * T * (full + 1);
+        for (uint32_t s = 2; s <= 8 && T >= 4 * s; s++) {
+            const double t = 1.9 * (T * full + (R * s + C - 1) / C * ((T + s - 1) / s)) + 7.0 +
+                             1.5 * s + R * s * QW_ATTN_PART(8) * 2 / 5e6;
+            if (t < best) {
+                best = t;
+                p.split = s;
+            }
+        }
+        /* the first block past `full` rounds of heavy ones; pairs are walked
+         * in order, light blocks first */
+        const uint64_t h = full * C;
+        p.dp = (uint32_t)(h / per * blocks(256) + (h % per ? light(256) + h % per : 0));
+        return p;
+    }
+    const uint32_t heavy = (blocks(128) - light(128)) * pairs;
+    auto us = [&](uint32_t s) { /* time of the launch in s pieces a block */
+        const uint64_t n = (uint64_t)heavy * s;
+        return (double)((n + 2 * C - 1) / (2 * C)) * ((T + s - 1) / s) * (n <= C ? 1.32 : 2.0) +
+               (s > 1 ? 7.0 + s + n * QW_ATTN_PART(4) / 5e6 : 3.0);
+    };
+    attn_plan p = {1, 0, 1};
+    double best = 0.95 * us(1);
+    for (uint32_t s = 2; s <= 8 && T >= 2 * s; s++)
+        if (us(s) < best) {
+            best = us(s);
+            p.split = s;
+        }
+    return p;
+}
+
 extern "C" int qw_gpu_attention_bf16(h3_gpu *g, const qw_attention_desc *d) {
     if (!g || !d) return 0;
     REQ_DT(d->out, H3_GPU_BF16, "attention out");
@@ -1559,19 +1631,32 @@ extern "C" int qw_gpu_attention_bf16(h3_gpu *g, const qw_attention_desc *d) {
     g->stats.mps_sdpa_dispatches += 0;
     if (((uint64_t)(d->kv_rows - 1) * std::max(d->ldk, d->ldv) + hd) * 2 >= (1ull << 31))
         return fail(g, "attention: one batch entry's K/V exceed 2 GiB");
-    /* Fewer 256-query blocks than CUs: 128-query workgroups, two per CU,
-     * bring the idle CUs in (the same bits; 1 x 24 heads x 1152 rows 28.7
-     * against 44.3 us, 320 rows 13.4 against 18.8; at 2 x 24 x 4352 rows the
-     * 256-query kernel stays ahead, 391.5 against 398.9 us). */
+    a.dp_blocks = 0;
+    a.split = 1;
+    a.part = NULL;
+    a.flag = NULL;
     const uint32_t aqb = g->attn_threads / 2; /* 32 query rows per 64-lane wave */
     const uint64_t nwg = (uint64_t)((d->q_rows + aqb - 1) / aqb) * d->heads * d->batch;
     if (nwg >= (1ull << 31)) return fail(g, "attention: grid too large");
-    if (g->attn_small && nwg < g->cus) {
-        const uint32_t aqb4 = g->attn4_threads / 2;
-        const uint64_t nwg4 = (uint64_t)((d->q_rows + aqb4 - 1) / aqb4) * d->heads * d->batch;
-        return launch(g, K_ATTN_W4, dim3((uint32_t)nwg4), dim3(g->attn4_threads), a);
-    }
-    return launch(g, K_ATTN, dim3((uint32_t)nwg), dim3(g->attn_threads), a);
+    const attn_plan p = plan_attention(g, d);
+    /* the launch's own kernel: a small plan keeps its pieces on either */
+    const int w4 = p.small && g->attn_small;
+    const uint32_t threads = w4 ? g->attn4_threads : g->attn_threads, qb = threads / 2;
+    const uint32_t nb = (d->q_rows + qb - 1) / qb * d->heads * d->batch;
+    const uint64_t R = nb - p.dp, np = R * p.split;
+    /* whole blocks where the pieces would not fit the workspace (a counter
+     * a block, a partial a piece) or there is none to be had */
+    if (p.split == 1 || R > (uint64_t)QW_FLAGS * g->cus ||
+        np * QW_ATTN_PART(threads / 64) > (size_t)QW_SPLIT_MAX_PIECES * g->cus * 256 * 256 * 4 ||
+        !can_split(g))
+        return launch(g, w4 ? K_ATTN_W4 : K_ATTN, dim3(nb), dim3(threads), a);
+    if (!split_workspace(g)) return 0;
+    a.dp_blocks = p.dp;
+    a.split = p.split;
+    a.part = g->sk_part;
+    a.flag = g->sk_flag;
+    return launch(g, w4 ? K_ATTN_W4_SPLIT : K_ATTN_SPLIT, dim3((uint32_t)(p.dp + np)),
+                  dim3(threads), a);
 }
 
 static int sdpa_contig(h3_gpu *g, h3_gpu_tensor *out, const h3_gpu_tensor *q,

@@ -43,10 +43,25 @@
 #define A_TILE (AKT * 256)          /* one K or V tile: AKT keys x 128 bf16 */
 
 __device__ __forceinline__ uint32_t attn_limit(const qw_attn_args &a, uint32_t r) {
-    if (r >= a.q_rows) return 0;
+    r = min(r, a.q_rows - 1); /* rows past the last are computed as it and not stored */
     if (a.kv_limit) return min(a.kv_limit[r], a.kv_rows);
     if (r < a.text_rows) return a.text_causal ? r + 1 : a.text_rows;
     return a.kv_rows;
+}
+
+/* The least or greatest closed-form limit (no kv_limit table) of rows
+ * [r, r + n), rows past the last taken as it. */
+__device__ __forceinline__ uint32_t attn_bound(const qw_attn_args &a, uint32_t r, uint32_t n,
+                                               bool greatest) {
+    const uint32_t first = min(r, a.q_rows - 1), last = min(r + n, a.q_rows) - 1;
+    const uint32_t end = max(first, last);
+    uint32_t lo = a.kv_rows, hi = a.kv_rows;
+    if (first < a.text_rows) {
+        lo = a.text_causal ? first + 1 : a.text_rows;
+        hi = a.text_causal ? min(end + 1, a.text_rows) : a.text_rows;
+        if (end >= a.text_rows) lo = min(lo, a.kv_rows), hi = max(hi, a.kv_rows);
+    }
+    return greatest ? hi : lo;
 }
 
 /* Key of s[kbk][v] in a tile: kv0 + 32 kbk + 8 (v / 4) + 4 h + v % 4.
@@ -121,12 +136,21 @@ __device__ __forceinline__ void attn_barrier() {
 
 typedef __attribute__((address_space(3))) bf16x4 attn_lds_b4;
 
-/* 256 queries per workgroup: launches that fill the part */
+/* 256 queries per workgroup: launches that fill the part. The kernels with
+ * split blocks are entry points of their own, so that the loop of the others
+ * keeps its registers and its order. */
 #define ANW 8 /* waves per workgroup, 32 queries each */
 #define AQB (32 * ANW) /* queries per workgroup */
+#define QW_ATTN_SPLIT 0
 #define QW_ATTN_NAME qw_attention_bf16
 #include "attention_kernel.inc"
 #undef QW_ATTN_NAME
+#undef QW_ATTN_SPLIT
+#define QW_ATTN_SPLIT 1
+#define QW_ATTN_NAME qw_attention_split_bf16
+#include "attention_kernel.inc"
+#undef QW_ATTN_NAME
+#undef QW_ATTN_SPLIT
 #undef AQB
 #undef ANW
 
@@ -134,8 +158,15 @@ typedef __attribute__((address_space(3))) bf16x4 attn_lds_b4;
  * blocks than CUs (the 512^2 and 320-row configurations) */
 #define ANW 4
 #define AQB (32 * ANW)
+#define QW_ATTN_SPLIT 0
 #define QW_ATTN_NAME qw_attention_w4_bf16
 #include "attention_kernel.inc"
 #undef QW_ATTN_NAME
+#undef QW_ATTN_SPLIT
+#define QW_ATTN_SPLIT 1
+#define QW_ATTN_NAME qw_attention_w4_split_bf16
+#include "attention_kernel.inc"
+#undef QW_ATTN_NAME
+#undef QW_ATTN_SPLIT
 #undef AQB
 #undef ANW

@@ -186,6 +186,14 @@ typedef struct {
     int32_t text_causal;
     float scale;      /* softmax scale */
     float scale_log2; /* softmax scale * log2(e) */
+    /* Split blocks (the _split kernels): the first dp_blocks query blocks run
+     * one per workgroup, each later block r in `split` pieces of its key
+     * tiles, numbered piece-major; a piece keeps its unnormalised output, row
+     * maxima and sums in part, and the last to count itself in flag[r] (0
+     * between launches) adds them in piece order. */
+    uint32_t dp_blocks, split;
+    float *part;
+    uint32_t *flag;
 } qw_attn_args;
 
 /* LoRA fusion: out[rows, cols] = RNE(fp32(base) + sum of the terms) */
