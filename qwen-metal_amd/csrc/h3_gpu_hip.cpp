@@ -30,7 +30,7 @@ enum {
     K_WIDEN, K_LN_MOD_WIDE, K_EULER, K_LORA,
     K_GEMV_BF16_STORE, K_GEMV_BF16_GELU, K_GEMV_I8_STORE, K_GEMV_I8_GELU, K_ZERO,
     K_GEMM_W8_STORE_Q, K_GEMM_W8_GELU_Q, K_GEMM_W8_GATE_Q, K_GEMM_W8_QKN_Q, K_GEMM_W8_SWIGLU_Q,
-    K_GEMM_BF16_STORE_T224, K_GEMM_BF16_GELU_T224, K_GEMM_BF16_GATE_T224, K_GEMM_BF16_QKN_T224, K_GEMM_BF16_SWIGLU_T224,
+    K_GEMM_BF16_STORE_MIX, K_GEMM_BF16_GELU_MIX, K_GEMM_BF16_GATE_MIX, K_GEMM_BF16_QKN_MIX, K_GEMM_BF16_SWIGLU_MIX,
     /* narrow tiles of 64, 128, 192 and 256 rows, each in the same order */
     K_GEMM_N1, K_GEMM_N1_LAST = K_GEMM_N1 + 4, K_GEMM_N2, K_GEMM_N2_LAST = K_GEMM_N2 + 4,
     K_GEMM_N3, K_GEMM_N3_LAST = K_GEMM_N3 + 4, K_GEMM_N4, K_GEMM_N4_LAST = K_GEMM_N4 + 4,
@@ -48,8 +48,8 @@ static const char *k_names[K_COUNT] = {
     "qw_gemv_bf16_store", "qw_gemv_bf16_gelu", "qw_gemv_i8_store", "qw_gemv_i8_gelu",
     "qw_zero_u32",
     "qw_gemm_w8_store_q", "qw_gemm_w8_gelu_q", "qw_gemm_w8_gate_q", "qw_gemm_w8_qkn_q", "qw_gemm_w8_swiglu_q",
-    "qw_gemm_bf16_store_t224", "qw_gemm_bf16_gelu_t224", "qw_gemm_bf16_gate_t224",
-    "qw_gemm_bf16_qkn_t224", "qw_gemm_bf16_swiglu_t224",
+    "qw_gemm_bf16_store_mix", "qw_gemm_bf16_gelu_mix", "qw_gemm_bf16_gate_mix",
+    "qw_gemm_bf16_qkn_mix", "qw_gemm_bf16_swiglu_mix",
     "qw_gemm_bf16_store_n1", "qw_gemm_bf16_gelu_n1", "qw_gemm_bf16_gate_n1", "qw_gemm_bf16_qkn_n1", "qw_gemm_bf16_swiglu_n1",
     "qw_gemm_bf16_store_n2", "qw_gemm_bf16_gelu_n2", "qw_gemm_bf16_gate_n2", "qw_gemm_bf16_qkn_n2", "qw_gemm_bf16_swiglu_n2",
     "qw_gemm_bf16_store_n3", "qw_gemm_bf16_gelu_n3", "qw_gemm_bf16_gate_n3", "qw_gemm_bf16_qkn_n3", "qw_gemm_bf16_swiglu_n3",
@@ -86,10 +86,9 @@ struct h3_gpu {
     uint32_t attn4_threads; /* the same for the small launches' kernel */
     int attn_small; /* launches of fewer 256-query blocks than CUs on the 4-wave kernel (QW_ATTN_W4=0: off) */
     int int8_route; /* QW_INT8_* : how int8 linears of many rows run */
-    int t224;       /* 224-row tiles allowed (QW_GEMM_T224=0 turns them off, for measurement) */
+    int mixed;      /* 192- and 224-row tiles allowed (QW_GEMM_T224=0 turns them off, for measurement) */
     uint32_t split_min_steps, split_force; /* measurement: QW_SPLIT_MIN_STEPS, QW_SPLIT_FORCE */
     uint32_t widen_min_rows; /* int8: fewest rows for the widening route (QW_WIDEN_MIN_ROWS) */
-    int t224_over_split; /* 224-row tiles preferred to split tiles (QW_T224_OVER_SPLIT=0: off) */
     int narrow;     /* narrow tiles allowed (QW_GEMM_HALF_SMALL=0: off) */
     /* qw_gpu_span_*: event pairs recorded on the stream, read after a sync */
     hipEvent_t *span_ev;
@@ -203,16 +202,14 @@ extern "C" h3_gpu *h3_gpu_create(const char *code_object_path, char *error,
         if (!strcmp(r, "w8")) g->int8_route = QW_INT8_W8;
         else if (!strcmp(r, "widen")) g->int8_route = QW_INT8_WIDEN;
     }
-    g->t224 = 1;
-    if (const char *r = getenv("QW_GEMM_T224")) g->t224 = atoi(r) != 0;
+    g->mixed = 1;
+    if (const char *r = getenv("QW_GEMM_T224")) g->mixed = atoi(r) != 0;
     g->split_min_steps = 32;
     if (const char *r = getenv("QW_SPLIT_MIN_STEPS")) g->split_min_steps = (uint32_t)atoi(r);
     g->split_force = 0;
     if (const char *r = getenv("QW_SPLIT_FORCE")) g->split_force = (uint32_t)atoi(r);
     g->widen_min_rows = QW_WIDEN_MIN_ROWS;
     if (const char *r = getenv("QW_WIDEN_MIN_ROWS")) g->widen_min_rows = (uint32_t)atoi(r);
-    g->t224_over_split = 1;
-    if (const char *r = getenv("QW_T224_OVER_SPLIT")) g->t224_over_split = atoi(r) != 0;
     g->narrow = 1;
     if (const char *r = getenv("QW_GEMM_HALF_SMALL")) g->narrow = atoi(r) != 0;
     g->cus = 0;
@@ -981,38 +978,50 @@ static uint32_t split_choice(h3_gpu *g, uint32_t tiles, uint32_t ksteps,
     return best;
 }
 
-/* 224-row tiles where they leave fewer (work-weighted) waves than 256-row
- * tiles with their half-tile tail: a wave of 224-row tiles is 0.875 of one
- * of 256-row tiles. Out projection, M = 8704: 2 waves of 0.875 (468 tiles)
- * against 2 waves (408 tiles). */
-static int rule_224(const h3_gpu *g, uint32_t rows, uint32_t cols) {
-    if (!g->t224 || g->cus % 8) return 0;
-    const uint32_t C = g->cus, tn = (cols + 255) / 256, tiles = (rows + 255) / 256 * tn;
-    const uint32_t t224 = (rows + 223) / 224 * tn, R = tiles % C;
-    const double w256 = (double)(tiles / C) + (R ? (2 * R <= C ? 0.5 : 1.0) : 0.0);
-    return 0.875 * (double)((t224 + C - 1) / C) < 0.97 * w256;
-}
-
 /* Time models of a linear on bf16 W, in microseconds, that pick its tiles.
  *
- * Wide (gemm_q.h): a round of 256 x 256 tiles takes 1.3 us a k-step (64 k)
- * and 12 us for prologue and epilogue (measured at M = 1152-8704: 75-88 us a
+ * Wide (gemm_q.h): a round of 256-row tiles takes 1.3 us a k-step (64 k) and
+ * 12 us for prologue and epilogue (measured at M = 1152-8704: 75-88 us a
  * round at K = 3072, 92-102 at 4096, 274 at 12288); a partly filled last
  * round the length of split_choice's pieces and 8 + 0.055 R s^2 us for their
  * partial sums (M = 4119 against 4096, K = 4096: 59, 65 and 79 us for 16, 48
  * and 96 tail tiles in 2; K = 12288: 79 us for 16 in 6, 138 for 60 in 4), or
- * half a round on half tiles. */
-static double wide_us(h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t ksteps) {
+ * 0.6 of a round on half tiles. Mixed heights instead fill `n` rounds with T
+ * tile rows, as few of the taller as cover the rows; each CU's tiles, tallest
+ * first, in proportion to their heights. h1 = 0: 256-row tiles. */
+struct wide_plan {
+    double us;
+    uint32_t h1, h2, rows1, rows2;
+};
+static wide_plan plan_wide(h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t ksteps) {
     const uint32_t C = g->cus, tn = (cols + 255) / 256, tiles = (rows + 255) / 256 * tn;
-    const double round = 1.3 * ksteps + 12.0;
-    if (rule_224(g, rows, cols)) return 0.875 * round * (((rows + 223) / 224 * tn + C - 1) / C);
+    const double step = 1.3 * ksteps, fix = 12.0, round = step + fix;
     const uint32_t R = tiles % C, s = split_choice(g, tiles, ksteps);
-    double t = (double)(tiles / C) * round;
+    wide_plan p = {(double)(tiles / C) * round, 0, 0, 0, 0};
     if (s > 1)
-        t += (double)((R * s + C - 1) / C) / s * round + 8.0 + 0.055 * R * s * s;
+        p.us += (double)((R * s + C - 1) / C) / s * round + 8.0 + 0.055 * R * s * s;
     else if (R)
-        t += tiles > C && 2 * R <= C ? 0.5 * round : round;
-    return t;
+        p.us += tiles > C && 2 * R <= C ? 0.6 * round : round;
+    if (!g->mixed || C % 8) return p;
+    const uint32_t m32 = (rows + 31) / 32;
+    double best = 0.98 * p.us;
+    const uint32_t n0 = std::max(1u, (uint32_t)((uint64_t)m32 * tn / 8 / C));
+    for (uint32_t n = n0; n <= n0 + 2; n++) {
+        const uint32_t T = (uint32_t)((uint64_t)n * C / tn);
+        for (uint32_t h = 7; h >= 6; h--) { /* r1 rows of h + 1, r2 of h */
+            if (!T || (uint64_t)T * (h + 1) < m32) continue;
+            const uint32_t low = T * h;
+            const uint32_t r1 = m32 > low ? m32 - low : 0;
+            const uint32_t r2 = m32 > r1 * (h + 1) ? (m32 - r1 * (h + 1) + h - 1) / h : 0;
+            const uint32_t all = ((r1 + r2) * tn + C - 1) / C, tall = (r1 * tn + C - 1) / C;
+            const double us = tall * (step * (h + 1) / 8 + fix) + (all - tall) * (step * h / 8 + fix);
+            if (us < best) {
+                best = us;
+                p = {us, h + 1, h, r1, r2};
+            }
+        }
+    }
+    return p;
 }
 
 /* Narrow (gemm_s.h), tiles of 64 mb rows x 128 columns in s k-range pieces:
@@ -1067,23 +1076,29 @@ static int can_split(h3_gpu *g) {
  * for M = 4096), and one or two us per column of narrow tiles. */
 struct linear_plan {
     uint32_t wide, mb, s;
+    wide_plan w; /* how the first run */
 };
 static linear_plan plan_linear(h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t ksteps) {
-    linear_plan p = {rows, 0, 1};
+    linear_plan p = {rows, 0, 1, plan_wide(g, rows, cols, ksteps)};
     if (!g->narrow) return p;
     uint32_t mb, s;
     const uint32_t max_s = can_split(g) ? 8 : 1;
-    double best = wide_us(g, rows, cols, ksteps);
+    double best = p.w.us;
     const double all = narrow_us(g, rows, cols, ksteps, max_s, &mb, &s);
     if (all < 0.98 * best) {
         best = all;
-        p = {0, mb, s};
+        p = {0, mb, s, p.w};
     }
-    const uint32_t rem = rows % 256;
-    if (rem && rows > 256) {
-        const double t = wide_us(g, rows - rem, cols, ksteps) +
-                         narrow_us(g, rem, cols, ksteps, max_s, &mb, &s);
-        if (t < 0.97 * best) p = {rows - rem, mb, s};
+    /* the last, ragged tile row on narrow tiles, or up to three more with it */
+    for (uint32_t j = 0; j < 4; j++) {
+        const uint32_t rem = rows % 256 + 256 * j;
+        if (!rem || rows < rem + 256) continue;
+        const wide_plan w = plan_wide(g, rows - rem, cols, ksteps);
+        const double t = w.us + narrow_us(g, rem, cols, ksteps, max_s, &mb, &s);
+        if (t < 0.97 * best) {
+            best = t;
+            p = {rows - rem, mb, s, w};
+        }
     }
     return p;
 }
@@ -1222,27 +1237,26 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc) {
      * VALU work (1.5 instructions per weight per workgroup): the same
      * kernel with the conversion left out runs as fast as the widening
      * pass plus the bf16 kernel. */
-    const int rule224 = rule_224(g, d->rows, d->cols); /* on whole tiles, bf16 kernels */
+    const linear_plan wide_all = {d->rows, 0, 1, plan_wide(g, d->rows, d->cols, d->k / 64)};
+    linear_plan plan = no_alloc || (int8 && g->int8_route == QW_INT8_W8)
+                           ? wide_all : plan_linear(g, d->rows, d->cols, d->k / 64);
     /* K >= 8192 keeps the in-LDS widening, unless the widened weight's bf16
-     * kernel takes 224-row tiles (the down projection at M = 8704: whole
+     * kernel takes lower tiles (224-row ones for the down projection at M = 8704: whole
      * steps 64.07 against 65.39 ms with the pass and 224-row tiles, medians
      * of 8, same box, alternating) */
     int route = g->int8_route;
     if (route == QW_INT8_AUTO)
-        route = d->k >= 8192 && !(rule224 && g->t224_over_split) ? QW_INT8_W8 : QW_INT8_WIDEN;
+        route = d->k >= 8192 && !wide_all.w.h1 ? QW_INT8_W8 : QW_INT8_WIDEN;
     /* Where the bf16 kernels take narrow tiles, for all rows or for the last
      * few, the weight is widened by a pass at any row count and K: they beat
      * the whole "_w8" tiles by more than the pass costs (M = 64-448, us, w8 /
      * pass + 128 x 256 half tiles, which narrow tiles beat in turn: QKV
      * 64-66 / 48-55, out 63 / 35-38, up 65-67 / 56-59, down 74-84 / 66-76). */
-    linear_plan plan = {d->rows, 0, 1};
-    if (!no_alloc && (!int8 || g->int8_route != QW_INT8_W8))
-        plan = plan_linear(g, d->rows, d->cols, d->k / 64);
     const int small_w = g->int8_route == QW_INT8_AUTO && plan.mb != 0;
     if (small_w) route = QW_INT8_WIDEN;
     const int widen = int8 && !no_alloc && (d->rows >= g->widen_min_rows || small_w) &&
                       route == QW_INT8_WIDEN;
-    if (int8 && !widen) plan = {d->rows, 0, 1};
+    if (int8 && !widen) plan = wide_all;
     const void *wptr = d->weight->ptr;
     if (widen) {
         const size_t n = (size_t)d->cols * d->k, bytes = n * 2;
@@ -1300,6 +1314,7 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc) {
     a.half_from = 0;
     a.half_count = 0;
     a.m_base = 0;
+    a.mix_h1 = a.mix_h2 = a.mix_rows1 = a.mix_rows2 = a.mix_dealt = 0;
     a.sk_part = NULL;
     a.sk_flag = NULL;
     if (plan.mb) { /* the rows past plan.wide on narrow tiles */
@@ -1332,8 +1347,7 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc) {
     a.dp_tiles = tiles;
     a.split = 1;
     uint32_t grid = tiles;
-    const uint32_t t224 = ((rows + 223) / 224) * a.tiles_n;
-    const int use224 = !(int8 && !widen) && rule_224(g, rows, d->cols);
+    const int mix = !(int8 && !widen) && plan.w.h1;
     if (no_alloc) {
         const uint32_t s = split_choice(g, tiles, d->k / 64, QW_STATIC_PARTS);
         if (s > 1) {
@@ -1359,11 +1373,10 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc) {
             grid = a.dp_tiles + R * s;
         }
     } else {
-        /* where 224-row tiles fill the waves better they also beat split
-         * tiles (down projection shape, bf16 W, M = 8704: 500 us unsplit on
-         * 224-row tiles against 568 with 256-row tiles and a 3-piece tail) */
-        const uint32_t s =
-            use224 && g->t224_over_split ? 1u : split_choice(g, tiles, d->k / 64);
+        /* where mixed heights fill the rounds they also beat split tiles
+         * (down projection shape, bf16 W, M = 8704: 500 us on 224-row tiles
+         * against 568 with 256-row tiles and a 3-piece tail) */
+        const uint32_t s = mix ? 1u : split_choice(g, tiles, d->k / 64);
         if (s > 1) {
             if (!split_workspace(g)) return 0;
             const uint32_t R = tiles % g->cus;
@@ -1382,10 +1395,20 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc) {
      * the tiles, so a tile's output stores drain under the next tile's first
      * loads (up 521 -> 514 us, QKV 365 -> 359 us against one workgroup per
      * tile) */
-    if (a.split == 1 && use224) {
-        a.tiles_m = (rows + 223) / 224;
-        return launch(g, K_GEMM_BF16_STORE_T224 + d->epilogue,
-                      dim3(t224 < g->cus ? t224 : g->cus), dim3(threads), a);
+    if (a.split == 1 && mix) {
+        a.mix_h1 = plan.w.h1;
+        a.mix_h2 = plan.w.h2;
+        a.mix_rows1 = plan.w.rows1;
+        a.mix_rows2 = plan.w.rows2;
+        /* few tile columns: an XCD's share of the ids as they are dealt (one
+         * row of each group of 4, every second column) spans no more panels
+         * than a range of tiles does, and at long K their slices stay in step
+         * better (down projection, M = 8704, int8 weights, 240 + 264 tiles:
+         * 500 against 530 us; at 36 and more columns a range is 3-7% ahead) */
+        a.mix_dealt = a.tiles_n <= 16 && d->k >= 8192;
+        const uint32_t n = (a.mix_rows1 + a.mix_rows2) * a.tiles_n;
+        return launch(g, K_GEMM_BF16_STORE_MIX + d->epilogue, dim3(n < g->cus ? n : g->cus),
+                      dim3(threads), a);
     }
     if (a.split == 1 && grid > g->cus && g->cus % 8 == 0) {
         grid = g->cus;

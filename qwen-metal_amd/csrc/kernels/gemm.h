@@ -157,20 +157,30 @@ QW_KERNEL void __launch_bounds__(256) qw_gemv_i8_gelu(qw_gemm_args a) {
  * 8 XCDs; the id is remapped so each XCD owns a contiguous range of tiles,
  * walked in groups of 4 tile-rows (column-major inside a group), so the A
  * and W panels an XCD touches stay hot in its L2. */
-__device__ __forceinline__ void gemm_tile_at(const qw_gemm_args &a, uint32_t pid, uint32_t &tm,
-                                             uint32_t &tn) {
+__device__ __forceinline__ void gemm_tile_in(uint32_t tiles_m, uint32_t tiles_n, uint32_t pid,
+                                             uint32_t &tm, uint32_t &tn) {
 #ifndef QW_GEMM_GROUP
 /* 4 against 8 (same box, alternating, M = 8704): QKV 381 / 388, out 150 /
  * 152, up 509 / 514, down 572 / 578 us (medians), steps 66.15 / 66.62 ms */
 #define QW_GEMM_GROUP 4
 #endif
     const uint32_t G = QW_GEMM_GROUP;
-    const uint32_t per_group = G * a.tiles_n;
+    const uint32_t per_group = G * tiles_n;
     const uint32_t first_m = (pid / per_group) * G;
-    const uint32_t gsize = min(a.tiles_m - first_m, G);
+    const uint32_t gsize = min(tiles_m - first_m, G);
     const uint32_t inner = pid % per_group;
     tm = first_m + inner % gsize;
     tn = inner / gsize;
+}
+__device__ __forceinline__ void gemm_tile_at(const qw_gemm_args &a, uint32_t pid, uint32_t &tm,
+                                             uint32_t &tn) {
+    gemm_tile_in(a.tiles_m, a.tiles_n, pid, tm, tn);
+}
+/* id -> its place among n when each residue class mod 8 (one XCD, as ids are
+ * dealt) takes one contiguous range, for any n */
+__device__ __forceinline__ uint32_t gemm_xcd_range(uint32_t id, uint32_t n) {
+    const uint32_t x = id & 7u;
+    return x * (n >> 3) + min(x, n & 7u) + (id >> 3);
 }
 /* Epilogue through LDS: the fp32 sums of each 32-row slab of the wave's
  * block are first written to a wave-private LDS region (row stride

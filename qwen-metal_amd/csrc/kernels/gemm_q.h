@@ -64,12 +64,14 @@ struct QgCtx {
  * widening, register copies) is placed before it, and supplies the 2. */
 template <int N = 8>
 __device__ __forceinline__ void qg_ready(const bf16x8 (&f)[8]) {
-    static_assert(N == 4 || N == 7 || N == 8, "fragment count");
+    static_assert(N == 4 || N == 6 || N == 7 || N == 8, "fragment count");
     if constexpr (N == 8)
         asm volatile("s_nop 1" ::"v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(f[4]), "v"(f[5]),
                      "v"(f[6]), "v"(f[7]));
     else if constexpr (N == 4)
         asm volatile("s_nop 1" ::"v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]));
+    else if constexpr (N == 6)
+        asm volatile("s_nop 1" ::"v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(f[4]), "v"(f[5]));
     else
         asm volatile("s_nop 1" ::"v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(f[4]), "v"(f[5]),
                      "v"(f[6]));
@@ -162,17 +164,18 @@ __device__ __forceinline__ void qg_slice(const QgCtx &c, floatx4 (&acc)[8][8], b
     for (int i = 0; i < 8; i++) pw[i] = bw1[i];
 }
 
-/* Sums of tile (tm, tn) over k-steps [kb, ke) into acc; ends with the LDS
- * stages free (after a barrier). MB = 8: 256-row tiles; MB = 7: 224-row
- * tiles (each wave's 112 rows; the A stage's last 32 rows unused). */
+/* Sums of the tile at rows m0, tile column tn over k-steps [kb, ke) into acc;
+ * ends with the LDS stages free (after a barrier). MB = 8: 256-row tiles; MB
+ * = 7, 6: 224- and 192-row tiles (each wave's 16 MB rows; the rest of the A
+ * stage unused). */
 template <int MB = 8, bool GLU = false>
 __device__ __forceinline__ void qg_mainloop(const qw_gemm_args &a, unsigned char *lds,
-                                            unsigned char *lds_b, uint32_t tm, uint32_t tn,
+                                            unsigned char *lds_b, uint32_t m0, uint32_t tn,
                                             uint32_t kb, uint32_t ke, floatx4 (&acc)[8][8]) {
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wm = wave >> 1, wn = wave & 1;
-    const uint32_t m0 = tm * (MB * 32), n0 = tn * 256;
+    const uint32_t n0 = tn * 256;
     QgCtx c;
     const uint32_t lrow = lane >> 3, lp = lane & 7;
 #pragma unroll
@@ -592,7 +595,7 @@ __device__ __forceinline__ void qg_mainloop_any(const qw_gemm_args &a, unsigned 
     if constexpr (INT8)
         qw8_mainloop<GLU>(a, lds, lds_b, tm, tn, kb, ke, acc);
     else
-        qg_mainloop<8, GLU>(a, lds, lds_b, tm, tn, kb, ke, acc);
+        qg_mainloop<8, GLU>(a, lds, lds_b, tm * 256, tn, kb, ke, acc);
 }
 
 /* The epilogue of one wave's MB x 8 accumulator blocks, whose rows start at
@@ -762,24 +765,38 @@ __device__ __forceinline__ void qg_impl(const qw_gemm_args &a, unsigned char *ld
         __hip_atomic_store(a.sk_flag + r, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-/* 224-row tiles (bf16 W, no split tiles): one workgroup per CU walks the
- * tiles, as the 256-row kernels do. Chosen where the tile count leaves a
- * partly filled last wave that 224-row tiles avoid (the out projection at
- * M = 8704: 468 tiles of 224 x 256 in 2 waves of 0.875 of a 256-row tile's
- * work, against 408 tiles in 2 waves). */
+/* Mixed tile heights (bf16 W, no split tiles): one workgroup per CU walks
+ * the tiles, first mix_rows1 tile rows of 32 mix_h1 rows, then mix_rows2 of
+ * 32 mix_h2. A tile's time goes by its height, so a launch whose 256-row
+ * tiles leave a partly filled last round is walked in as many rounds of
+ * lower tiles that fill it: M = 8704, 12 tile columns: 408 tiles of 256 rows
+ * take 2 rounds, 468 of 224 2 of 0.875, and 240 of 224 with 264 of 192 one
+ * of 0.875 and one of 0.75. */
 template <int EPI>
-__device__ __forceinline__ void qg_impl_t224(const qw_gemm_args &a, unsigned char *lds,
-                                             unsigned char *lds_b) {
+__device__ __forceinline__ void qg_impl_mix(const qw_gemm_args &a, unsigned char *lds,
+                                            unsigned char *lds_b) {
+    constexpr bool GLU = EPI == QW_EPI_SWIGLU;
     const uint32_t KT = a.k / GBK;
-    const uint32_t nt = a.tiles_m * a.tiles_n;
+    const uint32_t n1 = a.mix_rows1 * a.tiles_n, nt = n1 + a.mix_rows2 * a.tiles_n;
     floatx4 acc[8][8];
     uint32_t tm, tn;
     for (uint32_t id = blockIdx.x; id < nt; id += gridDim.x) {
-        uint32_t q = id;
-        if ((nt & 7u) == 0) q = (q & 7u) * (nt >> 3) + (q >> 3);
-        gemm_tile_at(a, q, tm, tn);
-        qg_mainloop<7, EPI == QW_EPI_SWIGLU>(a, lds, lds_b, tm, tn, 0, KT, acc);
-        qg_finish_at<EPI, 0, 7>(a, lds, lds_b, tm * 224, tn * 256, acc);
+        const bool first = id < n1;
+        const uint32_t h = first ? a.mix_h1 : a.mix_h2;
+        uint32_t q = first ? id : id - n1;
+        if (!a.mix_dealt) q = gemm_xcd_range(q, first ? n1 : nt - n1);
+        gemm_tile_in(first ? a.mix_rows1 : a.mix_rows2, a.tiles_n, q, tm, tn);
+        const uint32_t m0 = (first ? 0u : a.mix_rows1 * a.mix_h1 * 32) + tm * h * 32;
+        if (h == 8) {
+            qg_mainloop<8, GLU>(a, lds, lds_b, m0, tn, 0, KT, acc);
+            qg_finish_at<EPI, 0, 8>(a, lds, lds_b, m0, tn * 256, acc);
+        } else if (h == 7) {
+            qg_mainloop<7, GLU>(a, lds, lds_b, m0, tn, 0, KT, acc);
+            qg_finish_at<EPI, 0, 7>(a, lds, lds_b, m0, tn * 256, acc);
+        } else {
+            qg_mainloop<6, GLU>(a, lds, lds_b, m0, tn, 0, KT, acc);
+            qg_finish_at<EPI, 0, 6>(a, lds, lds_b, m0, tn * 256, acc);
+        }
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
 }
@@ -807,15 +824,15 @@ QG_ENTRY(qw_gemm_w8_gelu_q, QW_EPI_GELU, 1)
 QG_ENTRY(qw_gemm_w8_gate_q, QW_EPI_GATE, 1)
 QG_ENTRY(qw_gemm_w8_qkn_q, QW_EPI_QKNORM, 1)
 QG_ENTRY(qw_gemm_w8_swiglu_q, QW_EPI_SWIGLU, 1)
-/* bf16 W, 224-row tiles */
-#define QG_ENTRY_T224(name, EPI)                                                               \
+/* bf16 W, mixed tile heights */
+#define QG_ENTRY_MIX(name, EPI)                                                               \
     QW_KERNEL void __launch_bounds__(256, 1) name(qw_gemm_args a) {                            \
         __shared__ __attribute__((aligned(16))) unsigned char smem[2 * QG_STAGE + 16];          \
-        qg_impl_t224<EPI>(a, smem, smem + QG_STAGE);                                           \
+        qg_impl_mix<EPI>(a, smem, smem + QG_STAGE);                                           \
     }
-QG_ENTRY_T224(qw_gemm_bf16_store_t224, QW_EPI_STORE)
-QG_ENTRY_T224(qw_gemm_bf16_gelu_t224, QW_EPI_GELU)
-QG_ENTRY_T224(qw_gemm_bf16_gate_t224, QW_EPI_GATE)
-QG_ENTRY_T224(qw_gemm_bf16_qkn_t224, QW_EPI_QKNORM)
-QG_ENTRY_T224(qw_gemm_bf16_swiglu_t224, QW_EPI_SWIGLU)
+QG_ENTRY_MIX(qw_gemm_bf16_store_mix, QW_EPI_STORE)
+QG_ENTRY_MIX(qw_gemm_bf16_gelu_mix, QW_EPI_GELU)
+QG_ENTRY_MIX(qw_gemm_bf16_gate_mix, QW_EPI_GATE)
+QG_ENTRY_MIX(qw_gemm_bf16_qkn_mix, QW_EPI_QKNORM)
+QG_ENTRY_MIX(qw_gemm_bf16_swiglu_mix, QW_EPI_SWIGLU)
 #include "gemm_s.h"

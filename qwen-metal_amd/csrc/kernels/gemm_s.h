@@ -175,8 +175,7 @@ __device__ __forceinline__ void qs_impl(const qw_gemm_args &a, unsigned char *ld
     /* ids are dealt round-robin to the 8 XCDs: each XCD takes one contiguous
      * range of the pieces (numbered k-range-major, tile rows first), so the
      * tile rows that share a W panel read it through one L2 */
-    const uint32_t x = blockIdx.x & 7u, per = np >> 3, rem = np & 7u;
-    const uint32_t q = x * per + min(x, rem) + (blockIdx.x >> 3);
+    const uint32_t q = gemm_xcd_range(blockIdx.x, np);
     const uint32_t piece = q / R, r = q % R;
     const uint32_t kb = piece * KT / S, ke = (piece + 1) * KT / S;
     uint32_t tm, tn;

@@ -54,6 +54,10 @@ typedef struct {
     uint32_t half_from, half_count;
     /* narrow tiles: first row of tile row 0 */
     uint32_t m_base;
+    /* mixed tile heights: h1 tile rows of 32 mix_h1 rows, then h2 of 32
+     * mix_h2 (heights 6-8); mix_dealt: tiles in the order of the ids, not in
+     * a range an XCD */
+    uint32_t mix_h1, mix_h2, mix_rows1, mix_rows2, mix_dealt;
 } qw_gemm_args;
 
 typedef struct {
