@@ -147,12 +147,27 @@ __device__ __forceinline__ void qs_mainloop(const qw_gemm_args &a, unsigned char
     bf16x8 pa[MB], pw[8];
     landed();
     qs_slice<false, MB>(c, acc, pa, pw, lds, base + PF * STAGE, ko(kb + PF), off(kb + PF));
-    uint32_t cur = STAGE, nxt = 0; /* stages of slices kt and kt + PF */
-    for (uint32_t kt = kb + 1; kt < ke; kt++) {
-        landed();
-        qs_slice<true, MB>(c, acc, pa, pw, lds + cur, base + nxt, ko(kt + PF), off(kt + PF));
-        nxt = cur;
-        cur = cur + STAGE == NST * STAGE ? 0u : cur + STAGE;
+    uint32_t kt = kb + 1;
+    if constexpr (MB >= 3) {
+        /* NST slices a turn, so that the stages are constants */
+        while (kt < ke) {
+#pragma unroll
+            for (int st = 1; st <= NST; st++) {
+                if (kt >= ke) break;
+                landed();
+                qs_slice<true, MB>(c, acc, pa, pw, lds + (st % NST) * STAGE,
+                                   base + ((st + PF) % NST) * STAGE, ko(kt + PF), off(kt + PF));
+                kt++;
+            }
+        }
+    } else {
+        uint32_t cur = STAGE, nxt = 0; /* stages of slices kt and kt + PF */
+        for (; kt < ke; kt++) {
+            landed();
+            qs_slice<true, MB>(c, acc, pa, pw, lds + cur, base + nxt, ko(kt + PF), off(kt + PF));
+            nxt = cur;
+            cur = cur + STAGE == NST * STAGE ? 0u : cur + STAGE;
+        }
     }
     asm volatile("s_nop 1" ::"v"(pw[0]), "v"(pw[1]), "v"(pw[2]), "v"(pw[3]), "v"(pw[4]),
                  "v"(pw[5]), "v"(pw[6]), "v"(pw[7]));
