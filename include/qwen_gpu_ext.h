@@ -202,6 +202,22 @@ int qw_gpu_modulation_reorder_bf16(h3_gpu *gpu, h3_gpu_tensor *slots_out,
                                    uint32_t mod_rows, uint32_t hidden,
                                    int shift_variant);
 
+/* The whole conditioning chain (qwen_dit.m:1098-1192) of 1 or 2 rows in three
+ * launches: temb = l2(silu(l1(bf16(features)))), modulation = the slot-ordered
+ * mod(silu(temb)) as qw_gpu_modulation_reorder_bf16 leaves it, norm_out_scale
+ * = norm_out(silu(temb)). Weights bf16 [n, k]; biases may be NULL; wide and
+ * silu are scratch, bf16 [rows, hidden]. The results are those of the
+ * separate linears and activations, bit for bit. No counterpart in the
+ * reference. */
+typedef struct {
+    const h3_gpu_tensor *features; /* f32 [rows, 256] */
+    const h3_gpu_tensor *l1, *l1_bias, *l2, *l2_bias, *mod, *mod_bias, *norm_out, *norm_out_bias;
+    h3_gpu_tensor *wide, *silu, *temb, *modulation, *norm_out_scale;
+    uint32_t rows, hidden;
+    int shift_variant; /* 6 slots and [2 hidden] of norm_out; else 4 and [hidden] */
+} qw_conditioning_desc;
+int qw_gpu_conditioning_bf16(h3_gpu *gpu, const qw_conditioning_desc *desc);
+
 /* Seeded synthetic values: bf16(std * z + offset), z from the counter-based
  * generator keyed by (seed, stream, index) — bit-identical to the host
  * restatement used by the tests. Fills [offset_elems, +count). */

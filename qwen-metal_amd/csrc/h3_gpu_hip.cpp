@@ -34,7 +34,7 @@ enum {
     /* narrow tiles of 64, 128, 192 and 256 rows, each in the same order */
     K_GEMM_N1, K_GEMM_N1_LAST = K_GEMM_N1 + 4, K_GEMM_N2, K_GEMM_N2_LAST = K_GEMM_N2 + 4,
     K_GEMM_N3, K_GEMM_N3_LAST = K_GEMM_N3 + 4, K_GEMM_N4, K_GEMM_N4_LAST = K_GEMM_N4 + 4,
-    K_ATTN_W4, K_ATTN_SPLIT, K_ATTN_W4_SPLIT,
+    K_ATTN_W4, K_ATTN_SPLIT, K_ATTN_W4_SPLIT, K_COND_L1, K_COND_L2, K_COND_MOD,
     K_COUNT
 };
 static const char *k_names[K_COUNT] = {
@@ -54,7 +54,8 @@ static const char *k_names[K_COUNT] = {
     "qw_gemm_bf16_store_n2", "qw_gemm_bf16_gelu_n2", "qw_gemm_bf16_gate_n2", "qw_gemm_bf16_qkn_n2", "qw_gemm_bf16_swiglu_n2",
     "qw_gemm_bf16_store_n3", "qw_gemm_bf16_gelu_n3", "qw_gemm_bf16_gate_n3", "qw_gemm_bf16_qkn_n3", "qw_gemm_bf16_swiglu_n3",
     "qw_gemm_bf16_store_n4", "qw_gemm_bf16_gelu_n4", "qw_gemm_bf16_gate_n4", "qw_gemm_bf16_qkn_n4", "qw_gemm_bf16_swiglu_n4",
-    "qw_attention_w4_bf16", "qw_attention_split_bf16", "qw_attention_w4_split_bf16"};
+    "qw_attention_w4_bf16", "qw_attention_split_bf16", "qw_attention_w4_split_bf16",
+    "qw_cond_l1", "qw_cond_l2", "qw_cond_mod"};
 
 /* How int8 linears run (QW_INT8_ROUTE, a measurement switch): AUTO (the
  * default) widens the weight to a bf16 copy and runs the bf16 kernels when
@@ -849,6 +850,64 @@ extern "C" int qw_gpu_modulation_reorder_bf16(h3_gpu *g, h3_gpu_tensor *out,
     qw_reorder_args a = {(uint16_t *)out->ptr, (const uint16_t *)raw->ptr, mod_rows, hidden,
                          shift_variant};
     return launch(g, K_REORDER, dim3(blocks_for((uint64_t)mod_rows * hidden, 256)), dim3(256), a);
+}
+
+extern "C" int qw_gpu_conditioning_bf16(h3_gpu *g, const qw_conditioning_desc *d) {
+    if (!g || !d) return 0;
+    const uint32_t H = d->hidden, rows = d->rows, S = d->shift_variant ? 6 : 4;
+    const uint32_t nout = d->shift_variant ? 2 * H : H;
+    if (!rows || rows > 2) return fail(g, "conditioning: rows must be 1 or 2");
+    if (!H || H % 8 || (uint64_t)S * H * H >= (1ull << 32))
+        return fail(g, "conditioning: hidden %u must be a multiple of 8", H);
+    const struct { const h3_gpu_tensor *t; size_t n; h3_gpu_dtype type; int optional; } need[] = {
+        {d->features, (size_t)rows * 256, H3_GPU_F32, 0},  {d->l1, (size_t)H * 256, H3_GPU_BF16, 0},
+        {d->l2, (size_t)H * H, H3_GPU_BF16, 0},            {d->mod, (size_t)S * H * H, H3_GPU_BF16, 0},
+        {d->norm_out, (size_t)nout * H, H3_GPU_BF16, 0},   {d->l1_bias, H, H3_GPU_BF16, 1},
+        {d->l2_bias, H, H3_GPU_BF16, 1},                   {d->mod_bias, (size_t)S * H, H3_GPU_BF16, 1},
+        {d->norm_out_bias, nout, H3_GPU_BF16, 1},          {d->wide, (size_t)rows * H, H3_GPU_BF16, 0},
+        {d->silu, (size_t)rows * H, H3_GPU_BF16, 0},       {d->temb, (size_t)rows * H, H3_GPU_BF16, 0},
+        {d->modulation, (size_t)rows * S * H, H3_GPU_BF16, 0},
+        {d->norm_out_scale, (size_t)rows * nout, H3_GPU_BF16, 0}};
+    for (const auto &x : need) {
+        if (!x.t && x.optional) continue;
+        if (!x.t || x.t->dtype != x.type) return fail(g, "conditioning: missing tensor or wrong dtype");
+        if (!fits(x.t, 0, x.n)) return fail(g, "conditioning: tensor too small");
+    }
+    /* the operands that are read 16 bytes at a time */
+    for (const h3_gpu_tensor *t : {d->l1, d->l2, d->mod, d->norm_out,
+                                   (const h3_gpu_tensor *)d->wide, (const h3_gpu_tensor *)d->silu})
+        if ((uintptr_t)t->ptr % 16) return fail(g, "conditioning: tensors must be 16-byte aligned");
+    auto bias = [](const h3_gpu_tensor *t) { return t ? (const uint16_t *)t->ptr : NULL; };
+    auto grid = [](uint32_t n) { return dim3((n + 7) / 8); }; /* 4 waves of 2 columns */
+    qw_cond_args a;
+    memset(&a, 0, sizeof(a));
+    a.rows = rows;
+    a.hidden = H;
+    a.shift_variant = d->shift_variant;
+    a.in = d->features->ptr;
+    a.w = (const uint16_t *)d->l1->ptr;
+    a.bias = bias(d->l1_bias);
+    a.out = (uint16_t *)d->wide->ptr;
+    a.k = 256;
+    a.n = H;
+    if (!launch(g, K_COND_L1, grid(H), dim3(256), a)) return 0;
+    a.in = d->wide->ptr;
+    a.w = (const uint16_t *)d->l2->ptr;
+    a.bias = bias(d->l2_bias);
+    a.out = (uint16_t *)d->temb->ptr;
+    a.out2 = (uint16_t *)d->silu->ptr;
+    a.k = H;
+    if (!launch(g, K_COND_L2, grid(H), dim3(256), a)) return 0;
+    a.in = d->silu->ptr;
+    a.w = (const uint16_t *)d->mod->ptr;
+    a.bias = bias(d->mod_bias);
+    a.out = (uint16_t *)d->modulation->ptr;
+    a.n = S * H;
+    a.w2 = (const uint16_t *)d->norm_out->ptr;
+    a.bias2 = bias(d->norm_out_bias);
+    a.out2 = (uint16_t *)d->norm_out_scale->ptr;
+    a.n2 = nout;
+    return launch(g, K_COND_MOD, grid(a.n + a.n2), dim3(256), a);
 }
 
 extern "C" int qw_gpu_fill_normal_bf16(h3_gpu *g, h3_gpu_tensor *t, size_t off, size_t count,

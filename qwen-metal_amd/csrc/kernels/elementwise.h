@@ -290,6 +290,93 @@ QW_KERNEL void __launch_bounds__(256) qw_modulation_reorder_bf16(qw_reorder_args
     }
 }
 
+/* ---- conditioning chain --------------------------------------------------- */
+/* The timestep MLP, the modulation linear and the final norm's linear run on
+ * one or two rows (the sampled timestep and t = 0), so each is a stream of
+ * its weight. As the separate launches (cast, linear, silu, linear, silu, two
+ * linears, reorder) they took 63 us for 171 MB, 20 of them in the small
+ * passes and in the drain and fill of eight launches; here the passes ride
+ * the linears' loads and stores, the two last linears share a launch, and
+ * each wave has 4 chunks of both its weight rows in flight: 46 us. Same
+ * sums in the same order and the same roundings as those launches. */
+#define COND_COLS 2 /* weight rows per wave */
+template <int STAGE> __device__ __forceinline__ void qw_cond_impl(const qw_cond_args &a) {
+#pragma clang fp contract(off)
+    const uint32_t lane = threadIdx.x & 63;
+    uint32_t c0 = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * COND_COLS;
+    const uint32_t n_all = a.n + (STAGE == QW_COND_MOD ? a.n2 : 0);
+    if (c0 >= n_all) return; /* whole waves */
+    const bool second = STAGE == QW_COND_MOD && c0 >= a.n; /* n % COND_COLS == 0 */
+    if (second) c0 -= a.n;
+    const u16 *w = second ? a.w2 : a.w, *bias = second ? a.bias2 : a.bias;
+    const uint32_t kc = a.k / 8;
+    float acc[2][COND_COLS] = {};
+    for (uint32_t j0 = lane; j0 < kc; j0 += 256) {
+        u32x4 q[4][COND_COLS];
+        float x[4][2][8];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int c = 0; c < COND_COLS; c++)
+                q[u][c] = *(const u32x4 *)(w + (size_t)(c0 + c) * a.k + 8 * min(j0 + 64 * u, kc - 1));
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            if (j0 + 64 * u >= kc) break;
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                if ((uint32_t)r >= a.rows) break;
+                const size_t at = (size_t)r * a.k + 8 * (j0 + 64 * u);
+                if (STAGE == QW_COND_L1) {
+                    /* features may start at any float */
+#pragma unroll
+                    for (int i = 0; i < 8; i++)
+                        x[u][r][i] = bf2f(f2bf(((const float *)a.in)[at + i]));
+                } else {
+                    const u32x4 v = *(const u32x4 *)((const u16 *)a.in + at);
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        x[u][r][2 * i] = lo_bf(v[i]), x[u][r][2 * i + 1] = hi_bf(v[i]);
+                }
+#pragma unroll
+                for (int c = 0; c < COND_COLS; c++)
+#pragma unroll
+                    for (int i = 0; i < 8; i++)
+                        acc[r][c] = fmaf(x[u][r][i], (i & 1) ? hi_bf(q[u][c][i / 2]) : lo_bf(q[u][c][i / 2]),
+                                         acc[r][c]);
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        if ((uint32_t)r >= a.rows) break;
+#pragma unroll
+        for (int c = 0; c < COND_COLS; c++) {
+            const float t = wave_sum(acc[r][c]);
+            const uint32_t col = c0 + c;
+            if (lane != 0) continue;
+            const u16 y = f2bf(t + (bias ? bf2f(bias[col]) : 0.0f));
+            if (STAGE == QW_COND_L1) {
+                a.out[(size_t)r * a.n + col] = f2bf(silu_f(bf2f(y)));
+            } else if (STAGE == QW_COND_L2) {
+                a.out[(size_t)r * a.n + col] = y;
+                a.out2[(size_t)r * a.n + col] = f2bf(silu_f(bf2f(y)));
+            } else if (second) {
+                a.out2[(size_t)r * a.n2 + col] = y;
+            } else { /* as qw_modulation_reorder_bf16 */
+                const uint32_t H = a.hidden, s = col / H;
+                const bool gate = a.shift_variant ? s % 3 == 2 : s & 1;
+                const uint32_t half = a.shift_variant ? s / 3 : s / 2;
+                const uint32_t slot = gate ? 2 + half : a.shift_variant && s % 3 == 0 ? 4 + half : half;
+                a.out[(size_t)r * a.n + slot * H + col % H] =
+                    gate ? f2bf_trunc(tanhf(bf2f(y))) : y;
+            }
+        }
+    }
+}
+QW_KERNEL void __launch_bounds__(256) qw_cond_l1(qw_cond_args a) { qw_cond_impl<QW_COND_L1>(a); }
+QW_KERNEL void __launch_bounds__(256) qw_cond_l2(qw_cond_args a) { qw_cond_impl<QW_COND_L2>(a); }
+QW_KERNEL void __launch_bounds__(256) qw_cond_mod(qw_cond_args a) { qw_cond_impl<QW_COND_MOD>(a); }
+
 /* ---- seeded synthetic N(0, 1)-like values -------------------------------- */
 /* Counter-based (splitmix64 finaliser), integer sum of twelve 16-bit
  * uniforms; bit-identical to the host generator by construction. */

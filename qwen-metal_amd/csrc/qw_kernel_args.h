@@ -99,6 +99,20 @@ typedef struct {
     uint32_t rows, width, slots, gate_slot;
 } qw_gate_args;
 
+/* One stage of the conditioning chain (at most 2 rows): out = linear(in, w)
+ * with what follows it up to the next linear. */
+enum { QW_COND_L1 = 0, QW_COND_L2 = 1, QW_COND_MOD = 2 };
+typedef struct {
+    const void *in;           /* L1: f32 [rows, k]; else bf16 */
+    const uint16_t *w, *bias; /* bf16 [n, k], bf16 [n] or NULL */
+    uint16_t *out;            /* L1: silu(y); L2: y; MOD: y in slot order */
+    uint16_t *out2;           /* L2: silu(y); MOD: the second linear's y */
+    const uint16_t *w2, *bias2; /* MOD: second linear, [n2, k] */
+    uint32_t rows, k, n, n2;
+    uint32_t hidden;          /* MOD: columns a slot */
+    int32_t shift_variant;
+} qw_cond_args;
+
 enum { QW_ACT_GELU_TANH = 0, QW_ACT_SILU = 1, QW_ACT_TANH = 2 };
 
 typedef struct {

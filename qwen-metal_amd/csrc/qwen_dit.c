@@ -53,7 +53,7 @@ struct qw_dit {
     uint32_t ws_text_rows;
     h3_gpu_tensor *ws_tnorm, *ws_twide;
     /* conditioning (2 modulation rows) */
-    h3_gpu_tensor *feat, *feat_bf16, *c_wide, *c_silu, *temb, *mod_raw,
+    h3_gpu_tensor *feat, *c_wide, *c_silu, *temb,
         *modulation, *norm_out_mod;
     /* forward-owned joint sequence and row map */
     uint32_t joint_rows;
@@ -207,15 +207,12 @@ static int cond_buffers(qw_dit *d) {
     const uint32_t H = d->cfg.hidden;
     const uint32_t nmod = slots_of(&d->cfg) * H, nout = (d->cfg.adaln_shift ? 2 : 1) * H;
     d->feat = h3_gpu_tensor_new_f32(gpu, 2 * 256);
-    d->feat_bf16 = h3_gpu_tensor_new_bf16(gpu, 2 * 256);
     d->c_wide = h3_gpu_tensor_new_bf16(gpu, 2 * (size_t)H);
     d->c_silu = h3_gpu_tensor_new_bf16(gpu, 2 * (size_t)H);
     d->temb = h3_gpu_tensor_new_bf16(gpu, 2 * (size_t)H);
-    d->mod_raw = h3_gpu_tensor_new_bf16(gpu, 2 * (size_t)nmod);
     d->modulation = h3_gpu_tensor_new_bf16(gpu, 2 * (size_t)nmod);
     d->norm_out_mod = h3_gpu_tensor_new_bf16(gpu, 2 * (size_t)nout);
-    return d->feat && d->feat_bf16 && d->c_wide && d->c_silu && d->temb && d->mod_raw &&
-           d->modulation && d->norm_out_mod;
+    return d->feat && d->c_wide && d->c_silu && d->temb && d->modulation && d->norm_out_mod;
 }
 
 qw_dit *qw_dit_create_random(h3_gpu *gpu, const qw_dit_config *cfg, uint64_t seed,
@@ -729,8 +726,8 @@ void qw_dit_free(qw_dit *d) {
     lin_free(&d->norm_out);
     lin_free(&d->proj_out);
     h3_gpu_tensor *t[] = {d->txt_norm, d->ws_mod, d->ws_qkv, d->ws_attn, d->ws_wide,
-                          d->ws_tnorm, d->ws_twide, d->feat, d->feat_bf16, d->c_wide, d->c_silu,
-                          d->temb, d->mod_raw, d->modulation, d->norm_out_mod, d->joint,
+                          d->ws_tnorm, d->ws_twide, d->feat, d->c_wide, d->c_silu,
+                          d->temb, d->modulation, d->norm_out_mod, d->joint,
                           d->row_map};
     for (size_t i = 0; i < sizeof(t) / sizeof(t[0]); i++) h3_gpu_tensor_free(t[i]);
     qw_dit_ti2i_cache_clear(d);
@@ -975,16 +972,11 @@ int qw_dit_conditioning(qw_dit *d, const h3_gpu_tensor *features, uint32_t mod_r
         h3_gpu_tensor_elements(modulation) < (size_t)mod_rows * S * H ||
         h3_gpu_tensor_elements(norm_out_scale) < (size_t)mod_rows * d->norm_out.n)
         return set_error(error, error_size, "conditioning tensors too small");
-    size_t n = (size_t)mod_rows * H;
-    int ok = h3_gpu_cast_f32_to_bf16(g, d->feat_bf16, features, mod_rows * 256) &&
-             plain(d, &d->time_l1, d->c_wide, d->feat_bf16, mod_rows, QW_LINEAR_STORE) &&
-             h3_gpu_silu_bf16(g, d->c_wide, d->c_wide, (uint32_t)n) &&
-             plain(d, &d->time_l2, temb, d->c_wide, mod_rows, QW_LINEAR_STORE) &&
-             h3_gpu_silu_bf16(g, d->c_silu, temb, (uint32_t)n) &&
-             plain(d, &d->norm_out, norm_out_scale, d->c_silu, mod_rows, QW_LINEAR_STORE) &&
-             plain(d, &d->mod, d->mod_raw, d->c_silu, mod_rows, QW_LINEAR_STORE) &&
-             qw_gpu_modulation_reorder_bf16(g, modulation, d->mod_raw, mod_rows, H,
-                                            d->cfg.adaln_shift);
+    const qw_conditioning_desc desc = {
+        features, d->time_l1.w, d->time_l1.bias, d->time_l2.w, d->time_l2.bias, d->mod.w,
+        d->mod.bias, d->norm_out.w, d->norm_out.bias, d->c_wide, d->c_silu, temb, modulation,
+        norm_out_scale, mod_rows, H, d->cfg.adaln_shift};
+    const int ok = qw_gpu_conditioning_bf16(g, &desc);
     if (!ok) return set_error(error, error_size, "conditioning failed: %s", h3_gpu_error(g));
     return 1;
 }

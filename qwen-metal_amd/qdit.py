@@ -73,6 +73,13 @@ class AttentionDesc(C.Structure):
                 ("text_rows", u32), ("text_causal", C.c_int), ("scale", C.c_float)]
 
 
+class ConditioningDesc(C.Structure):
+    _fields_ = [(n, vp) for n in (
+        "features", "l1", "l1_bias", "l2", "l2_bias", "mod", "mod_bias", "norm_out",
+        "norm_out_bias", "wide", "silu", "temb", "modulation", "norm_out_scale")] + [
+        ("rows", u32), ("hidden", u32), ("shift_variant", C.c_int)]
+
+
 # Every exported entry point with its (restype, argtypes). The CPU test
 # checks the library exports each name declared in include/*.h.
 SIGNATURES = {
@@ -131,6 +138,7 @@ SIGNATURES = {
     "qw_gpu_layer_norm_mod_shift_bf16": (C.c_int, [vp, vp, vp, vp, vp, u32, u32, u32, u32,
                                                    C.c_int32, C.c_float]),
     "qw_gpu_linear": (C.c_int, [vp, C.POINTER(LinearDesc)]),
+    "qw_gpu_conditioning_bf16": (C.c_int, [vp, C.POINTER(ConditioningDesc)]),
     "qw_gpu_linear_swiglu": (C.c_int, [vp, C.POINTER(LinearDesc)]),
     "qw_gpu_linear_static": (C.c_int, [vp, C.POINTER(LinearDesc)]),
     "qw_gpu_qk_norm_rope_bf16": (C.c_int, [vp, vp, u32, u32, u32, u32, vp, vp, vp, vp, u32,
