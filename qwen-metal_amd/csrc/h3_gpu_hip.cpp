@@ -34,7 +34,8 @@ enum {
     /* narrow tiles of 64, 128, 192 and 256 rows, each in the same order */
     K_GEMM_N1, K_GEMM_N1_LAST = K_GEMM_N1 + 4, K_GEMM_N2, K_GEMM_N2_LAST = K_GEMM_N2 + 4,
     K_GEMM_N3, K_GEMM_N3_LAST = K_GEMM_N3 + 4, K_GEMM_N4, K_GEMM_N4_LAST = K_GEMM_N4 + 4,
-    K_ATTN_W4, K_ATTN_SPLIT, K_ATTN_W4_SPLIT, K_COND_L1, K_COND_L2, K_COND_MOD,
+    K_ATTN_W4, K_ATTN_SPLIT, K_ATTN_W4_SPLIT, K_COND_L1, K_COND_L2, K_COND_MOD, /* with and without shift, width up to 4096 and 3072 */
+    K_LN_MOD_SHIFT, K_LN_MOD_3072, K_LN_MOD_3072_SHIFT,
     K_COUNT
 };
 static const char *k_names[K_COUNT] = {
@@ -55,7 +56,8 @@ static const char *k_names[K_COUNT] = {
     "qw_gemm_bf16_store_n3", "qw_gemm_bf16_gelu_n3", "qw_gemm_bf16_gate_n3", "qw_gemm_bf16_qkn_n3", "qw_gemm_bf16_swiglu_n3",
     "qw_gemm_bf16_store_n4", "qw_gemm_bf16_gelu_n4", "qw_gemm_bf16_gate_n4", "qw_gemm_bf16_qkn_n4", "qw_gemm_bf16_swiglu_n4",
     "qw_attention_w4_bf16", "qw_attention_split_bf16", "qw_attention_w4_split_bf16",
-    "qw_cond_l1", "qw_cond_l2", "qw_cond_mod"};
+    "qw_cond_l1", "qw_cond_l2", "qw_cond_mod", "qw_layer_norm_mod_shift_bf16",
+    "qw_layer_norm_mod_3072_bf16", "qw_layer_norm_mod_3072_shift_bf16"};
 
 /* How int8 linears run (QW_INT8_ROUTE, a measurement switch): AUTO (the
  * default) widens the weight to a bf16 copy and runs the bf16 kernels when
@@ -619,7 +621,10 @@ static int ln_mod(h3_gpu *g, h3_gpu_tensor *out, const h3_gpu_tensor *in,
     qw_ln_mod_args a = {(uint16_t *)out->ptr, (const uint16_t *)in->ptr,
                         (const uint16_t *)mod->ptr, (const uint32_t *)row_map->ptr,
                         rows, width, slots, scale_slot, shift_slot, eps};
-    if (width <= 4096) return launch(g, K_LN_MOD, dim3((rows + 3) / 4), dim3(256), a);
+    if (width <= 4096)
+        return launch(g, shift_slot >= 0 ? (width <= 3072 ? K_LN_MOD_3072_SHIFT : K_LN_MOD_SHIFT)
+                                         : (width <= 3072 ? K_LN_MOD_3072 : K_LN_MOD),
+                      dim3((rows + 3) / 4), dim3(256), a);
     return launch(g, K_LN_MOD_WIDE, dim3(rows), dim3((width / 8 + 63) / 64 * 64), a);
 }
 

@@ -11,64 +11,88 @@
 /* h3_shaders.metal:4767-4815. One wave per row (width <= 4096), four rows
  * per block: lane l owns the 16-byte chunks l, l + 64, ... of the row,
  * held in registers for both passes, and both reductions are wave
- * shuffles (no LDS, no barrier). */
-#define LN_CH 8 /* chunks of 8 per lane: width <= 64 * 8 * 8 = 4096 */
-QW_KERNEL void __launch_bounds__(256) qw_layer_norm_mod_bf16(qw_ln_mod_args a) {
+ * shuffles (no LDS, no barrier). Large inputs are bound by HBM (4.4 TB/s at
+ * 8704 x 3072, against 5.0 of a large copy); a few hundred rows by the chain
+ * of loads and shuffles, so the modulation is read with the row and not
+ * after its statistics (320 x 3072 with shift: 5.1 -> 3.9 us, 8704: 26.6 -> 24.3; 4119 x
+ * 4096 without: 13.7 -> 12.7). CH: chunks of 8 per lane, width <= 512 CH. */
+template <int CH, bool SHIFT>
+__device__ __forceinline__ void qw_ln_mod_impl(const qw_ln_mod_args &a) {
 #pragma clang fp contract(off)
     const uint32_t lane = threadIdx.x & 63;
-    const uint32_t row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const uint32_t row = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (row >= a.rows) return; /* whole waves */
     const u16 *in = a.in + (size_t)row * a.width;
-    float x[LN_CH][8];
+    const u16 *mod = a.modulation + (size_t)a.row_map[row] * a.slots * a.width;
+    /* 8 chunks with shift: read late, or the registers cost more waves a SIMD
+     * than the latency (4119 x 4096: 15.4 us with the scales early, 14.5) */
+    constexpr bool EARLY = !SHIFT || CH < 8;
+    u32x4 raw[CH], sc[CH], sh[CH];
+#pragma unroll
+    for (int c = 0; c < CH; c++) {
+        const uint32_t c8 = (c * 64 + lane) * 8;
+        raw[c] = u32x4{0, 0, 0, 0};
+        if (c8 < a.width) raw[c] = *(const u32x4 *)(in + c8);
+    }
+    auto read_mod = [&](int c, uint32_t c8) __attribute__((always_inline)) {
+        sc[c] = *(const u32x4 *)(mod + (size_t)a.scale_slot * a.width + c8);
+        if (SHIFT) sh[c] = *(const u32x4 *)(mod + (size_t)a.shift_slot * a.width + c8);
+    };
+#pragma unroll
+    for (int c = 0; c < CH; c++) {
+        const uint32_t c8 = (c * 64 + lane) * 8;
+        sc[c] = sh[c] = u32x4{0, 0, 0, 0};
+        if (EARLY && c8 < a.width) read_mod(c, c8);
+    }
     float s = 0.0f;
 #pragma unroll
-    for (int c = 0; c < LN_CH; c++) {
-        const uint32_t c8 = (c * 64 + lane) * 8;
-        u32x4 raw = {0, 0, 0, 0};
-        if (c8 < a.width) raw = *(const u32x4 *)(in + c8);
+    for (int c = 0; c < CH; c++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            x[c][2 * i] = lo_bf(raw[i]);
-            x[c][2 * i + 1] = hi_bf(raw[i]);
+            s += lo_bf(raw[c][i]);
+            s += hi_bf(raw[c][i]);
         }
-#pragma unroll
-        for (int i = 0; i < 8; i++) s += x[c][i];
-    }
     const float mean = wave_sum(s) / (float)a.width;
     float q = 0.0f;
 #pragma unroll
-    for (int c = 0; c < LN_CH; c++) {
+    for (int c = 0; c < CH; c++) {
         if ((c * 64 + lane) * 8 >= a.width) continue;
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const float d = x[c][i] - mean;
-            q = fmaf(d, d, q);
+        for (int i = 0; i < 4; i++) {
+            const float d0 = lo_bf(raw[c][i]) - mean, d1 = hi_bf(raw[c][i]) - mean;
+            q = fmaf(d0, d0, q);
+            q = fmaf(d1, d1, q);
         }
     }
     const float var = wave_sum(q) / (float)a.width;
     const float inv = 1.0f / sqrtf(var + a.eps);
-    const u16 *mod = a.modulation + (size_t)a.row_map[row] * a.slots * a.width;
 #pragma unroll
-    for (int c = 0; c < LN_CH; c++) {
+    for (int c = 0; c < CH; c++) {
         const uint32_t c8 = (c * 64 + lane) * 8;
         if (c8 >= a.width) continue;
-        const u32x4 sc = *(const u32x4 *)(mod + (size_t)a.scale_slot * a.width + c8);
-        u32x4 sh = {0, 0, 0, 0};
-        if (a.shift_slot >= 0) sh = *(const u32x4 *)(mod + (size_t)a.shift_slot * a.width + c8);
+        if (!EARLY) read_mod(c, c8);
         u32x4 o;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            float v0 = ((x[c][2 * i] - mean) * inv) * (1.0f + lo_bf(sc[i]));
-            float v1 = ((x[c][2 * i + 1] - mean) * inv) * (1.0f + hi_bf(sc[i]));
-            if (a.shift_slot >= 0) {
-                v0 += lo_bf(sh[i]);
-                v1 += hi_bf(sh[i]);
+            float v0 = ((lo_bf(raw[c][i]) - mean) * inv) * (1.0f + lo_bf(sc[c][i]));
+            float v1 = ((hi_bf(raw[c][i]) - mean) * inv) * (1.0f + hi_bf(sc[c][i]));
+            if (SHIFT) {
+                v0 += lo_bf(sh[c][i]);
+                v1 += hi_bf(sh[c][i]);
             }
             o[i] = pack_bf(v0, v1);
         }
         *(u32x4 *)(a.out + (size_t)row * a.width + c8) = o;
     }
 }
+#define LN_ENTRY(name, CH, SHIFT)                                                              \
+    QW_KERNEL void __launch_bounds__(256, SHIFT && CH == 8 ? 5 : 4) name(qw_ln_mod_args a) {                          \
+        qw_ln_mod_impl<CH, SHIFT>(a);                                                          \
+    }
+LN_ENTRY(qw_layer_norm_mod_bf16, 8, false)
+LN_ENTRY(qw_layer_norm_mod_shift_bf16, 8, true)
+LN_ENTRY(qw_layer_norm_mod_3072_bf16, 6, false)
+LN_ENTRY(qw_layer_norm_mod_3072_shift_bf16, 6, true)
 
 /* The same for rows wider than 4096: one block per row, width / 8 threads
  * rounded up to whole waves, each owning one 16-byte chunk (idle tail
