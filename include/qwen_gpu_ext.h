@@ -134,6 +134,13 @@ int qw_gpu_linear(h3_gpu *gpu, const qw_linear_desc *desc);
  * be QW_LINEAR_STORE. No counterpart in the reference, which runs two
  * kernels. */
 int qw_gpu_linear_swiglu(h3_gpu *gpu, const qw_linear_desc *desc);
+/* The QKNORM linear with the k and v thirds of its output (after the norm and
+ * the rotation) in tensors of their own, rows [rows, cols / 3] at kv_offset
+ * elements: a cache that attention reads, without a copy. Columns cols / 3 and
+ * up of out are left undefined. The values are qw_gpu_linear's. No
+ * counterpart in the reference. */
+int qw_gpu_qkv_linear(h3_gpu *gpu, const qw_linear_desc *desc, h3_gpu_tensor *k,
+                      h3_gpu_tensor *v, size_t kv_offset);
 /* No counterpart in the reference. For callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc): qw_gpu_linear with every workspace in

@@ -1192,7 +1192,14 @@ static int split_workspace(h3_gpu *g) {
 /* no_alloc: the workspace-free form behind qw_gpu_linear_static (int8
  * weights always widen inside the GEMM; split-tile partials and counters live
  * in the static workspace, as far as it holds them) */
-static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc) {
+/* kv: outputs of their own for the k and v thirds (QKNORM), or NULL */
+struct kv_out {
+    uint16_t *k, *v;
+    uint32_t ld;
+    size_t bytes;
+};
+static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc,
+                       const kv_out *kv = NULL) {
     if (!g || !d) return 0;
     REQ_DT(d->out, H3_GPU_BF16, "linear out");
     REQ_DT(d->in, H3_GPU_BF16, "linear in");
@@ -1375,6 +1382,10 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc) {
     a.rope_rows = qkn ? d->rope_rows : 1;
     a.qk_cols = qkn ? d->cols / 3 * 2 : 0;
     a.eps = qkn ? d->eps : 0.0f;
+    a.out_k = kv ? kv->k : NULL;
+    a.out_v = kv ? kv->v : NULL;
+    a.ld_kv = kv ? kv->ld : 0;
+    a.kv_bytes = kv ? (uint32_t)kv->bytes : 0;
     a.half_from = 0;
     a.half_count = 0;
     a.m_base = 0;
@@ -1497,6 +1508,30 @@ static int check_epilogue(h3_gpu *g, const qw_linear_desc *d) {
 
 extern "C" int qw_gpu_linear(h3_gpu *g, const qw_linear_desc *d) {
     return check_epilogue(g, d) ? linear_impl(g, d, 0) : 0;
+}
+
+/* Where the fused epilogue does not run (a RoPE table of fewer than 128
+ * rows), the k and v thirds are copied out of the projection. */
+extern "C" int qw_gpu_copy_rows(h3_gpu *g, h3_gpu_tensor *dst, size_t doff, uint32_t dstride,
+                                const h3_gpu_tensor *src, size_t soff, uint32_t sstride,
+                                uint32_t rows, uint32_t row_elems);
+extern "C" int qw_gpu_qkv_linear(h3_gpu *g, const qw_linear_desc *d, h3_gpu_tensor *k,
+                                 h3_gpu_tensor *v, size_t kv_offset) {
+    if (!g || !d) return 0;
+    if (d->epilogue != QW_LINEAR_QKNORM) return fail(g, "qkv_linear: epilogue must be QKNORM");
+    REQ_DT(k, H3_GPU_BF16, "qkv_linear k");
+    REQ_DT(v, H3_GPU_BF16, "qkv_linear v");
+    const uint32_t H = d->cols / 3;
+    const size_t n = (size_t)d->rows * H;
+    if (!fits(k, kv_offset, n) || !fits(v, kv_offset, n))
+        return fail(g, "qkv_linear: k or v too small");
+    if (d->rows == 0 || d->cols == 0) return 1;
+    if (d->rope_rows < 128 || n * 2 >= (1ull << 31))
+        return linear_impl(g, d, 0) &&
+               qw_gpu_copy_rows(g, k, kv_offset, H, d->out, H, d->ldc, d->rows, H) &&
+               qw_gpu_copy_rows(g, v, kv_offset, H, d->out, 2 * (size_t)H, d->ldc, d->rows, H);
+    const kv_out kv = {(uint16_t *)k->ptr + kv_offset, (uint16_t *)v->ptr + kv_offset, H, n * 2};
+    return linear_impl(g, d, 0, &kv);
 }
 
 /* The tile kernels from 9 rows on; fewer rows keep the streaming linear and

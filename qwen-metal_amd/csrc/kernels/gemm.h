@@ -220,13 +220,24 @@ __device__ __forceinline__ void gemm_epilogue_mode(const qw_gemm_args &a, SlabWr
      * each other's sums without any L2 write-back or invalidate */
     const __amdgpu_buffer_rsrc_t part_rsrc = __builtin_amdgcn_make_buffer_rsrc(
         (void *)a.sk_part, (short)0, (int)0x7FFFFFF0, 0x00020000);
-    const __amdgpu_buffer_rsrc_t out_rsrc =
-        __builtin_amdgcn_make_buffer_rsrc((void *)a.out, (short)0, (int)a.out_bytes, 0x00020000);
     /* read-back geometry: lane -> (row within a 4-row group, 8-column chunk
      * of the wave's 128 columns) */
     const uint32_t rr = lane >> 4, cc = lane & 15;
     const uint32_t col = col0 + cc * 8;
     const bool col_ok = col < a.n;                 /* n % 8 == 0 */
+    /* where this wave's columns go: with separate k and v outputs, one head of
+     * 128 columns lies in one of them */
+    void *out = (void *)a.out;
+    uint32_t out_bytes = a.out_bytes, ldc = a.ldc, out_col = col;
+    if (EPI == QW_EPI_QKNORM && MODE != 1 && a.out_k && col0 >= a.qk_cols / 2) {
+        const bool v = col0 >= a.qk_cols;
+        out = v ? (void *)a.out_v : (void *)a.out_k;
+        out_bytes = a.kv_bytes;
+        ldc = a.ld_kv;
+        out_col = col - (v ? a.qk_cols : a.qk_cols / 2);
+    }
+    const __amdgpu_buffer_rsrc_t out_rsrc =
+        __builtin_amdgcn_make_buffer_rsrc(out, (short)0, (int)out_bytes, 0x00020000);
     const uint32_t colc = col_ok ? col : a.n - 8;  /* in-range column for operand loads */
     float sc[8], bias[8];
 #pragma unroll
@@ -274,7 +285,7 @@ __device__ __forceinline__ void gemm_epilogue_mode(const qw_gemm_args &a, SlabWr
 #pragma unroll
             for (int i = 0; i < RP; i++) {
                 const uint32_t row = row0 + mi * SR + 4 * (p0 + i) + rr;
-                ooff[i] = col_ok && row < a.m ? (row * a.ldc + col) * 2 : 0x80000000u;
+                ooff[i] = col_ok && row < a.m ? (row * ldc + out_col) * 2 : 0x80000000u;
                 if (EPI == QW_EPI_GATE && MODE != 1) {
                     const uint32_t mrow = a.row_map[min(row, a.m - 1)];
                     gv[i] = *(const u32x4 *)(a.gate + (size_t)mrow * a.gate_row_stride + colc);

@@ -49,6 +49,10 @@ typedef struct {
     const float *rope_cos, *rope_sin;
     uint32_t rope_rows, qk_cols;
     float eps;
+    /* k and v thirds to [rows, n / 3] outputs of their own (row stride
+     * ld_kv); NULL: beside q */
+    uint16_t *out_k, *out_v;
+    uint32_t ld_kv, kv_bytes;
     /* Tile walk (split <= 1, bf16 W): tiles [half_from, tiles) run as
      * half_count = 2 (tiles - half_from) half tiles of 128 x 256; 0: none. */
     uint32_t half_from, half_count;

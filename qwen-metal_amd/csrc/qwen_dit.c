@@ -995,9 +995,11 @@ typedef struct {
 /* The fused q|k|v projection with the per-head RMS norm of q and k
  * (h3_shaders.metal:4309-4329) and their RoPE (4864-4896) in its epilogue:
  * one launch, the same result as the linear followed by
- * qw_gpu_qk_norm_rope_bf16. */
+ * qw_gpu_qk_norm_rope_bf16. With k and v, those thirds go there (rows of H at
+ * kv_offset) instead of beside q. */
 static int qkv_linear(qw_dit *d, const qw_layer *L, uint32_t M, const h3_gpu_tensor *rope_cos,
-                      const h3_gpu_tensor *rope_sin, uint32_t rope_rows) {
+                      const h3_gpu_tensor *rope_sin, uint32_t rope_rows, h3_gpu_tensor *k,
+                      h3_gpu_tensor *v, size_t kv_offset) {
     const uint32_t H = d->cfg.hidden;
     qw_linear_desc desc;
     memset(&desc, 0, sizeof(desc));
@@ -1018,7 +1020,17 @@ static int qkv_linear(qw_dit *d, const qw_layer *L, uint32_t M, const h3_gpu_ten
     desc.rope_sin = rope_sin;
     desc.rope_rows = rope_rows;
     desc.eps = 1e-6f;
-    return qw_gpu_linear(d->gpu, &desc);
+    return k ? qw_gpu_qkv_linear(d->gpu, &desc, k, v, kv_offset) : qw_gpu_linear(d->gpu, &desc);
+}
+
+/* Whether a caller's K and V outputs can hold the projection's while
+ * attention reads them: both there, apart, and aligned to 16 bytes (a view may
+ * start anywhere). */
+static int kv_direct(const h3_gpu_tensor *k, const h3_gpu_tensor *v, size_t n) {
+    if (!k || !v) return 0;
+    const uintptr_t a = (uintptr_t)h3_gpu_tensor_device_ptr(k);
+    const uintptr_t b = (uintptr_t)h3_gpu_tensor_device_ptr(v);
+    return !((a | b) % 16) && (a + 2 * n <= b || b + 2 * n <= a);
 }
 
 /* The fused gate|up projection and its SwiGLU in one launch:
@@ -1059,7 +1071,12 @@ static int block_run(qw_dit *d, int li, h3_gpu_tensor *hidden, uint32_t batch, u
                                           sh ? 4 : -1, 1e-6f);
     span_e(d);
     span_b(d, QW_SPAN_QKV);
-    ok = ok && qkv_linear(d, L, M, rope_cos, rope_sin, rows);
+    /* K and V straight into the cache they are kept in, which attention then
+     * reads (as a copy of 4096 x 4096 each they took 23 us a tensor) */
+    h3_gpu_tensor *ko = kvc ? kvc->k : kv_direct(k_out, v_out, (size_t)M * H) ? k_out : NULL;
+    h3_gpu_tensor *vo = kvc ? kvc->v : ko ? v_out : NULL;
+    ok = ok && qkv_linear(d, L, M, rope_cos, rope_sin, rows, ko, vo,
+                          kvc ? (size_t)kvc->base * H : 0);
     span_e(d);
     prof_end(d, P_INPUT);
     if (!ok) return 0;
@@ -1081,15 +1098,13 @@ static int block_run(qw_dit *d, int li, h3_gpu_tensor *hidden, uint32_t batch, u
     ad.text_rows = text_rows;
     ad.text_causal = d->cfg.text_causal;
     ad.scale = 1.0f / sqrtf(128.0f);
-    if (kvc) { /* this step's rows into the cache, then attend to all of it */
-        ok = qw_gpu_copy_rows(g, kvc->k, (size_t)kvc->base * H, H, d->ws_qkv, H, 3 * H, M, H) &&
-             qw_gpu_copy_rows(g, kvc->v, (size_t)kvc->base * H, H, d->ws_qkv, 2 * (size_t)H,
-                              3 * H, M, H);
-        if (!ok) return 0;
-        ad.k = kvc->k;
-        ad.v = kvc->v;
+    if (ko) {
+        ad.k = ko;
+        ad.v = vo;
         ad.k_offset = ad.v_offset = 0;
         ad.ldk = ad.ldv = H;
+    }
+    if (kvc) { /* this step's rows are in the cache; attend to all of it */
         ad.kv_rows = kvc->rows;
         ad.kv_limit = NULL;
         ad.text_rows = 0; /* every query sees every cached key */
@@ -1097,8 +1112,9 @@ static int block_run(qw_dit *d, int li, h3_gpu_tensor *hidden, uint32_t batch, u
     span_b(d, QW_SPAN_ATTN);
     ok = qw_gpu_attention_bf16(g, &ad);
     span_e(d);
-    if (ok && k_out) ok = qw_gpu_copy_rows(g, k_out, 0, H, d->ws_qkv, H, 3 * H, M, H);
-    if (ok && v_out) ok = qw_gpu_copy_rows(g, v_out, 0, H, d->ws_qkv, 2 * (size_t)H, 3 * H, M, H);
+    if (ok && k_out && !ko) ok = qw_gpu_copy_rows(g, k_out, 0, H, d->ws_qkv, H, 3 * H, M, H);
+    if (ok && v_out && !ko)
+        ok = qw_gpu_copy_rows(g, v_out, 0, H, d->ws_qkv, 2 * (size_t)H, 3 * H, M, H);
     if (ok && debug_attn) ok = h3_gpu_copy_bf16(g, debug_attn, 0, d->ws_attn, 0, (size_t)M * H);
     prof_end(d, P_ATTN);
     if (!ok) return 0;

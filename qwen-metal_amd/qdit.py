@@ -139,6 +139,7 @@ SIGNATURES = {
                                                    C.c_int32, C.c_float]),
     "qw_gpu_linear": (C.c_int, [vp, C.POINTER(LinearDesc)]),
     "qw_gpu_conditioning_bf16": (C.c_int, [vp, C.POINTER(ConditioningDesc)]),
+    "qw_gpu_qkv_linear": (C.c_int, [vp, C.POINTER(LinearDesc), vp, vp, sz]),
     "qw_gpu_linear_swiglu": (C.c_int, [vp, C.POINTER(LinearDesc)]),
     "qw_gpu_linear_static": (C.c_int, [vp, C.POINTER(LinearDesc)]),
     "qw_gpu_qk_norm_rope_bf16": (C.c_int, [vp, vp, u32, u32, u32, u32, vp, vp, vp, vp, u32,

@@ -1,0 +1,81 @@
+"""The fused q|k|v projection with k and v in tensors of their own, against
+the same projection beside q, bit for bit; and a block's K/V outputs, which
+are those tensors where they can be."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from test_gpu_kernels import synth
+
+pytestmark = pytest.mark.gpu
+
+
+# narrow tiles in pieces, whole and with a wide part above them; mixed tile
+# heights; int8 widened; a table too short for the fused epilogue
+@pytest.mark.parametrize("rows,k,heads,int8,rope_rows", [
+    (70, 2048, 2, False, 200), (320, 256, 24, True, 320), (4119, 512, 10, False, 4119),
+    (3000, 192, 12, False, 1500), (300, 128, 2, False, 100)])
+def test_qkv_linear_outputs(gpu, qd, oracle, rows, k, heads, int8, rope_rows):
+    H = heads * 128
+    n = 3 * H
+    x = gpu.put(synth(oracle, rows * k, 91))
+    w = gpu.put(synth(oracle, n * k, 92, 0.05))
+    s = None
+    if int8:
+        q, s = gpu.new(n * k, qd.I8), gpu.new(n, qd.F32)
+        gpu.check(qd.lib().h3_gpu_quantize_weight_int8(gpu.h, q.h, s.h, w.h, n, k), "q")
+        w = q
+    ang = np.random.default_rng(9).uniform(-3, 3, (rope_rows, 64)).astype(np.float32)
+    nq, nk = gpu.put(synth(oracle, 128, 34, 0.1)), gpu.put(synth(oracle, 128, 35, 0.1))
+    ct, st = gpu.put(np.cos(ang)), gpu.put(np.sin(ang))
+    ref, out = gpu.new(rows * n, qd.BF16), gpu.new(rows * n, qd.BF16)
+    gpu.linear(ref, x, w, rows, k, n, wscale=s, epilogue=qd.LINEAR_QKNORM,
+               qknorm=(nq, nk, ct, st, rope_rows, 1e-6))
+    at = 8 * H  # rows before and after the written ones stay untouched
+    kt, vt = (gpu.put(np.full((rows + 16) * H, 0x1234, np.uint16)) for _ in range(2))
+    d = qd.LinearDesc(out.h, 0, n, x.h, 0, k, w.h, s.h if s else None, None, rows, k, n,
+                      qd.LINEAR_QKNORM, None, None, 0, 0, nq.h, nk.h, ct.h, st.h, rope_rows, 1e-6)
+    gpu.check(qd.lib().qw_gpu_qkv_linear(gpu.h, C.byref(d), kt.h, vt.h, at), "qkv")
+    gpu.submit()
+    want = ref.read().reshape(rows, 3, H)
+    assert np.array_equal(out.read().reshape(rows, 3, H)[:, 0], want[:, 0])
+    for i, t in ((1, kt), (2, vt)):
+        got = t.read().reshape(rows + 16, H)
+        assert (got[:8] == 0x1234).all() and (got[rows + 8:] == 0x1234).all()
+        assert np.array_equal(got[8:rows + 8], want[:, i])
+    d.epilogue = qd.LINEAR_STORE
+    assert not qd.lib().qw_gpu_qkv_linear(gpu.h, C.byref(d), kt.h, vt.h, at)
+    d.epilogue = qd.LINEAR_QKNORM
+    assert not qd.lib().qw_gpu_qkv_linear(gpu.h, C.byref(d), kt.h, vt.h, at + 9 * H)
+    gpu.submit()
+
+
+def test_block_kv_outputs(gpu, qd, oracle):
+    """K/V outputs that attention reads in place (aligned, apart), and ones it
+    cannot (at an odd element, or one tensor for both): the same hidden state
+    and the same rows."""
+    T, R = 16, 80
+    cfg = dict(hidden=256, heads=2, mlp_width=512, text_dim=256, z_dim=64, layers=1, mlp_act=0,
+               adaln_shift=0, has_bias=0, text_causal=1, int8_weights=0)
+    dit = qd.Dit(gpu, cfg, 5)
+    H = 256
+    x, mod = synth(oracle, R * H, 1), synth(oracle, 2 * 4 * H, 2, 0.2)
+    cos, sin = oracle.rope_tables(T, 8, 8)
+    ct, st, mt = gpu.put(cos), gpu.put(sin), gpu.put(mod)
+    rm = gpu.put((np.arange(R) < T).astype(np.uint32))
+    res = []
+    for form in ("none", "aligned", "odd", "one"):
+        h = gpu.put(x)
+        a, b = gpu.new(R * H + 8, qd.BF16), gpu.new(R * H + 8, qd.BF16)
+        kv = {"none": (None, None), "aligned": (a, b), "one": (a, a),
+              "odd": (a.view(2, R * H), b.view(2, R * H))}[form]
+        dit.block(0, h, mt, ct, st, rm, R, T, k_out=kv[0], v_out=kv[1])
+        gpu.submit()
+        res.append((h.read(), [t.read()[:R * H] if t else None for t in kv]))
+    dit.close()
+    for h, _ in res[1:]:
+        assert np.array_equal(h, res[0][0])
+    assert np.array_equal(res[1][1][0], res[2][1][0])
+    assert np.array_equal(res[1][1][1], res[2][1][1])
+    assert np.array_equal(res[3][1][0], res[1][1][1])  # v after k, in one tensor
