@@ -52,7 +52,8 @@ def int8_in_lds(M, K, N, cus=256):
     kernels (or, for at most 8 rows, the GEMV kernels widen in registers).
     A launch of at most cus / 2 tiles widens by a pass; a larger one of
     fewer than 512 rows stays on "_w8"; from 512 rows "_w8" needs K >= 8192
-    and a shape on which the bf16 kernels would not take 224-row tiles."""
+    and a shape on which the bf16 kernels would not take lower tiles (told
+    here by 224-row ones, which settles it at this workload's shapes)."""
     tn = (N + 255) // 256
     tiles = (M + 255) // 256 * tn
     if M <= 8 or 2 * tiles <= cus:
@@ -103,7 +104,7 @@ def kernel_breakdown(qd, gpu, reps=10):
     library's stream. `ms` is the int8 linear as the step runs it: at this
     workload all four are two launches, the weight widening pass
     (qw_widen_i8_bf16) and the bf16 GEMM with the scale in its epilogue (the
-    out and down projections on 224-row tiles), both also timed on their own
+    out and down projections on 224- and 192-row tiles), both also timed on their own
     (`widen_ms`, `gemm_ms`); a shape the library runs on a "_w8" kernel (the
     int8 weight widened in LDS inside the GEMM) is one launch, `gemm_ms`
     being that launch."""
@@ -424,7 +425,7 @@ def profile_kernel(qd, gpu, reps=5):
     size (the counter calibration: 256 MiB read + 256 MiB written), then
     the dominant GEMM -- the down projection, M=8704 K=12288 N=3072, on the
     int8 weight with the residual-gate epilogue, as the step runs it (the
-    widening pass qw_widen_i8_bf16, then qw_gemm_bf16_gate_t224) -- `reps`
+    widening pass qw_widen_i8_bf16, then qw_gemm_bf16_gate_mix) -- `reps`
     times. Nothing is timed or printed as a result."""
     H, F, M = CFG["hidden"], CFG["mlp_width"], BATCH * (TEXT + GH * GW)
     L = qd.lib()
@@ -682,9 +683,9 @@ def main():
                                "int8 weight widened to bf16 in LDS once per workgroup, scale "
                                "and residual gate in the epilogue)"
                                if int8_in_lds(down["M"], down["K"], down["N"]) else
-                               "qw_widen_i8_bf16 + qw_gemm_bf16_gate_t224 (down projection, "
+                               "qw_widen_i8_bf16 + qw_gemm_bf16_gate_mix (down projection, "
                                "M=8704 K=12288 N=3072: the int8 weight widened to bf16 by a "
-                               "pass, then 224 x 256 tiles in 2 waves, scale and residual "
+                               "pass, then 224- and 192-row tiles in 2 rounds, scale and residual "
                                "gate in the epilogue; the span covers both launches)"),
                     "flop_per_launch": fl, "ms_per_launch": down["ms"],
                     "ms_per_launch_alone": brk["down"]["ms"] if brk else None,
