@@ -518,7 +518,7 @@ __device__ __forceinline__ void gemm_epilogue_swiglu(const qw_gemm_args &a, Slab
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const uint32_t g =
-                    pack_bf(silu_fast_f(y[0][2 * j]), silu_fast_f(y[0][2 * j + 1]));
+                    pack_bf(silu_epi_f(y[0][2 * j]), silu_epi_f(y[0][2 * j + 1]));
                 pk[j] = pack_bf(lo_bf(g) * y[1][2 * j], hi_bf(g) * y[1][2 * j + 1]);
             }
             __builtin_amdgcn_raw_buffer_store_b128(u32x4{pk[0], pk[1], pk[2], pk[3]}, out_rsrc,
