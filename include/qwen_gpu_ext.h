@@ -137,8 +137,10 @@ int qw_gpu_linear_swiglu(h3_gpu *gpu, const qw_linear_desc *desc);
 /* The QKNORM linear with the k and v thirds of its output (after the norm and
  * the rotation) in tensors of their own, rows [rows, cols / 3] at kv_offset
  * elements: a cache that attention reads, without a copy. Columns cols / 3 and
- * up of out are left undefined. The values are qw_gpu_linear's. No
- * counterpart in the reference. */
+ * up of out are left undefined. The values are qw_gpu_linear's. Both outputs
+ * start at 16-byte addresses and overlap neither each other nor in or out
+ * (else the call is refused, whatever rope_rows is). No counterpart in the
+ * reference. */
 int qw_gpu_qkv_linear(h3_gpu *gpu, const qw_linear_desc *desc, h3_gpu_tensor *k,
                       h3_gpu_tensor *v, size_t kv_offset);
 /* No counterpart in the reference. For callers that cannot allocate

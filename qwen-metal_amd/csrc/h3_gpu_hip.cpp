@@ -1526,6 +1526,21 @@ extern "C" int qw_gpu_qkv_linear(h3_gpu *g, const qw_linear_desc *d, h3_gpu_tens
     if (!fits(k, kv_offset, n) || !fits(v, kv_offset, n))
         return fail(g, "qkv_linear: k or v too small");
     if (d->rows == 0 || d->cols == 0) return 1;
+    /* The epilogue stores k and v 16 bytes at a time, in workgroups that run
+     * in any order beside those that read in and write out; the copies below
+     * would take less, but what is accepted does not depend on the table. */
+    const uintptr_t kp = (uintptr_t)k->ptr + kv_offset * 2, vp = (uintptr_t)v->ptr + kv_offset * 2;
+    if ((kp | vp) % 16) return fail(g, "qkv_linear: k and v must be 16-byte aligned");
+    auto apart = [&](uintptr_t p, const h3_gpu_tensor *t, size_t off, size_t elements) {
+        const uintptr_t b = t ? (uintptr_t)t->ptr + off * 2 : 0;
+        return p + n * 2 <= b || b + elements * 2 <= p;
+    };
+    const size_t in_n = (size_t)(d->rows - 1) * d->lda + d->k;
+    const size_t out_n = (size_t)(d->rows - 1) * d->ldc + d->cols;
+    for (uintptr_t p : {kp, vp})
+        if (!apart(p, d->in, d->in_offset, in_n) || !apart(p, d->out, d->out_offset, out_n))
+            return fail(g, "qkv_linear: k or v overlaps the input or the output");
+    if (!apart(kp, v, kv_offset, n)) return fail(g, "qkv_linear: k and v overlap");
     if (d->rope_rows < 128 || n * 2 >= (1ull << 31))
         return linear_impl(g, d, 0) &&
                qw_gpu_copy_rows(g, k, kv_offset, H, d->out, H, d->ldc, d->rows, H) &&

@@ -51,6 +51,34 @@ def test_qkv_linear_outputs(gpu, qd, oracle, rows, k, heads, int8, rope_rows):
     gpu.submit()
 
 
+@pytest.mark.parametrize("rope_rows", [100, 200])  # copied out, and stored by the epilogue
+def test_qkv_linear_refusals(gpu, qd, rope_rows):
+    """What k and v may be does not depend on the RoPE table's length: apart,
+    16-byte aligned, and clear of the input and the output."""
+    rows, k, H = 24, 512, 128
+    n = 3 * H
+    x, w, out = (gpu.new(m, qd.BF16) for m in (rows * k + rows * H, n * k, rows * n + rows * H))
+    nq, ct = gpu.new(128, qd.BF16), gpu.new(rope_rows * 64, qd.F32)
+    kv = gpu.new(4 * rows * H, qd.BF16)
+    size = rows * H
+    d = qd.LinearDesc(out.h, 0, n, x.h, 0, k, w.h, None, None, rows, k, n, qd.LINEAR_QKNORM, None,
+                      None, 0, 0, nq.h, nq.h, ct.h, ct.h, rope_rows, 1e-6)
+    call = lambda a, b, off=0: qd.lib().qw_gpu_qkv_linear(gpu.h, C.byref(d), a.h, b.h, off)  # noqa: E731
+    assert call(kv, kv.view(size, size))
+    assert call(kv.view(size, size), kv)
+    assert call(out.view(rows * n, size), x.view(rows * k, size))
+    assert not call(kv, kv)
+    assert not call(kv, kv.view(size - 8, size)) and not call(kv.view(size - 8, size), kv)
+    for off in (1, 2, 4):
+        assert not call(kv, kv.view(2 * size, 2 * size), off)
+        assert not call(kv.view(off, size), kv.view(2 * size, size))
+        assert not call(kv, kv.view(2 * size + off, size))
+    assert call(kv, kv.view(2 * size, 2 * size), 8)
+    assert not call(out.view(rows * n - 8, size), kv) and not call(kv, out.view(0, size))
+    assert not call(x.view(rows * k - 8, size), kv) and not call(kv, x.view(0, size))
+    gpu.submit()
+
+
 def test_block_kv_outputs(gpu, qd, oracle):
     """K/V outputs that attention reads in place (aligned, apart), and ones it
     cannot (at an odd element, or one tensor for both): the same hidden state
