@@ -1549,21 +1549,20 @@ extern "C" int qw_gpu_qkv_linear(h3_gpu *g, const qw_linear_desc *d, h3_gpu_tens
     return linear_impl(g, d, 0, &kv);
 }
 
-/* The tile kernels from 9 rows on; fewer rows keep the streaming linear and
- * the separate pass over its few rows, in the runtime's scratch buffer. */
+/* The tile kernels from 9 rows on, and for an output that the separate pass
+ * cannot write (strided, or at an offset); else at most 8 rows keep the
+ * streaming linear and that pass, in the runtime's scratch buffer. */
 static void *scratch(h3_gpu *g, size_t bytes);
 extern "C" int qw_gpu_linear_swiglu(h3_gpu *g, const qw_linear_desc *d) {
     if (!g || !d) return 0;
     if (!check_epilogue(g, d)) return 0;
     if (d->epilogue != QW_LINEAR_STORE) return fail(g, "linear_swiglu: epilogue must be STORE");
     qw_linear_desc t = *d;
-    if (d->rows > 8) {
+    if (d->rows > 8 || d->cols % 16 || d->ldc != d->cols / 2 || d->out_offset) {
         t.epilogue = QW_EPI_SWIGLU;
         return linear_impl(g, &t, 0);
     }
     if (!d->rows || !d->cols) return 1;
-    if (d->cols % 16 || d->ldc != d->cols / 2 || d->out_offset)
-        return fail(g, "linear_swiglu: at most 8 rows go to a whole [rows, cols / 2] output");
     const size_t wide = (size_t)d->rows * d->cols;
     void *s = scratch(g, wide * 2);
     if (!s) return fail(g, "linear_swiglu: scratch allocation failed");

@@ -103,6 +103,32 @@ def test_swiglu_linear_gate_range(gpu, qd, oracle):
     assert (np.abs(got)[~live] <= 1e-35).all()
 
 
+@pytest.mark.parametrize("rows", [1, 8, 9])
+@pytest.mark.parametrize("ldc,off", [(80, 0), (72, 16), (92, 4)])
+def test_swiglu_linear_strided_output(gpu, qd, oracle, rows, ldc, off):
+    """A strided output, or one at an offset, at any row count: the dense
+    output's values (within the order of the sums), nothing beside them."""
+    k, F = 128, 72
+    x = gpu.put(oracle.fill_normal_bf16(rows * k, 7, 1, 1.0))
+    w = gpu.put(oracle.fill_normal_bf16(2 * F * k, 7, 2, 1.5 / np.sqrt(k)))
+    dense = gpu.new(rows * F, qd.BF16)
+    gpu.check(fused(gpu, qd, dense, x, w, rows, k, F), "dense")
+    out = gpu.put(np.full(off + rows * ldc, 0x1234, np.uint16))
+    gpu.check(fused(gpu, qd, out, x, w, rows, k, F, ldc=ldc, out_offset=off), "strided")
+    gpu.submit()
+    got = out.read()
+    assert (got[:off] == 0x1234).all()
+    got = got[off:].reshape(rows, ldc)
+    assert (got[:, F:] == 0x1234).all()
+    a, b = oracle.bf16_to_f32(got[:, :F].ravel()), oracle.bf16_to_f32(dense.read())
+    # g and u each a bf16 ulp apart at most where their sums' order differs
+    # (silu passes at most 1.1 of g's step on), silu and the product one more
+    # rounding each: 4 ulps of 2^-8, or of what a gate that cancels leaves
+    assert (np.abs(a - b) <= 4 * 2.0 ** -8 * np.abs(b) + 2.0 ** -8).all()
+    if rows == 9:
+        assert np.array_equal(a, b)  # one kernel
+
+
 def test_swiglu_linear_refusals(gpu, qd):
     F, k, rows = 64, 64, 16
     x, w, out = gpu.new(rows * k, qd.BF16), gpu.new(2 * F * k, qd.BF16), gpu.new(rows * F, qd.BF16)
@@ -111,7 +137,8 @@ def test_swiglu_linear_refusals(gpu, qd):
     assert not fused(gpu, qd, out, x, w, rows + 1, k, F)
     assert not fused(gpu, qd, out, x, w, rows, k, F, epilogue=qd.LINEAR_GELU)
     assert not fused(gpu, qd, out, x, w, rows, k, F, epilogue=4)
-    assert not fused(gpu, qd, out, x, w, 4, k, F, ldc=F + 8)
+    assert not fused(gpu, qd, out, x, w, 4, k, F, ldc=F - 8)
+    assert not fused(gpu, qd, out, x, w, rows, k, F, ldc=F + 8)  # past the output's end
     d = qd.LinearDesc(out.h, 0, F, x.h, 0, k, w.h, None, None, rows, k, F, 4, None, None, 0, 0,
                       None, None, None, None, 0, 0.0)
     assert not qd.lib().qw_gpu_linear(gpu.h, C.byref(d))  # not an epilogue of qw_gpu_linear
