@@ -92,6 +92,7 @@ struct h3_gpu {
     int mixed;      /* 192- and 224-row tiles allowed (QW_GEMM_T224=0 turns them off, for measurement) */
     uint32_t split_min_steps, split_force; /* measurement: QW_SPLIT_MIN_STEPS, QW_SPLIT_FORCE */
     uint32_t widen_min_rows; /* int8: fewest rows for the widening route (QW_WIDEN_MIN_ROWS) */
+    int workspaces; /* split partials and widened copies allowed (QW_WORKSPACES=0: as if none could be had) */
     int narrow;     /* narrow tiles allowed (QW_GEMM_HALF_SMALL=0: off) */
     /* qw_gpu_span_*: event pairs recorded on the stream, read after a sync */
     hipEvent_t *span_ev;
@@ -213,6 +214,8 @@ extern "C" h3_gpu *h3_gpu_create(const char *code_object_path, char *error,
     if (const char *r = getenv("QW_SPLIT_FORCE")) g->split_force = (uint32_t)atoi(r);
     g->widen_min_rows = QW_WIDEN_MIN_ROWS;
     if (const char *r = getenv("QW_WIDEN_MIN_ROWS")) g->widen_min_rows = (uint32_t)atoi(r);
+    g->workspaces = 1;
+    if (const char *r = getenv("QW_WORKSPACES")) g->workspaces = atoi(r) != 0;
     g->narrow = 1;
     if (const char *r = getenv("QW_GEMM_HALF_SMALL")) g->narrow = atoi(r) != 0;
     g->cus = 0;
@@ -1125,12 +1128,37 @@ static double narrow_us(const h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t 
     return best;
 }
 
-/* Whether a launch may be split: the workspace is there, or can be made now
- * (not while the stream is being captured into a graph). */
-static int can_split(h3_gpu *g) {
+/* Whether workspaces may be made now: not while the stream is being captured
+ * into a graph, nor where they are switched off. */
+static int can_allocate(h3_gpu *g) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    return g->sk_part ||
-           (hipStreamIsCapturing(g->stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone);
+    return g->workspaces && hipStreamIsCapturing(g->stream, &st) == hipSuccess &&
+           st == hipStreamCaptureStatusNone;
+}
+
+/* Partial sums and piece counters of split tiles (and of split attention
+ * blocks), from the first one on. 0 where there are none and none can be had:
+ * the launch then runs whole. */
+#define QW_FLAGS 4
+static int split_workspace(h3_gpu *g) {
+    if (g->sk_part) return 1;
+    if (!can_allocate(g)) return 0;
+    hipStreamSynchronize(g->stream);
+    const size_t n = (size_t)QW_SPLIT_MAX_PIECES * g->cus * 256 * 256 * 4;
+    const size_t flags = (size_t)g->cus * QW_FLAGS * 4;
+    if (hipMalloc((void **)&g->sk_part, n) == hipSuccess) {
+        if (hipMalloc((void **)&g->sk_flag, flags) == hipSuccess &&
+            hipMemset(g->sk_flag, 0, flags) == hipSuccess) {
+            g->stats.allocated_bytes += n + flags;
+            return 1;
+        }
+        if (g->sk_flag) hipFree(g->sk_flag);
+        hipFree(g->sk_part);
+    }
+    (void)hipGetLastError(); /* seen to here */
+    g->sk_part = NULL;
+    g->sk_flag = NULL;
+    return 0;
 }
 
 /* How the rows of a linear on bf16 W run: the first `wide` of them (a
@@ -1142,11 +1170,11 @@ struct linear_plan {
     uint32_t wide, mb, s;
     wide_plan w; /* how the first run */
 };
-static linear_plan plan_linear(h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t ksteps) {
+static linear_plan plan_linear(h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t ksteps,
+                               uint32_t max_s) {
     linear_plan p = {rows, 0, 1, plan_wide(g, rows, cols, ksteps)};
     if (!g->narrow) return p;
     uint32_t mb, s;
-    const uint32_t max_s = can_split(g) ? 8 : 1;
     double best = p.w.us;
     const double all = narrow_us(g, rows, cols, ksteps, max_s, &mb, &s);
     if (all < 0.98 * best) {
@@ -1167,25 +1195,22 @@ static linear_plan plan_linear(h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t
     return p;
 }
 
-/* partial sums and piece counters of split tiles (and of split attention
- * blocks), from the first one on */
-#define QW_FLAGS 4
-static int split_workspace(h3_gpu *g) {
-    if (g->sk_part) return 1;
+/* the widened copy of an int8 weight, grown to `bytes`; 0 where it cannot be
+ * (the "_w8" kernels need none) */
+static int widen_workspace(h3_gpu *g, size_t bytes) {
+    if (g->widen_bytes >= bytes) return 1;
+    if (!can_allocate(g)) return 0;
     hipStreamSynchronize(g->stream);
-    const size_t n = (size_t)QW_SPLIT_MAX_PIECES * g->cus;
-    g->stats.allocated_bytes += n * 256 * 256 * 4 + (size_t)g->cus * QW_FLAGS * 4;
-    if (hipMalloc((void **)&g->sk_part, n * 256 * 256 * 4) != hipSuccess) {
-        g->sk_part = NULL;
-        return fail(g, "linear: split-tile workspace allocation failed");
+    if (g->widen) hipFree(g->widen);
+    g->widen = NULL;
+    g->widen_bytes = 0;
+    if (hipMalloc(&g->widen, bytes) != hipSuccess) {
+        (void)hipGetLastError(); /* seen to here */
+        g->widen = NULL;
+        return 0;
     }
-    if (hipMalloc((void **)&g->sk_flag, (size_t)g->cus * QW_FLAGS * 4) != hipSuccess ||
-        hipMemset(g->sk_flag, 0, (size_t)g->cus * QW_FLAGS * 4) != hipSuccess) {
-        hipFree(g->sk_part);
-        g->sk_part = NULL;
-        g->sk_flag = NULL;
-        return fail(g, "linear: split-tile flag allocation failed");
-    }
+    g->widen_bytes = bytes;
+    g->stats.allocated_bytes += bytes; /* runtime workspaces count too */
     return 1;
 }
 
@@ -1310,7 +1335,7 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc,
      * pass plus the bf16 kernel. */
     const linear_plan wide_all = {d->rows, 0, 1, plan_wide(g, d->rows, d->cols, d->k / 64)};
     linear_plan plan = no_alloc || (int8 && g->int8_route == QW_INT8_W8)
-                           ? wide_all : plan_linear(g, d->rows, d->cols, d->k / 64);
+                           ? wide_all : plan_linear(g, d->rows, d->cols, d->k / 64, 8);
     /* K >= 8192 keeps the in-LDS widening, unless the widened weight's bf16
      * kernel takes lower tiles (224-row ones for the down projection at M = 8704: whole
      * steps 64.07 against 65.39 ms with the pass and 224-row tiles, medians
@@ -1325,23 +1350,15 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc,
      * 64-66 / 48-55, out 63 / 35-38, up 65-67 / 56-59, down 74-84 / 66-76). */
     const int small_w = g->int8_route == QW_INT8_AUTO && plan.mb != 0;
     if (small_w) route = QW_INT8_WIDEN;
+    const size_t weights = (size_t)d->cols * d->k;
     const int widen = int8 && !no_alloc && (d->rows >= g->widen_min_rows || small_w) &&
-                      route == QW_INT8_WIDEN;
+                      route == QW_INT8_WIDEN && widen_workspace(g, weights * 2);
     if (int8 && !widen) plan = wide_all;
+    if (plan.s > 1 && !split_workspace(g))
+        plan = plan_linear(g, d->rows, d->cols, d->k / 64, 1);
     const void *wptr = d->weight->ptr;
     if (widen) {
-        const size_t n = (size_t)d->cols * d->k, bytes = n * 2;
-        if (g->widen_bytes < bytes) {
-            hipStreamSynchronize(g->stream);
-            if (g->widen) hipFree(g->widen);
-            g->widen = NULL;
-            g->widen_bytes = 0;
-            if (hipMalloc(&g->widen, bytes) != hipSuccess)
-                return fail(g, "linear: widen buffer allocation (%zu bytes) failed", bytes);
-            g->widen_bytes = bytes;
-            g->stats.allocated_bytes += bytes; /* runtime workspaces count too */
-        }
-        if (!widen_launch(g, (uint16_t *)g->widen, (const int8_t *)d->weight->ptr, n)) return 0;
+        if (!widen_launch(g, (uint16_t *)g->widen, (const int8_t *)d->weight->ptr, weights)) return 0;
         wptr = g->widen;
     }
     qw_gemm_args a;
@@ -1405,7 +1422,6 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc,
             /* narrow_us keeps the pieces within a round: checked, so that a
              * change to it fails loudly */
             if (np > g->cus) return fail(g, "linear: internal error: %llu pieces", (unsigned long long)np);
-            if (!split_workspace(g)) return 0;
             n.sk_part = g->sk_part;
             n.sk_flag = g->sk_flag;
         }
@@ -1452,8 +1468,7 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc,
          * (down projection shape, bf16 W, M = 8704: 500 us on 224-row tiles
          * against 568 with 256-row tiles and a 3-piece tail) */
         const uint32_t s = mix ? 1u : split_choice(g, tiles, d->k / 64);
-        if (s > 1) {
-            if (!split_workspace(g)) return 0;
+        if (s > 1 && split_workspace(g)) {
             const uint32_t R = tiles % g->cus;
             /* the workspace holds QW_SPLIT_MAX_PIECES * cus partials and
              * cus counters; split_choice keeps within both */
@@ -1784,9 +1799,8 @@ extern "C" int qw_gpu_attention_bf16(h3_gpu *g, const qw_attention_desc *d) {
      * a block, a partial a piece) or there is none to be had */
     if (p.split == 1 || R > (uint64_t)QW_FLAGS * g->cus ||
         np * QW_ATTN_PART(threads / 64) > (size_t)QW_SPLIT_MAX_PIECES * g->cus * 256 * 256 * 4 ||
-        !can_split(g))
+        !split_workspace(g))
         return launch(g, w4 ? K_ATTN_W4 : K_ATTN, dim3(nb), dim3(threads), a);
-    if (!split_workspace(g)) return 0;
     a.dp_blocks = p.dp;
     a.split = p.split;
     a.part = g->sk_part;
