@@ -1352,7 +1352,8 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc,
     if (small_w) route = QW_INT8_WIDEN;
     const size_t weights = (size_t)d->cols * d->k;
     const int widen = int8 && !no_alloc && (d->rows >= g->widen_min_rows || small_w) &&
-                      route == QW_INT8_WIDEN && widen_workspace(g, weights * 2);
+                      route == QW_INT8_WIDEN && weights * 2 < (1ull << 31) /* a buffer's range */ &&
+                      widen_workspace(g, weights * 2);
     if (int8 && !widen) plan = wide_all;
     if (plan.s > 1 && !split_workspace(g))
         plan = plan_linear(g, d->rows, d->cols, d->k / 64, 1);

@@ -110,3 +110,26 @@ def test_wide_split_tiles(qd, oracle, monkeypatch, case):
         K.test_linear_split_tiles(gpu, qd, oracle, *case)
     finally:
         gpu.close()
+
+
+def test_narrow_int8_weight_past_a_buffer_widened(gpu, qd, oracle):
+    """An int8 weight of over 2^30 elements, whose widened copy would pass the 2
+    GiB that a buffer covers: a launch that narrow tiles would suit stays on
+    the kernels that widen inside."""
+    rows, k, n, step = 60, 33792, 33024, 4128
+    x = synth(oracle, rows * k, 81)
+    xt, w, q, s = gpu.put(x), gpu.new(step * k, qd.BF16), gpu.new(n * k, qd.I8), gpu.new(n, qd.F32)
+    for r in range(0, n, step):
+        gpu.check(qd.lib().qw_gpu_fill_normal_bf16(gpu.h, w.h, 0, step * k, 3, r, 0.02, 0.0), "fill")
+        qv, sv = q.view(r * k, step * k), s.view(r, step)
+        gpu.check(qd.lib().h3_gpu_quantize_weight_int8(gpu.h, qv.h, sv.h, w.h, step, k), "quantize")
+    out = gpu.new(rows * n, qd.BF16)
+    gpu.linear(out, xt, q, rows, k, n, wscale=s)
+    gpu.submit()
+    got = out.read().reshape(rows, n)
+    for c in (0, 8, 16384, n - 16):  # 8 columns at a time
+        qc = q.view(c * k, 8 * k).read()
+        lin = oracle.linear_i8(x, qc, s.view(c, 8).read(), None, rows, k, 8)
+        mag = np.abs(oracle.bf16_to_f32(x).reshape(rows, k)) @ np.abs(qc.reshape(8, k).T.astype(np.float32))
+        assert_linear_close(oracle, np.ascontiguousarray(got[:, c:c + 8]).ravel(), lin.ravel(),
+                            (mag * s.view(c, 8).read()).ravel())
