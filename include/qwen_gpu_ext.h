@@ -158,6 +158,14 @@ int qw_gpu_qkv_linear(h3_gpu *gpu, const qw_linear_desc *desc, h3_gpu_tensor *k,
  * contents. */
 int qw_gpu_linear_static(h3_gpu *gpu, const qw_linear_desc *desc);
 
+/* No counterpart in the reference (a measurement and test aid): the kernels
+ * that the last linear (or attention) call on this context launched, in
+ * order, separated by spaces, each with what applies of ":split=s" (its tiles
+ * or last blocks cut in s pieces), ":half=n" (n half tiles) and ":from=r" (r
+ * rows above it, or whole blocks ahead of the cut ones). Writes at most size
+ * bytes and returns the number of kernels, or -1. */
+int qw_gpu_last_route(const h3_gpu *gpu, char *text, size_t size);
+
 /* No counterpart in the reference (a measurement aid, like h3_gpu_timer_*):
  * spans time pieces of the work on the stream without synchronising it.
  * span_begin records an event tagged `tag`, span_end the matching end

@@ -94,6 +94,9 @@ struct h3_gpu {
     uint32_t widen_min_rows; /* int8: fewest rows for the widening route (QW_WIDEN_MIN_ROWS) */
     int workspaces; /* split partials and widened copies allowed (QW_WORKSPACES=0: as if none could be had) */
     int narrow;     /* narrow tiles allowed (QW_GEMM_HALF_SMALL=0: off) */
+    /* qw_gpu_last_route: the launches of the last linear or attention call */
+    struct { int kid; uint32_t split, half, from; } route[4];
+    int route_n;
     /* qw_gpu_span_*: event pairs recorded on the stream, read after a sync */
     hipEvent_t *span_ev;
     int *span_tag;
@@ -197,6 +200,7 @@ extern "C" h3_gpu *h3_gpu_create(const char *code_object_path, char *error,
     g->scratch_bytes = 0;
     g->widen = NULL;
     g->widen_bytes = 0;
+    g->route_n = 0;
     g->span_ev = NULL;
     g->span_tag = NULL;
     g->span_n = 0;
@@ -595,6 +599,29 @@ static int launch(h3_gpu *g, int kid, dim3 grid, dim3 block, const T &args) {
     if (e != hipSuccess) return fail(g, "launch %s: %s", k_names[kid], hipGetErrorString(e));
     g->stats.direct_dispatches++;
     return 1;
+}
+
+/* launch(), kept for qw_gpu_last_route: split: pieces a tile or block is cut
+ * into, half: half tiles, from: first row */
+template <typename T>
+static int launch_step(h3_gpu *g, int kid, dim3 grid, dim3 block, const T &args, uint32_t split,
+                       uint32_t half = 0, uint32_t from = 0) {
+    if (g->route_n < 4) g->route[g->route_n++] = {kid, split, half, from};
+    return launch(g, kid, grid, block, args);
+}
+
+extern "C" int qw_gpu_last_route(const h3_gpu *g, char *text, size_t size) {
+    if (!g || !text || !size) return -1;
+    size_t n = 0;
+    text[0] = '\0';
+    for (int i = 0; i < g->route_n && n < size; i++) {
+        const auto &r = g->route[i];
+        n += snprintf(text + n, size - n, "%s%s", i ? " " : "", k_names[r.kid]);
+        if (r.split > 1 && n < size) n += snprintf(text + n, size - n, ":split=%u", r.split);
+        if (r.half && n < size) n += snprintf(text + n, size - n, ":half=%u", r.half);
+        if (r.from && n < size) n += snprintf(text + n, size - n, ":from=%u", r.from);
+    }
+    return g->route_n;
 }
 
 static bool fits(const h3_gpu_tensor *t, size_t offset, size_t elements) {
@@ -1317,7 +1344,8 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc,
         const int kid = (int8 ? K_GEMV_I8_STORE : K_GEMV_BF16_STORE) +
                         (d->epilogue == QW_LINEAR_GELU ? 1 : 0);
         const uint32_t waves = (d->cols + 1) / 2; /* 2 columns per wave */
-        return launch(g, kid, dim3((waves + 3) / 4), dim3(256), a);
+        g->route_n = 0;
+        return launch_step(g, kid, dim3((waves + 3) / 4), dim3(256), a, 1);
     }
     /* int8 weights: the "_w8" kernels widen each int8 W tile once per
      * workgroup into the bf16 W stage in LDS (no copy through HBM, half
@@ -1351,6 +1379,7 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc,
     const int small_w = g->int8_route == QW_INT8_AUTO && plan.mb != 0;
     if (small_w) route = QW_INT8_WIDEN;
     const size_t weights = (size_t)d->cols * d->k;
+    g->route_n = 0;
     const int widen = int8 && !no_alloc && (d->rows >= g->widen_min_rows || small_w) &&
                       route == QW_INT8_WIDEN && weights * 2 < (1ull << 31) /* a buffer's range */ &&
                       widen_workspace(g, weights * 2);
@@ -1427,7 +1456,8 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc,
             n.sk_flag = g->sk_flag;
         }
         static const int first[4] = {K_GEMM_N1, K_GEMM_N2, K_GEMM_N3, K_GEMM_N4};
-        if (!launch(g, first[plan.mb - 1] + d->epilogue, dim3((uint32_t)np), dim3(threads), n))
+        if (!launch_step(g, first[plan.mb - 1] + d->epilogue, dim3((uint32_t)np), dim3(threads), n,
+                         plan.s, 0, plan.wide))
             return 0;
         if (!plan.wide) return 1;
         a.m = plan.wide;
@@ -1498,8 +1528,8 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc,
          * 500 against 530 us; at 36 and more columns a range is 3-7% ahead) */
         a.mix_dealt = a.tiles_n <= 16 && d->k >= 8192;
         const uint32_t n = (a.mix_rows1 + a.mix_rows2) * a.tiles_n;
-        return launch(g, K_GEMM_BF16_STORE_MIX + d->epilogue, dim3(n < g->cus ? n : g->cus),
-                      dim3(threads), a);
+        return launch_step(g, K_GEMM_BF16_STORE_MIX + d->epilogue, dim3(n < g->cus ? n : g->cus),
+                           dim3(threads), a, 1);
     }
     if (a.split == 1 && grid > g->cus && g->cus % 8 == 0) {
         grid = g->cus;
@@ -1513,7 +1543,7 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc,
             a.half_count = 2 * R;
         }
     }
-    return launch(g, kid, dim3(grid), dim3(threads), a);
+    return launch_step(g, kid, dim3(grid), dim3(threads), a, a.split, a.half_count);
 }
 
 static int check_epilogue(h3_gpu *g, const qw_linear_desc *d) {
@@ -1791,6 +1821,7 @@ extern "C" int qw_gpu_attention_bf16(h3_gpu *g, const qw_attention_desc *d) {
     const uint64_t nwg = (uint64_t)((d->q_rows + aqb - 1) / aqb) * d->heads * d->batch;
     if (nwg >= (1ull << 31)) return fail(g, "attention: grid too large");
     const attn_plan p = plan_attention(g, d);
+    g->route_n = 0;
     /* the launch's own kernel: a small plan keeps its pieces on either */
     const int w4 = p.small && g->attn_small;
     const uint32_t threads = w4 ? g->attn4_threads : g->attn_threads, qb = threads / 2;
@@ -1801,13 +1832,13 @@ extern "C" int qw_gpu_attention_bf16(h3_gpu *g, const qw_attention_desc *d) {
     if (p.split == 1 || R > (uint64_t)QW_FLAGS * g->cus ||
         np * QW_ATTN_PART(threads / 64) > (size_t)QW_SPLIT_MAX_PIECES * g->cus * 256 * 256 * 4 ||
         !split_workspace(g))
-        return launch(g, w4 ? K_ATTN_W4 : K_ATTN, dim3(nb), dim3(threads), a);
+        return launch_step(g, w4 ? K_ATTN_W4 : K_ATTN, dim3(nb), dim3(threads), a, 1);
     a.dp_blocks = p.dp;
     a.split = p.split;
     a.part = g->sk_part;
     a.flag = g->sk_flag;
-    return launch(g, w4 ? K_ATTN_W4_SPLIT : K_ATTN_SPLIT, dim3((uint32_t)(p.dp + np)),
-                  dim3(threads), a);
+    return launch_step(g, w4 ? K_ATTN_W4_SPLIT : K_ATTN_SPLIT, dim3((uint32_t)(p.dp + np)),
+                       dim3(threads), a, p.split, 0, p.dp);
 }
 
 static int sdpa_contig(h3_gpu *g, h3_gpu_tensor *out, const h3_gpu_tensor *q,

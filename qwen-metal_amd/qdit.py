@@ -203,6 +203,7 @@ SIGNATURES = {
     "qw_pipe_rope_tables": (C.c_int, [vp, u32, u32, u32, vp, vp, C.c_char_p, sz]),
     "qw_pipe_rope_tables_host": (None, [u32, u32, u32, vp, vp]),
     "qw_pipe_rope_tables_blocks": (C.c_int, [vp, vp, vp, vp, u32, vp, vp, C.c_char_p, sz]),
+    "qw_gpu_last_route": (C.c_int, [vp, C.c_char_p, sz]),
     "qw_gpu_span_begin": (C.c_int, [vp, C.c_int]),
     "qw_gpu_span_end": (C.c_int, [vp]),
     "qw_gpu_span_collect": (C.c_int, [vp, vp, vp, C.c_int]),
@@ -335,6 +336,12 @@ class Gpu:
         s = Stats()
         lib().h3_gpu_get_stats(self.h, C.byref(s))
         return s
+
+    def route(self):
+        """The kernels of the last linear or attention call (qw_gpu_last_route)."""
+        text = C.create_string_buffer(512)
+        lib().qw_gpu_last_route(self.h, text, 512)
+        return text.value.decode()
 
     def timer_begin(self):
         self.check(lib().h3_gpu_timer_begin(self.h), "timer")
