@@ -77,3 +77,22 @@ def test_split_attention_large_scores(gpu, qd, oracle):
     ref = oracle.attention(q.ravel(), oracle.f32_to_bf16(kf).ravel(), v, lim, rows, rows, 1)
     assert np.isfinite(oracle.bf16_to_f32(got.ravel())).all()
     assert rel_l2(oracle.bf16_to_f32(got.ravel()), oracle.bf16_to_f32(ref).ravel()) < 5e-3
+
+
+@pytest.mark.parametrize("causal", [0, 1])
+def test_split_attention_more_text_rows_than_keys(gpu, qd, oracle, monkeypatch, causal):
+    """Text rows past the last key: the keys that whole blocks count."""
+    rows, kv, heads = 2600, 2000, 1
+    q, k, v = synth(oracle, rows * 128, 230), synth(oracle, kv * 128, 231), synth(oracle, kv * 128, 232)
+    got = run(gpu, qd, q, k, v, 1, rows, kv, heads, text_rows=rows, text_causal=causal)
+    assert "split=" in gpu.route()
+    monkeypatch.setenv("QW_WORKSPACES", "0")
+    whole = qd.Gpu()
+    try:
+        want = run(whole, qd, q, k, v, 1, rows, kv, heads, text_rows=rows, text_causal=causal)
+        assert "split=" not in whole.route()
+    finally:
+        whole.close()
+    a, b = (oracle.bf16_to_f32(x.ravel()).reshape(rows, 128) for x in (got, want))
+    for r in (range(0, kv), range(kv, rows)):
+        assert rel_l2(a[r], b[r]) < 5e-3
