@@ -161,9 +161,10 @@ int qw_gpu_linear_static(h3_gpu *gpu, const qw_linear_desc *desc);
 /* No counterpart in the reference (a measurement and test aid): the kernels
  * that the last linear (or attention) call on this context launched, in
  * order, separated by spaces, each with what applies of ":split=s" (its tiles
- * or last blocks cut in s pieces), ":half=n" (n half tiles) and ":from=r" (r
- * rows above it, or whole blocks ahead of the cut ones). Writes at most size
- * bytes and returns the number of kernels, or -1. */
+ * or last blocks cut in s pieces), ":half=n" (n half tiles), ":from=r" (r
+ * rows above it, or whole blocks ahead of the cut ones) and ":axh+bxl" (a tile
+ * rows of h rows, then b of l). Writes at most size bytes and returns the
+ * number of kernels, or -1. */
 int qw_gpu_last_route(const h3_gpu *gpu, char *text, size_t size);
 
 /* No counterpart in the reference (a measurement aid, like h3_gpu_timer_*):

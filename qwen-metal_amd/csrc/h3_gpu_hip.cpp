@@ -95,7 +95,7 @@ struct h3_gpu {
     int workspaces; /* split partials and widened copies allowed (QW_WORKSPACES=0: as if none could be had) */
     int narrow;     /* narrow tiles allowed (QW_GEMM_HALF_SMALL=0: off) */
     /* qw_gpu_last_route: the launches of the last linear or attention call */
-    struct { int kid; uint32_t split, half, from; } route[4];
+    struct { int kid; uint32_t split, half, from, h1, rows1, h2, rows2; } route[4];
     int route_n;
     /* qw_gpu_span_*: event pairs recorded on the stream, read after a sync */
     hipEvent_t *span_ev;
@@ -606,7 +606,7 @@ static int launch(h3_gpu *g, int kid, dim3 grid, dim3 block, const T &args) {
 template <typename T>
 static int launch_step(h3_gpu *g, int kid, dim3 grid, dim3 block, const T &args, uint32_t split,
                        uint32_t half = 0, uint32_t from = 0) {
-    if (g->route_n < 4) g->route[g->route_n++] = {kid, split, half, from};
+    if (g->route_n < 4) g->route[g->route_n++] = {kid, split, half, from, 0, 0, 0, 0};
     return launch(g, kid, grid, block, args);
 }
 
@@ -620,6 +620,8 @@ extern "C" int qw_gpu_last_route(const h3_gpu *g, char *text, size_t size) {
         if (r.split > 1 && n < size) n += snprintf(text + n, size - n, ":split=%u", r.split);
         if (r.half && n < size) n += snprintf(text + n, size - n, ":half=%u", r.half);
         if (r.from && n < size) n += snprintf(text + n, size - n, ":from=%u", r.from);
+        if (r.h1 && n < size)
+            n += snprintf(text + n, size - n, ":%ux%u+%ux%u", r.rows1, 32 * r.h1, r.rows2, 32 * r.h2);
     }
     return g->route_n;
 }
@@ -1528,8 +1530,12 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc,
          * 500 against 530 us; at 36 and more columns a range is 3-7% ahead) */
         a.mix_dealt = a.tiles_n <= 16 && d->k >= 8192;
         const uint32_t n = (a.mix_rows1 + a.mix_rows2) * a.tiles_n;
-        return launch_step(g, K_GEMM_BF16_STORE_MIX + d->epilogue, dim3(n < g->cus ? n : g->cus),
-                           dim3(threads), a, 1);
+        if (!launch_step(g, K_GEMM_BF16_STORE_MIX + d->epilogue, dim3(n < g->cus ? n : g->cus),
+                         dim3(threads), a, 1))
+            return 0;
+        auto &r = g->route[g->route_n - 1];
+        r.h1 = a.mix_h1, r.rows1 = a.mix_rows1, r.h2 = a.mix_h2, r.rows2 = a.mix_rows2;
+        return 1;
     }
     if (a.split == 1 && grid > g->cus && g->cus % 8 == 0) {
         grid = g->cus;

@@ -65,13 +65,16 @@ def test_narrow_tiles_store_gelu_gate(gpu, qd, oracle, rows, k, n):
     assert best.max() <= 1, best.max()
 
 
-@pytest.mark.parametrize("rows,k,heads", [(70, 512, 2), (320, 3072, 4), (640, 256, 24),
-                                          (4119, 512, 10)])
-def test_narrow_tiles_qknorm(gpu, qd, oracle, rows, k, heads):
+@pytest.mark.parametrize("rows,k,heads,route", [
+    (70, 512, 2, "qw_gemm_bf16_qkn_n1"), (320, 3072, 4, "qw_gemm_bf16_qkn_n1:split=4"),
+    (640, 256, 24, "qw_gemm_bf16_qkn_n4"), (4119, 512, 10, "qw_gemm_bf16_qkn_q"),
+    (11400, 512, 4, "qw_gemm_bf16_qkn_n1:from=10752 qw_gemm_bf16_qkn_q"),
+    (2900, 256, 17, "qw_gemm_bf16_qkn_n2:from=2304 qw_gemm_bf16_qkn_q")])
+def test_narrow_tiles_qknorm(gpu, qd, oracle, rows, k, heads, route):
     """The q/k norm + RoPE epilogue bit for bit against the plain linear and
     the standalone kernel (the same tiles, whatever the epilogue): rows past
-    a table's end wrap, and a last tile row's table rows start where it
-    does."""
+    a table's end wrap, and the table rows of narrow tiles below wide ones
+    start where those end."""
     n = 3 * heads * 128
     xt, wt, _, bt, _, _ = _operands(gpu, oracle, rows, k, n, False)
     rope_rows = 200
@@ -81,6 +84,7 @@ def test_narrow_tiles_qknorm(gpu, qd, oracle, rows, k, heads):
     fused, ref = gpu.new(rows * n, qd.BF16), gpu.new(rows * n, qd.BF16)
     gpu.linear(fused, xt, wt, rows, k, n, bias=bt, epilogue=qd.LINEAR_QKNORM,
                qknorm=(nq, nk, ct, st, rope_rows, 1e-6))
+    assert gpu.route() == route
     gpu.linear(ref, xt, wt, rows, k, n, bias=bt)
     gpu.check(qd.lib().qw_gpu_qk_norm_rope_bf16(gpu.h, ref.h, rows, heads, n, n // 3, nq.h, nk.h,
                                                  ct.h, st.h, rope_rows, 1e-6), "qk")
@@ -88,14 +92,31 @@ def test_narrow_tiles_qknorm(gpu, qd, oracle, rows, k, heads):
     assert np.array_equal(fused.read(), ref.read())
 
 
-@pytest.mark.parametrize("n,int8", [(1800, False), (1784, True)])
-def test_wide_224_row_tiles(qd, oracle, monkeypatch, n, int8):
-    """The shapes of test_linear_224_row_tiles_ragged_cols with narrow tiles
-    off, so that the 224-row kernels run them."""
+# columns: in 8 tile columns 184 tiles of 192 rows fit a round, in 12 the 240
+# of 224 rows do
+@pytest.mark.parametrize("n,int8,tiles", [(1800, False, "0x224+23x192"), (1784, True, "0x224+23x192"),
+                                          (3000, False, "0x256+20x224"), (2984, True, "0x256+20x224")])
+def test_wide_low_tiles(qd, oracle, monkeypatch, n, int8, tiles):
+    """test_linear_224_row_tiles_ragged_cols on tiles of 192 and 224 rows,
+    with narrow tiles off; int8 weights widened by a pass."""
     monkeypatch.setenv("QW_GEMM_HALF_SMALL", "0")
+    monkeypatch.setenv("QW_INT8_ROUTE", "widen")
     gpu = qd.Gpu()
     try:
         K.test_linear_224_row_tiles_ragged_cols(gpu, qd, oracle, n, int8)
+        assert gpu.route() == "qw_gemm_bf16_store_mix:" + tiles
+    finally:
+        gpu.close()
+
+
+def test_wide_half_tiles_qknorm(qd, oracle, monkeypatch):
+    """The q/k norm + RoPE epilogue on the half tiles that end a tile walk
+    (270 tiles: the last 14 as 28), with narrow tiles off."""
+    monkeypatch.setenv("QW_GEMM_HALF_SMALL", "0")
+    gpu = qd.Gpu()
+    try:
+        K.test_linear_qknorm_epilogue_bit_identical(gpu, qd, oracle, 11400, False, 11400, 512)
+        assert gpu.route() == "qw_gemm_bf16_store_q:half=28"  # the plain linear it ends with
     finally:
         gpu.close()
 
@@ -108,6 +129,7 @@ def test_wide_split_tiles(qd, oracle, monkeypatch, case):
     gpu = qd.Gpu()
     try:
         K.test_linear_split_tiles(gpu, qd, oracle, *case)
+        assert "_q:split=" in gpu.route()
     finally:
         gpu.close()
 

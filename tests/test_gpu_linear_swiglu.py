@@ -22,9 +22,8 @@ def fused(gpu, qd, out, x, w, rows, k, F, ldc=None, **kw):
     return qd.lib().qw_gpu_linear_swiglu(gpu.h, C.byref(d))
 
 
-# rows, k, F: half tiles and ragged columns; split pieces of small launches;
-# the streaming rows; whole tiles with a split tail; 224-row tiles; the walk
-# with its half-tile tail
+# rows, k, F: narrow tiles of 64, 128 and 192 rows, whole and in pieces, ragged
+# columns; the streaming rows; 256-row tiles above narrow ones, and alone
 CASES = [(9, 64, 64, False), (100, 128, 200, True), (300, 1024, 448, False), (130, 4096, 256, True),
          (3, 256, 72, True), (8, 64, 128, False), (520, 2304, 4096, False), (2100, 64, 4224, True),
          (4119, 64, 3072, False)]
@@ -56,6 +55,45 @@ def test_swiglu_linear_is_linear_then_swiglu(qd, oracle, monkeypatch, rows, k, F
         assert (got[:, F:] == 0x1234).all()
         d = ulp_diff(np.ascontiguousarray(got[:, :F]).ravel(), two.read())
         assert d.max() == 0, (d.max(), np.mean(d != 0))
+    finally:
+        gpu.close()
+
+
+# rows, k, F, narrow tiles allowed, the fused launch's kernels
+ROUTES = [
+    (4100, 256, 3072, True, "qw_gemm_bf16_swiglu_mix:3x224+18x192"),
+    (2300, 256, 9224, True, "qw_gemm_bf16_swiglu_mix:2x256+8x224"),
+    (2820, 64, 3072, False, "qw_gemm_bf16_swiglu_q:half=64"),
+    (300, 4096, 1032, False, "qw_gemm_bf16_swiglu_q:split=2"),
+    (2100, 64, 4224, True, "qw_gemm_bf16_swiglu_n2:from=1792 qw_gemm_bf16_swiglu_q"),
+    (2900, 256, 3328, True, "qw_gemm_bf16_swiglu_n3:from=2304 qw_gemm_bf16_swiglu_q"),
+    (1500, 256, 6664, True, "qw_gemm_bf16_swiglu_n4:from=1024 qw_gemm_bf16_swiglu_q"),
+    (1000, 64, 4096, True, "qw_gemm_bf16_swiglu_n4"),
+    (700, 4096, 1544, True, "qw_gemm_bf16_swiglu_n3:split=2"),
+]
+
+
+@pytest.mark.parametrize("rows,k,F,narrow,route", ROUTES)
+def test_swiglu_linear_each_kernel(qd, monkeypatch, rows, k, F, narrow, route):
+    """The same comparison on each bf16 kernel, by the route that ran: mixed
+    tile heights, the half-tile and the split tail of wide tiles, narrow tiles
+    below wide ones and alone; ragged columns among them."""
+    if not narrow:
+        monkeypatch.setenv("QW_GEMM_HALF_SMALL", "0")
+    gpu = qd.Gpu()
+    try:
+        x, w, b = gpu.new(rows * k, qd.BF16), gpu.new(2 * F * k, qd.BF16), gpu.new(2 * F, qd.BF16)
+        for i, (t, std) in enumerate(((x, 1.0), (w, 1.5 / np.sqrt(k)), (b, 0.2))):
+            gpu.check(qd.lib().qw_gpu_fill_normal_bf16(gpu.h, t.h, 0, t.n, 7, i, std, 0.0), "fill")
+        wide, two = gpu.new(rows * 2 * F, qd.BF16), gpu.new(rows * F, qd.BF16)
+        gpu.linear(wide, x, w, rows, k, 2 * F, bias=b)
+        gpu.check(qd.lib().qw_gpu_swiglu_bf16(gpu.h, two.h, wide.h, rows, F), "swiglu")
+        one = gpu.put(np.full((rows + 1) * F, 0x1234, np.uint16))
+        gpu.check(fused(gpu, qd, one, x, w, rows, k, F, bias=b), "fused")
+        assert gpu.route() == route
+        gpu.submit()
+        got = one.read()
+        assert np.array_equal(got[:rows * F], two.read()) and (got[rows * F:] == 0x1234).all()
     finally:
         gpu.close()
 

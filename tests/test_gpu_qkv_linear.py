@@ -11,12 +11,19 @@ from test_gpu_kernels import synth
 pytestmark = pytest.mark.gpu
 
 
-# narrow tiles in pieces, whole and with a wide part above them; mixed tile
-# heights; int8 widened; a table too short for the fused epilogue
-@pytest.mark.parametrize("rows,k,heads,int8,rope_rows", [
-    (70, 2048, 2, False, 200), (320, 256, 24, True, 320), (4119, 512, 10, False, 4119),
-    (3000, 192, 12, False, 1500), (300, 128, 2, False, 100)])
-def test_qkv_linear_outputs(gpu, qd, oracle, rows, k, heads, int8, rope_rows):
+# narrow tiles in pieces, whole (int8 widened) and below wide ones; 256-row
+# tiles wide and narrow; mixed tile heights of 224 and 192 and of 256 and 224
+# rows; a table too short for the fused epilogue
+@pytest.mark.parametrize("rows,k,heads,int8,rope_rows,route", [
+    (70, 2048, 2, False, 200, "qw_gemm_bf16_qkn_n1:split=3"),
+    (320, 256, 24, True, 320, "qw_gemm_bf16_qkn_n2"),
+    (11400, 512, 4, False, 5700, "qw_gemm_bf16_qkn_n1:from=10752 qw_gemm_bf16_qkn_q"),
+    (4119, 512, 10, False, 4119, "qw_gemm_bf16_qkn_q"),
+    (3000, 192, 12, False, 1500, "qw_gemm_bf16_qkn_n4"),
+    (4100, 192, 16, False, 4100, "qw_gemm_bf16_qkn_mix:3x224+18x192"),
+    (2300, 256, 48, True, 1150, "qw_gemm_bf16_qkn_mix:2x256+8x224"),
+    (300, 128, 2, False, 100, "qw_gemm_bf16_store_n1")])
+def test_qkv_linear_outputs(gpu, qd, oracle, rows, k, heads, int8, rope_rows, route):
     H = heads * 128
     n = 3 * H
     x = gpu.put(synth(oracle, rows * k, 91))
@@ -37,6 +44,7 @@ def test_qkv_linear_outputs(gpu, qd, oracle, rows, k, heads, int8, rope_rows):
     d = qd.LinearDesc(out.h, 0, n, x.h, 0, k, w.h, s.h if s else None, None, rows, k, n,
                       qd.LINEAR_QKNORM, None, None, 0, 0, nq.h, nk.h, ct.h, st.h, rope_rows, 1e-6)
     gpu.check(qd.lib().qw_gpu_qkv_linear(gpu.h, C.byref(d), kt.h, vt.h, at), "qkv")
+    assert gpu.route() == route
     gpu.submit()
     want = ref.read().reshape(rows, 3, H)
     assert np.array_equal(out.read().reshape(rows, 3, H)[:, 0], want[:, 0])
