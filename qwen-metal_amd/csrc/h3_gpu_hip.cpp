@@ -1051,9 +1051,7 @@ extern "C" int qw_gpu_widen_int8_bf16(h3_gpu *g, h3_gpu_tensor *out, const h3_gp
  * R s <= QW_SPLIT_MAX_PIECES * cus bounds the partial workspace. */
 #define QW_SPLIT_MAX_PIECES 2
 static uint32_t split_choice(h3_gpu *g, uint32_t tiles, uint32_t ksteps,
-                             uint64_t max_pieces = (uint64_t)QW_SPLIT_MAX_PIECES * 1024u,
-                             uint32_t min_steps = 0) {
-    if (!min_steps) min_steps = g->split_min_steps;
+                             uint64_t max_pieces = (uint64_t)QW_SPLIT_MAX_PIECES * 1024u) {
     const uint32_t G = g->cus, R = tiles % G;
     if (R == 0) return 1; /* every wave is full: nothing to split */
     if (g->split_force > 1 && (uint64_t)R * g->split_force <= (uint64_t)QW_SPLIT_MAX_PIECES * G &&
@@ -1063,7 +1061,7 @@ static uint32_t split_choice(h3_gpu *g, uint32_t tiles, uint32_t ksteps,
     double best_t = 0.9;
     for (uint32_t s = 2; s <= 8; s++) {
         if ((uint64_t)R * s > (uint64_t)QW_SPLIT_MAX_PIECES * G || (uint64_t)R * s > max_pieces ||
-            ksteps < min_steps * s)
+            ksteps < g->split_min_steps * s)
             break;
         const double t = (double)((R * s + G - 1) / G) / s + 0.02 * (s - 1);
         if (t < best_t) {
