@@ -42,30 +42,18 @@ PEAK_HBM_GBS = 8000.0
 CFG = dict(hidden=3072, heads=24, mlp_width=12288, text_dim=4096, z_dim=64, layers=32,
            mlp_act=1, adaln_shift=1, has_bias=1, text_causal=0, int8_weights=1)
 TEXT, GH, GW, BATCH, SIGMA, SEED = 256, 64, 64, 2, 0.5, 2026
-W8_MIN_K = 8192  # int8 linears with K >= this may widen in LDS inside the GEMM ("_w8")
 
 
-def int8_in_lds(M, K, N, cus=256):
-    """The library's automatic int8 route for an M-row linear (linear_impl
-    in h3_gpu_hip.cpp): True where the "_w8" kernels widen the weight in LDS
-    inside the GEMM, False where a widening pass runs ahead of the bf16
-    kernels (or, for at most 8 rows, the GEMV kernels widen in registers).
-    A launch of at most cus / 2 tiles widens by a pass; a larger one of
-    fewer than 512 rows stays on "_w8"; from 512 rows "_w8" needs K >= 8192
-    and a shape on which the bf16 kernels would not take lower tiles (told
-    here by 224-row ones, which settles it at this workload's shapes)."""
-    tn = (N + 255) // 256
-    tiles = (M + 255) // 256 * tn
-    if M <= 8 or 2 * tiles <= cus:
-        return False
-    if M < 512:
-        return True
-    if K < W8_MIN_K:
-        return False
-    r = tiles % cus
-    w256 = tiles // cus + ((0.5 if 2 * r <= cus else 1.0) if r else 0.0)
-    w224 = 0.875 * (((M + 223) // 224 * tn + cus - 1) // cus)
-    return not w224 < 0.97 * w256
+def int8_in_lds(qd, gpu, M, K, N):
+    """The library's own int8 route for an M-row linear, from the kernels that
+    one call on zeros launches: True where a "_w8" kernel widens the weight in
+    LDS inside the GEMM, False where a widening pass runs ahead of the bf16
+    kernels (or, for at most 8 rows, the GEMV kernels widen in registers)."""
+    out, a, q, s = (gpu.new(n, t) for n, t in ((M * N, qd.BF16), (M * K, qd.BF16), (N * K, qd.I8),
+                                               (N, qd.F32)))
+    gpu.linear(out, a, q, M, K, N, wscale=s)
+    gpu.submit()
+    return "_w8_" in gpu.route()
 
 
 def load_qdit():
@@ -133,7 +121,7 @@ def kernel_breakdown(qd, gpu, reps=10):
         gemm = lambda: gpu.linear(big, a, wb, M, k, n, wscale=s, epilogue=epi, **kw)  # noqa
         full()
         ms = time_ms(gpu, full, reps)
-        in_gemm = int8_in_lds(M, k, n)  # the library's int8 route at these rows
+        in_gemm = "_w8_" in gpu.route()  # the library's int8 route at these rows
         if in_gemm:
             gemm_ms, widen_ms = ms, 0.0
         else:
@@ -682,7 +670,7 @@ def main():
                     "kernel": ("qw_gemm_w8_gate_q (down projection, M=8704 K=12288 N=3072, "
                                "int8 weight widened to bf16 in LDS once per workgroup, scale "
                                "and residual gate in the epilogue)"
-                               if int8_in_lds(down["M"], down["K"], down["N"]) else
+                               if int8_in_lds(qd, gpu, down["M"], down["K"], down["N"]) else
                                "qw_widen_i8_bf16 + qw_gemm_bf16_gate_mix (down projection, "
                                "M=8704 K=12288 N=3072: the int8 weight widened to bf16 by a "
                                "pass, then 224- and 192-row tiles in 2 rounds, scale and residual "

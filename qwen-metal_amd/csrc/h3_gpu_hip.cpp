@@ -59,18 +59,14 @@ static const char *k_names[K_COUNT] = {
     "qw_cond_l1", "qw_cond_l2", "qw_cond_mod", "qw_layer_norm_mod_shift_bf16",
     "qw_layer_norm_mod_3072_bf16", "qw_layer_norm_mod_3072_shift_bf16"};
 
-/* How int8 linears run (QW_INT8_ROUTE, a measurement switch): AUTO (the
- * default) widens the weight to a bf16 copy and runs the bf16 kernels when
- * that measured faster -- 512+ rows and K < 8192 -- and otherwise runs the
- * int8 kernels that widen each W tile once per workgroup in LDS; WIDEN and
+/* How int8 linears of more than 8 rows run (QW_INT8_ROUTE, a measurement
+ * switch): AUTO (the default) widens the weight to a bf16 copy by a pass and
+ * runs the bf16 kernels, or runs the int8 kernels that widen each W tile once
+ * per workgroup in LDS, whichever w8_faster expects to be faster; WIDEN and
  * W8 force one route wherever it can run. */
 enum { QW_INT8_AUTO = 0, QW_INT8_WIDEN = 1, QW_INT8_W8 = 2 };
 
 #define QW_SPAN_MAX 4096
-
-/* below this many rows an int8 linear widens inside its GEMM, unless the
- * launch is small enough for narrow tiles (linear_impl) */
-#define QW_WIDEN_MIN_ROWS 512
 
 struct h3_gpu {
     int device;
@@ -91,7 +87,6 @@ struct h3_gpu {
     int int8_route; /* QW_INT8_* : how int8 linears of many rows run */
     int mixed;      /* 192- and 224-row tiles allowed (QW_GEMM_T224=0 turns them off, for measurement) */
     uint32_t split_min_steps, split_force; /* measurement: QW_SPLIT_MIN_STEPS, QW_SPLIT_FORCE */
-    uint32_t widen_min_rows; /* int8: fewest rows for the widening route (QW_WIDEN_MIN_ROWS) */
     int workspaces; /* split partials and widened copies allowed (QW_WORKSPACES=0: as if none could be had) */
     int narrow;     /* narrow tiles allowed (QW_GEMM_HALF_SMALL=0: off) */
     /* qw_gpu_last_route: the launches of the last linear or attention call */
@@ -216,8 +211,6 @@ extern "C" h3_gpu *h3_gpu_create(const char *code_object_path, char *error,
     if (const char *r = getenv("QW_SPLIT_MIN_STEPS")) g->split_min_steps = (uint32_t)atoi(r);
     g->split_force = 0;
     if (const char *r = getenv("QW_SPLIT_FORCE")) g->split_force = (uint32_t)atoi(r);
-    g->widen_min_rows = QW_WIDEN_MIN_ROWS;
-    if (const char *r = getenv("QW_WIDEN_MIN_ROWS")) g->widen_min_rows = (uint32_t)atoi(r);
     g->workspaces = 1;
     if (const char *r = getenv("QW_WORKSPACES")) g->workspaces = atoi(r) != 0;
     g->narrow = 1;
@@ -1087,15 +1080,20 @@ struct wide_plan {
     double us;
     uint32_t h1, h2, rows1, rows2;
 };
-static wide_plan plan_wide(h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t ksteps) {
-    const uint32_t C = g->cus, tn = (cols + 255) / 256, tiles = (rows + 255) / 256 * tn;
-    const double step = 1.3 * ksteps, fix = 12.0, round = step + fix;
+/* 256-row tiles in rounds of `round` us; half: the share of a round that a
+ * last one on half tiles takes */
+static double wide_us(h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t ksteps, double round,
+                      double half) {
+    const uint32_t C = g->cus, tiles = (rows + 255) / 256 * ((cols + 255) / 256);
     const uint32_t R = tiles % C, s = split_choice(g, tiles, ksteps);
-    wide_plan p = {(double)(tiles / C) * round, 0, 0, 0, 0};
-    if (s > 1)
-        p.us += (double)((R * s + C - 1) / C) / s * round + 8.0 + 0.055 * R * s * s;
-    else if (R)
-        p.us += tiles > C && 2 * R <= C ? 0.6 * round : round;
+    const double us = (double)(tiles / C) * round;
+    if (s > 1) return us + (double)((R * s + C - 1) / C) / s * round + 8.0 + 0.055 * R * s * s;
+    return us + (!R ? 0.0 : tiles > C && 2 * R <= C ? half * round : round);
+}
+static wide_plan plan_wide(h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t ksteps) {
+    const uint32_t C = g->cus, tn = (cols + 255) / 256;
+    const double step = 1.3 * ksteps, fix = 12.0;
+    wide_plan p = {wide_us(g, rows, cols, ksteps, step + fix, 0.6), 0, 0, 0, 0};
     if (!g->mixed || C % 8) return p;
     const uint32_t m32 = (rows + 31) / 32;
     double best = 0.98 * p.us;
@@ -1196,30 +1194,49 @@ static int split_workspace(h3_gpu *g) {
 struct linear_plan {
     uint32_t wide, mb, s;
     wide_plan w; /* how the first run */
+    double us;
 };
 static linear_plan plan_linear(h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t ksteps,
                                uint32_t max_s) {
-    linear_plan p = {rows, 0, 1, plan_wide(g, rows, cols, ksteps)};
+    linear_plan p = {rows, 0, 1, plan_wide(g, rows, cols, ksteps), 0.0};
+    p.us = p.w.us;
     if (!g->narrow) return p;
     uint32_t mb, s;
-    double best = p.w.us;
     const double all = narrow_us(g, rows, cols, ksteps, max_s, &mb, &s);
-    if (all < 0.98 * best) {
-        best = all;
-        p = {0, mb, s, p.w};
-    }
+    if (all < 0.98 * p.us) p = {0, mb, s, p.w, all};
     /* the last, ragged tile row on narrow tiles, or up to three more with it */
     for (uint32_t j = 0; j < 4; j++) {
         const uint32_t rem = rows % 256 + 256 * j;
         if (!rem || rows < rem + 256) continue;
         const wide_plan w = plan_wide(g, rows - rem, cols, ksteps);
         const double t = w.us + narrow_us(g, rem, cols, ksteps, max_s, &mb, &s);
-        if (t < 0.97 * best) {
-            best = t;
-            p = {rows - rem, mb, s, w};
-        }
+        if (t < 0.97 * p.us) p = {rows - rem, mb, s, w, t};
     }
     return p;
+}
+
+/* Whether an int8 linear is faster on the "_w8" kernels, which widen inside
+ * (256-row tiles whose round takes 1.45 us a k-step and 7 us, no half tiles),
+ * than as a pass that widens its weight (3 bytes an element at 6.2 TB/s, 2.5
+ * us more) and the bf16 kernels of plan p. Fewer than 512 rows that no narrow
+ * tiles suit, and long K on whole tiles of 256 rows, run there in any case;
+ * else the times decide, at K from 3072 (where the bf16 tiles' are fitted) or
+ * within a round of tiles.
+ *
+ * Against the faster of the two, at 430 shapes of 16 to 8704 rows with weights
+ * that are in no cache, the choice costs 0.2% on average at K >= 3072 and 1.4%
+ * over all. Where the sides meet, us (pass / _w8): 24576 x 4096 at 200 rows
+ * 122 / 76, at 700 208 / 156, at 1752 293 / 294, at 4119 629 / 680; 12288 x
+ * 4096 at 700 rows 88 / 88, at 1152 113 / 101, at 1400 137 / 155; 3072 x
+ * 12288 at 64 rows 40 / 77, at 1400 130 / 121, at 3000 196 / 237, at 8704 499
+ * / 549; 3072 x 3072 at 16 to 8704 rows 21-125 / 63-149. */
+static bool w8_faster(h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t ksteps,
+                      const linear_plan &p, bool low_tiles) {
+    if (!p.mb && (rows < 512 || (ksteps >= 128 && !low_tiles))) return true;
+    const uint64_t tiles = (uint64_t)((rows + 255) / 256) * ((cols + 255) / 256);
+    if (ksteps < 48 && tiles > g->cus) return false;
+    const double pass = 2.5 + 192.0 * cols * ksteps / 6.2e6;
+    return wide_us(g, rows, cols, ksteps, 1.45 * ksteps + 7.0, 1.0) < 0.94 * (pass + p.us);
 }
 
 /* the widened copy of an int8 weight, grown to `bytes`; 0 where it cannot be
@@ -1348,40 +1365,20 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc,
         return launch_step(g, kid, dim3((waves + 3) / 4), dim3(256), a, 1);
     }
     /* int8 weights: the "_w8" kernels widen each int8 W tile once per
-     * workgroup into the bf16 W stage in LDS (no copy through HBM, half
-     * the weight bytes). Where it measured faster -- 512+ rows and K <
-     * 8192 -- the weight is instead widened to a bf16 copy by one
-     * bandwidth-bound pass and the bf16 kernels run; both routes give the
-     * same bits (the per-row scale multiplies the finished fp32 sums). Same
-     * box, alternating, M = 8704, us (widening pass + bf16 kernel / w8):
-     * QKV 378-387 / 391-406, out 140-145 / 145-151, up 485-504 / 530-565,
-     * down 558-571 / 558-573; steps 66.30-66.49 ms with every int8 linear
-     * widened, 68.11-68.24 with every one on w8, 66.32-66.47 with w8 on the
-     * down projection only. The w8 kernels' extra cost is the widening's
-     * VALU work (1.5 instructions per weight per workgroup): the same
-     * kernel with the conversion left out runs as fast as the widening
-     * pass plus the bf16 kernel. */
-    const linear_plan wide_all = {d->rows, 0, 1, plan_wide(g, d->rows, d->cols, d->k / 64)};
+     * workgroup into the bf16 W stage in LDS (no copy through HBM, half the
+     * weight bytes; 1.5 VALU instructions per weight per workgroup), or one
+     * bandwidth-bound pass widens the weight to a bf16 copy for the bf16
+     * kernels. Both give the same bits where the sums' pieces are the same
+     * (the per-row scale multiplies the finished fp32 sums). */
+    const linear_plan wide_all = {d->rows, 0, 1, plan_wide(g, d->rows, d->cols, d->k / 64), 0.0};
     linear_plan plan = no_alloc || (int8 && g->int8_route == QW_INT8_W8)
                            ? wide_all : plan_linear(g, d->rows, d->cols, d->k / 64, 8);
-    /* K >= 8192 keeps the in-LDS widening, unless the widened weight's bf16
-     * kernel takes lower tiles (224-row ones for the down projection at M = 8704: whole
-     * steps 64.07 against 65.39 ms with the pass and 224-row tiles, medians
-     * of 8, same box, alternating) */
-    int route = g->int8_route;
-    if (route == QW_INT8_AUTO)
-        route = d->k >= 8192 && !wide_all.w.h1 ? QW_INT8_W8 : QW_INT8_WIDEN;
-    /* Where the bf16 kernels take narrow tiles, for all rows or for the last
-     * few, the weight is widened by a pass at any row count and K: they beat
-     * the whole "_w8" tiles by more than the pass costs (M = 64-448, us, w8 /
-     * pass + 128 x 256 half tiles, which narrow tiles beat in turn: QKV
-     * 64-66 / 48-55, out 63 / 35-38, up 65-67 / 56-59, down 74-84 / 66-76). */
-    const int small_w = g->int8_route == QW_INT8_AUTO && plan.mb != 0;
-    if (small_w) route = QW_INT8_WIDEN;
     const size_t weights = (size_t)d->cols * d->k;
     g->route_n = 0;
-    const int widen = int8 && !no_alloc && (d->rows >= g->widen_min_rows || small_w) &&
-                      route == QW_INT8_WIDEN && weights * 2 < (1ull << 31) /* a buffer's range */ &&
+    const int widen = int8 && !no_alloc && g->int8_route != QW_INT8_W8 &&
+                      (g->int8_route == QW_INT8_WIDEN ||
+                       !w8_faster(g, d->rows, d->cols, d->k / 64, plan, wide_all.w.h1)) &&
+                      weights * 2 < (1ull << 31) /* a buffer's range */ &&
                       widen_workspace(g, weights * 2);
     if (int8 && !widen) plan = wide_all;
     if (plan.s > 1 && !split_workspace(g))
