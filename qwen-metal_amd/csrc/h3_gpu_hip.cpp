@@ -1173,7 +1173,7 @@ static int split_workspace(h3_gpu *g) {
     const size_t flags = (size_t)g->cus * QW_FLAGS * 4;
     if (hipMalloc((void **)&g->sk_part, n) == hipSuccess) {
         if (hipMalloc((void **)&g->sk_flag, flags) == hipSuccess &&
-            hipMemset(g->sk_flag, 0, flags) == hipSuccess) {
+            hipMemsetAsync(g->sk_flag, 0, flags, g->stream) == hipSuccess) {
             g->stats.allocated_bytes += n + flags;
             return 1;
         }
