@@ -130,7 +130,8 @@ int qw_gpu_linear(h3_gpu *gpu, const qw_linear_desc *desc);
  * [2F, k] = [gate | up] rows, cols = 2F (a multiple of 16), out [rows, F] at
  * stride ldc >= F: bf16(bf16(silu(g)) * u) with g, u the linear's bf16
  * results, as qw_gpu_linear followed by qw_gpu_swiglu_bf16. epilogue must be
- * QW_LINEAR_STORE. No counterpart in the reference, which runs two kernels. */
+ * QW_LINEAR_STORE, and out clear of in. No counterpart in the reference, which
+ * runs two kernels. */
 int qw_gpu_linear_swiglu(h3_gpu *gpu, const qw_linear_desc *desc);
 /* The QKNORM linear with the k and v thirds of its output (after the norm and
  * the rotation) in tensors of their own, rows [rows, cols / 3] at kv_offset

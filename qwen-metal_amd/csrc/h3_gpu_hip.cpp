@@ -623,6 +623,11 @@ static bool fits(const h3_gpu_tensor *t, size_t offset, size_t elements) {
     return t && offset + elements <= t->elements;
 }
 
+static bool apart(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return x + a_bytes <= y || y + b_bytes <= x;
+}
+
 static uint32_t blocks_for(uint64_t n, uint32_t per) { return (uint32_t)((n + per - 1) / per); }
 
 static int ln_mod(h3_gpu *g, h3_gpu_tensor *out, const h3_gpu_tensor *in,
@@ -1578,16 +1583,15 @@ extern "C" int qw_gpu_qkv_linear(h3_gpu *g, const qw_linear_desc *d, h3_gpu_tens
      * would take less, but what is accepted does not depend on the table. */
     const uintptr_t kp = (uintptr_t)k->ptr + kv_offset * 2, vp = (uintptr_t)v->ptr + kv_offset * 2;
     if ((kp | vp) % 16) return fail(g, "qkv_linear: k and v must be 16-byte aligned");
-    auto apart = [&](uintptr_t p, const h3_gpu_tensor *t, size_t off, size_t elements) {
-        const uintptr_t b = t ? (uintptr_t)t->ptr + off * 2 : 0;
-        return p + n * 2 <= b || b + elements * 2 <= p;
+    auto clear_of = [&](uintptr_t p, const h3_gpu_tensor *t, size_t off, size_t elements) {
+        return !t || apart((const void *)p, n * 2, t->ptr + off * 2, elements * 2);
     };
     const size_t in_n = (size_t)(d->rows - 1) * d->lda + d->k;
     const size_t out_n = (size_t)(d->rows - 1) * d->ldc + d->cols;
     for (uintptr_t p : {kp, vp})
-        if (!apart(p, d->in, d->in_offset, in_n) || !apart(p, d->out, d->out_offset, out_n))
+        if (!clear_of(p, d->in, d->in_offset, in_n) || !clear_of(p, d->out, d->out_offset, out_n))
             return fail(g, "qkv_linear: k or v overlaps the input or the output");
-    if (!apart(kp, v, kv_offset, n)) return fail(g, "qkv_linear: k and v overlap");
+    if (!clear_of(kp, v, kv_offset, n)) return fail(g, "qkv_linear: k and v overlap");
     if (d->rope_rows < 128 || n * 2 >= (1ull << 31))
         return linear_impl(g, d, 0) &&
                qw_gpu_copy_rows(g, k, kv_offset, H, d->out, H, d->ldc, d->rows, H) &&
@@ -1604,6 +1608,10 @@ extern "C" int qw_gpu_linear_swiglu(h3_gpu *g, const qw_linear_desc *d) {
     if (!g || !d) return 0;
     if (!check_epilogue(g, d)) return 0;
     if (d->epilogue != QW_LINEAR_STORE) return fail(g, "linear_swiglu: epilogue must be STORE");
+    if (d->rows && d->in && d->out && d->in->dtype == H3_GPU_BF16 && d->out->dtype == H3_GPU_BF16 &&
+        !apart(d->in->ptr + d->in_offset * 2, ((size_t)(d->rows - 1) * d->lda + d->k) * 2,
+               d->out->ptr + d->out_offset * 2, ((size_t)(d->rows - 1) * d->ldc + d->cols / 2) * 2))
+        return fail(g, "linear_swiglu: the output overlaps the input");
     qw_linear_desc t = *d;
     if (d->rows > 8 || d->cols % 16 || d->ldc != d->cols / 2 || d->out_offset) {
         t.epilogue = QW_EPI_SWIGLU;

@@ -177,6 +177,11 @@ def test_swiglu_linear_refusals(gpu, qd):
     assert not fused(gpu, qd, out, x, w, rows, k, F, epilogue=4)
     assert not fused(gpu, qd, out, x, w, 4, k, F, ldc=F - 8)
     assert not fused(gpu, qd, out, x, w, rows, k, F, ldc=F + 8)  # past the output's end
+    for n in (4, rows):  # over the input, or its last elements, at any row count
+        assert not fused(gpu, qd, x, x, w, n, k, F)
+        both = gpu.new(2 * n * k, qd.BF16)
+        assert not fused(gpu, qd, both.view(n * k - 4, n * F), both, w, n, k, F)
+        assert fused(gpu, qd, both.view(n * k, n * F), both, w, n, k, F)
     d = qd.LinearDesc(out.h, 0, F, x.h, 0, k, w.h, None, None, rows, k, F, 4, None, None, 0, 0,
                       None, None, None, None, 0, 0.0)
     assert not qd.lib().qw_gpu_linear(gpu.h, C.byref(d))  # not an epilogue of qw_gpu_linear
