@@ -224,8 +224,9 @@ int qw_gpu_modulation_reorder_bf16(h3_gpu *gpu, h3_gpu_tensor *slots_out,
  * mod(silu(temb)) as qw_gpu_modulation_reorder_bf16 leaves it, norm_out_scale
  * = norm_out(silu(temb)). Weights bf16 [n, k]; biases may be NULL; wide and
  * silu are scratch, bf16 [rows, hidden]. The results are those of the
- * separate linears and activations, bit for bit. No counterpart in the
- * reference. */
+ * separate linears and activations, bit for bit. A linear's output may not
+ * overlap its input, nor silu temb (else the call is refused). No counterpart
+ * in the reference. */
 typedef struct {
     const h3_gpu_tensor *features; /* f32 [rows, 256] */
     const h3_gpu_tensor *l1, *l1_bias, *l2, *l2_bias, *mod, *mod_bias, *norm_out, *norm_out_bias;

@@ -908,6 +908,15 @@ extern "C" int qw_gpu_conditioning_bf16(h3_gpu *g, const qw_conditioning_desc *d
         if (!x.t || x.t->dtype != x.type) return fail(g, "conditioning: missing tensor or wrong dtype");
         if (!fits(x.t, 0, x.n)) return fail(g, "conditioning: tensor too small");
     }
+    /* within a launch, workgroups read and write in any order */
+    const size_t R = (size_t)rows * 2;
+    const struct { const h3_gpu_tensor *a; size_t an; const h3_gpu_tensor *b; size_t bn; } clear[] = {
+        {d->features, (size_t)rows * 256 * 4, d->wide, R * H}, {d->wide, R * H, d->temb, R * H},
+        {d->wide, R * H, d->silu, R * H},                      {d->temb, R * H, d->silu, R * H},
+        {d->silu, R * H, d->modulation, R * S * H},            {d->silu, R * H, d->norm_out_scale, R * nout}};
+    for (const auto &c : clear)
+        if (!apart(c.a->ptr, c.an, c.b->ptr, c.bn))
+            return fail(g, "conditioning: a stage's output overlaps its input or its other output");
     /* the operands that are read 16 bytes at a time */
     for (const h3_gpu_tensor *t : {d->l1, d->l2, d->mod, d->norm_out,
                                    (const h3_gpu_tensor *)d->wide, (const h3_gpu_tensor *)d->silu})
@@ -942,6 +951,13 @@ extern "C" int qw_gpu_conditioning_bf16(h3_gpu *g, const qw_conditioning_desc *d
     a.bias2 = bias(d->norm_out_bias);
     a.out2 = (uint16_t *)d->norm_out_scale->ptr;
     a.n2 = nout;
+    if (!apart(a.out, R * a.n, a.out2, R * a.n2)) {
+        /* one over the other: the modulation stands, as from separate linears */
+        qw_cond_args first = a;
+        first.n = 0;
+        if (!launch(g, K_COND_MOD, grid(nout), dim3(256), first)) return 0;
+        a.n2 = 0;
+    }
     return launch(g, K_COND_MOD, grid(a.n + a.n2), dim3(256), a);
 }
 

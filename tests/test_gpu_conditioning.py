@@ -58,3 +58,38 @@ def test_conditioning_refusals(gpu, qd):
     assert not ok(shift=1)  # six slots do not fit
     assert not ok(hidden=257) and not ok(hidden=512)
     gpu.submit()
+
+
+def test_conditioning_overlaps(gpu, qd, oracle):
+    """A stage whose output lies over its input, or silu over temb, is
+    refused; the modulation over the final norm's factor leaves what separate
+    linears do: the modulation whole, after the factor."""
+    H, rows, L = 256, 2, qd.lib()
+    put = lambda n, s: gpu.put(oracle.fill_normal_bf16(n, 31, s, 0.1))  # noqa: E731
+    f = gpu.put(np.random.default_rng(3).uniform(-1, 1, rows * 256).astype(np.float32))
+    w = [put(n, i) for i, n in enumerate((H * 256, H * H, 4 * H * H, H * H))]
+    names = ("wide", "silu", "temb", "modulation", "norm_out")
+    size = dict(zip(names, (rows * H, rows * H, rows * H, 4 * rows * H, rows * H)))
+
+    def call(**views):
+        o = {n: views.get(n) or gpu.new(size[n], qd.BF16) for n in names}
+        d = qd.ConditioningDesc(f.h, w[0].h, None, w[1].h, None, w[2].h, None, w[3].h, None,
+                                *(o[n].h for n in names), rows, H, 0)
+        ok = L.qw_gpu_conditioning_bf16(gpu.h, C.byref(d))
+        gpu.submit()
+        return {n: t.read() for n, t in o.items()} if ok else None
+
+    ref = call()
+    buf = gpu.new(8 * rows * H, qd.BF16)
+    for a, b in (("wide", "temb"), ("wide", "silu"), ("temb", "silu"), ("silu", "modulation"),
+                 ("silu", "norm_out")):
+        for off in (0, size[a] - 8):
+            assert call(**{a: buf.view(0, size[a]), b: buf.view(off, size[b])}) is None
+        assert call(**{a: buf.view(0, size[a]), b: buf.view(size[a], size[b])}) is not None
+    for off in (0, 3 * rows * H + 8):
+        got = call(modulation=buf.view(0, size["modulation"]), norm_out=buf.view(off, size["norm_out"]))
+        assert np.array_equal(got["modulation"], ref["modulation"])
+        assert np.array_equal(got["temb"], ref["temb"])
+        tail = max(0, off + size["norm_out"] - size["modulation"])
+        if tail:
+            assert np.array_equal(got["norm_out"][-tail:], ref["norm_out"][-tail:])
