@@ -132,7 +132,7 @@ def test_linear_store(gpu, qd, oracle, rows, k, n, bias, int8):
 def test_linear_int8_in_lds_route(qd, oracle, monkeypatch, rows, k, n, bias):
     """The "_w8" kernels (int8 W widened in LDS inside the GEMM) on the int8
     cases, forced by QW_INT8_ROUTE=w8: by default these small launches widen
-    by a pass and run the bf16 half tiles instead."""
+    by a pass and run narrow bf16 tiles instead."""
     monkeypatch.setenv("QW_INT8_ROUTE", "w8")
     gpu = qd.Gpu()
     try:
@@ -280,14 +280,13 @@ def test_linear_split_tiles(gpu, qd, oracle, rows, k, n, int8, epi):
 @pytest.mark.parametrize("rows,k,n,epi", [(300, 3072, 1024, "gelu"), (1100, 12288, 768, "gate"),
                                           (2000, 8192, 2000, "store")])
 def test_int8_in_gemm_widening_bit_identical(qd, oracle, monkeypatch, rows, k, n, epi):
-    """The int8 kernels that widen each W tile once per workgroup in LDS
-    (taken below 512 rows and for K >= 8192) give the same bits as widening
-    the weight to a bf16 copy (qw_gpu_widen_int8_bf16) and running the bf16
-    kernel with the same row scales: the widening is exact and the scale
-    multiplies the finished fp32 sums in both. Split tiles included
-    (K = 8192 and 12288). Same k-ranges on both sides: the bf16 kernels'
-    half tiles for small launches (which may split K differently) are
-    turned off for this context."""
+    """The int8 kernels that widen each W tile once per workgroup in LDS give
+    the same bits as widening the weight to a bf16 copy
+    (qw_gpu_widen_int8_bf16) and running the bf16 kernel with the same row
+    scales: the widening is exact and the scale multiplies the finished fp32
+    sums in both. Split tiles included (K = 8192 and 12288). Same k-ranges on
+    both sides: the bf16 kernels' narrow tiles (which may split K
+    differently) are turned off for this context."""
     monkeypatch.setenv("QW_GEMM_HALF_SMALL", "0")
     gpu = qd.Gpu()
     try:
@@ -355,11 +354,11 @@ def test_linear_full_waves_never_split(qd, oracle):
                                         (8604, 256, "gate"), (4315, 512, "qkn")])
 def test_linear_224_row_tiles(gpu, qd, oracle, rows, k, epi):
     """Shapes whose 256 x 256 tiling leaves a partly filled last wave that
-    224 x 256 tiles avoid (on 256 CUs: 204 tiles of 256 rows, 1 wave, become
-    240 of 224 rows; 408 tiles, 2 waves, become 468 in 2 waves of 0.875 the
-    work): ragged rows through all four epilogues, against the oracle, and
-    the fused q/k norm + RoPE bit for bit against the plain linear followed
-    by the standalone kernel."""
+    lower tiles avoid (on 256 CUs: 204 tiles of 256 rows, 1 wave, become 240
+    of 224 rows; 408 tiles, 2 waves, 204 of 224 and 300 of 192): ragged rows
+    through all four epilogues, against the oracle, and the fused q/k norm +
+    RoPE bit for bit against the plain linear followed by the standalone
+    kernel."""
     n = 3072
     x = synth(oracle, rows * k, 71)
     w = synth(oracle, n * k, 72, 0.02)
@@ -422,10 +421,9 @@ def test_linear_224_row_tiles(gpu, qd, oracle, rows, k, epi):
 
 @pytest.mark.parametrize("n,int8", [(1800, False), (1784, True)])
 def test_linear_224_row_tiles_ragged_cols(gpu, qd, oracle, n, int8):
-    """224-row tiles with a partial last tile column (N not a multiple of
-    256): 17 x 8 = 136 tiles of 256 rows (one wave, more than half full)
-    become 20 x 8 = 160 of 224 rows; int8 weights take the widening pass
-    (K < 8192, 512+ rows) into the same kernel."""
+    """A partial last tile column (N not a multiple of 256) at 17 x 8 = 136
+    tiles of 256 rows (one wave, more than half full), which lower or narrow
+    tiles replace; int8 weights widened by a pass into the same kernel."""
     rows, k = 4315, 512
     x = synth(oracle, rows * k, 81)
     w = synth(oracle, n * k, 82, 0.02)
@@ -451,9 +449,10 @@ def test_linear_tile_walk(gpu, qd, oracle, epi):
     workgroup per CU and each walks its tiles in strides of the grid. 17 x
     17 tiles of 256 x 256 (289 > 256), ragged in both the last tile row
     (4100 rows) and the last tile column (4104 columns), called twice in a
-    row (the workgroups keep no state between tiles or calls). The 33 tiles
-    of the last, partly filled wave run as 66 half tiles of 128 x 256; the
-    last tile row's second halves hold no rows at all."""
+    row (the workgroups keep no state between tiles or calls). With narrow
+    tiles off (test_wide_tile_walk) the 33 tiles of the last, partly filled
+    wave run as 66 half tiles of 128 x 256, the last tile row's second halves
+    without any row; else the last 260 rows run on narrow tiles."""
     rows, k, n = 4100, 256, 4104
     x = synth(oracle, rows * k, 41)
     w = synth(oracle, n * k, 42, 0.02)
@@ -513,11 +512,10 @@ def test_linear_tile_walk(gpu, qd, oracle, epi):
                                                    # tables under 128 rows: the plain
                                                    # linear, then the standalone kernel
                                                    (300, False, 100, 512), (300, True, 64, 512),
-                                                   # 270 tiles: a tile walk whose last 14
-                                                   # tiles run as half tiles
+                                                   # 10752 rows on whole tiles, the last
+                                                   # 648 on narrow ones
                                                    (11400, False, 11400, 512),
-                                                   # a small launch's half tiles in 3
-                                                   # k-range pieces
+                                                   # narrow tiles in k-range pieces
                                                    (300, False, 300, 3072),
                                                    (600, True, 600, 3072)])
 def test_linear_qknorm_epilogue_bit_identical(gpu, qd, oracle, rows, int8, rope_rows, k):

@@ -109,6 +109,19 @@ def test_wide_low_tiles(qd, oracle, monkeypatch, n, int8, tiles):
         gpu.close()
 
 
+@pytest.mark.parametrize("epi", ["store", "gelu", "gate"])
+def test_wide_tile_walk(qd, oracle, monkeypatch, epi):
+    """test_linear_tile_walk with narrow tiles off: the last 33 of its 289
+    tiles run as 66 half tiles."""
+    monkeypatch.setenv("QW_GEMM_HALF_SMALL", "0")
+    gpu = qd.Gpu()
+    try:
+        K.test_linear_tile_walk(gpu, qd, oracle, epi)
+        assert gpu.route() == f"qw_gemm_bf16_{epi}_q:half=66"
+    finally:
+        gpu.close()
+
+
 def test_wide_half_tiles_qknorm(qd, oracle, monkeypatch):
     """The q/k norm + RoPE epilogue on the half tiles that end a tile walk
     (270 tiles: the last 14 as 28), with narrow tiles off."""
