@@ -34,7 +34,8 @@ enum {
     /* narrow tiles of 64, 128, 192 and 256 rows, each in the same order */
     K_GEMM_N1, K_GEMM_N1_LAST = K_GEMM_N1 + 4, K_GEMM_N2, K_GEMM_N2_LAST = K_GEMM_N2 + 4,
     K_GEMM_N3, K_GEMM_N3_LAST = K_GEMM_N3 + 4, K_GEMM_N4, K_GEMM_N4_LAST = K_GEMM_N4 + 4,
-    K_ATTN_W4, K_ATTN_SPLIT, K_ATTN_W4_SPLIT, K_COND_L1, K_COND_L2, K_COND_MOD, /* with and without shift, width up to 4096 and 3072 */
+    K_ATTN_W4, K_ATTN_SPLIT, K_ATTN_W4_SPLIT, K_COND_L1, K_COND_L2, K_COND_MOD,
+    /* with K_LN_MOD: width up to 4096 and 3072, without shift and with */
     K_LN_MOD_SHIFT, K_LN_MOD_3072, K_LN_MOD_3072_SHIFT,
     K_COUNT
 };
@@ -1145,7 +1146,11 @@ static wide_plan plan_wide(h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t kst
  * 23-1152 at K = 3072, 4096 and 12288 within 15% (M = 320: 26, 14, 37, 42 us
  * for QKV, out, up and down, against 45, 33, 46 and 62 on the 128 x 256 tiles
  * that these replace; M = 100, K = 4096: 13 against 31). The weights cannot
- * come faster than 5 TB/s. Returns the least time and its mb and s. */
+ * come faster than 5 TB/s. The times are of calls repeated on the same
+ * weights, which a 256 MB cache holds; in a model each layer's come from HBM,
+ * and the short linears take up to 1.4 times as long (out projection, M =
+ * 1152: 32.9 us in the loop of layers, 23.9 alone). Returns the least time
+ * and its mb and s. */
 static double narrow_us(const h3_gpu *g, uint32_t rows, uint32_t cols, uint32_t ksteps,
                         uint32_t max_s, uint32_t *mb_out, uint32_t *s_out) {
     static const double step_us[4] = {0.30, 0.39, 0.56, 0.70}, long_k[4] = {1.35, 1.3, 1.15, 1.0};
@@ -1542,8 +1547,13 @@ static int linear_impl(h3_gpu *g, const qw_linear_desc *d, int no_alloc,
         /* few tile columns: an XCD's share of the ids as they are dealt (one
          * row of each group of 4, every second column) spans no more panels
          * than a range of tiles does, and at long K their slices stay in step
-         * better (down projection, M = 8704, int8 weights, 240 + 264 tiles:
-         * 500 against 530 us; at 36 and more columns a range is 3-7% ahead) */
+         * better. M = 8704 and 12000, us, range / dealt: 12 columns, K = 12288
+         * 497 / 483 and 748 / 718, K = 8192 306 / 303 and 453 / 432, K = 4096
+         * 159 / 160 and 234 / 225; 16 columns level within 1.5%; 20 columns
+         * 783 / 797 and 1106 / 1070; 24 columns 998 / 1033 and 1424 / 1326,
+         * but 484 / 542 at M = 4119 (int8); 32 columns 1269 / 1314; 36 columns
+         * 1459 / 1473 and 1968 / 2043, 3% either way at other row counts. So
+         * the line is at 16 columns, up to where no shape measured loses. */
         a.mix_dealt = a.tiles_n <= 16 && d->k >= 8192;
         const uint32_t n = (a.mix_rows1 + a.mix_rows2) * a.tiles_n;
         if (!launch_step(g, K_GEMM_BF16_STORE_MIX + d->epilogue, dim3(n < g->cus ? n : g->cus),
@@ -1738,8 +1748,8 @@ extern "C" int h3_gpu_mlp_bf16(h3_gpu *g, h3_gpu_tensor *out, const h3_gpu_tenso
  * first) are cut along the keys instead: the blocks past the full rounds
  * (`dp`) in `split` pieces, each a share of the key tiles, that meet in
  * memory (7 us, 1 to 1.5 more a piece, and the partials at 5 TB/s). 1 x 32
- * heads x 4119 rows (544 blocks, 2.1 rounds) 344 -> 295 us; 24 heads, 4096
- * queries of 8512 keys (1.5 rounds) 426 -> 373; 465 of 3323 72 -> 39. */
+ * heads x 4119 rows (544 blocks, 2.1 rounds) 344 -> 278 us; 24 heads, 4096
+ * queries of 8512 keys (1.5 rounds) 421 -> 369; 465 of 3323 71 -> 39. */
 #define QW_ATTN_PART(waves) ((size_t)(waves) * (16 * 1024 + 512)) /* bytes of a piece's partial */
 struct attn_plan {
     int small; /* 128-query blocks */

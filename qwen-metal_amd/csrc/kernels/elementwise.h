@@ -11,11 +11,11 @@
 /* h3_shaders.metal:4767-4815. One wave per row (width <= 4096), four rows
  * per block: lane l owns the 16-byte chunks l, l + 64, ... of the row,
  * held in registers for both passes, and both reductions are wave
- * shuffles (no LDS, no barrier). Large inputs are bound by HBM (4.4 TB/s at
+ * shuffles (no LDS, no barrier). Large inputs are bound by HBM (4.7 TB/s at
  * 8704 x 3072, against 5.0 of a large copy); a few hundred rows by the chain
  * of loads and shuffles, so the modulation is read with the row and not
- * after its statistics (320 x 3072 with shift: 5.1 -> 3.9 us, 8704: 26.6 -> 24.3; 4119 x
- * 4096 without: 13.7 -> 12.7). CH: chunks of 8 per lane, width <= 512 CH. */
+ * after its statistics (320 x 3072 with shift: 5.1 -> 3.9 us, 8704: 24.7 -> 22.8;
+ * 4119 x 4096 without: 13.8 -> 12.8). CH: chunks of 8 per lane, width <= 512 CH. */
 template <int CH, bool SHIFT>
 __device__ __forceinline__ void qw_ln_mod_impl(const qw_ln_mod_args &a) {
 #pragma clang fp contract(off)

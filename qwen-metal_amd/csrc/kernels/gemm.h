@@ -256,7 +256,7 @@ __device__ __forceinline__ void gemm_epilogue_mode(const qw_gemm_args &a, SlabWr
         }
     }
     /* QW_EPI_QKNORM: this wave's 128 columns are one head (tiles start at
-     * multiples of 256); q or k heads get the norm weight of their kind */
+     * multiples of 128); q or k heads get the norm weight of their kind */
     const bool qk_head = EPI == QW_EPI_QKNORM && MODE != 1 && col0 < a.qk_cols;
     float nw[8];
     if (EPI == QW_EPI_QKNORM && qk_head) {

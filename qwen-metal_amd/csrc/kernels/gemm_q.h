@@ -109,13 +109,13 @@ __device__ __forceinline__ void qg_read(const QgCtx &c, const unsigned char *cur
  * direct loads issued back to back, than the loads spread over both
  * sub-steps, and than the read placed before the load); under the 64 MFMAs
  * of sub-step 0 the 16 fragments of sub-step 1 are read, one every 4 MFMAs
- * (256-row tiles; 224-row tiles: 56 MFMAs, 15 loads and reads, the last
- * ones right after their MFMAs). */
+ * (256-row tiles; 224- and 192-row tiles: 56 and 48 MFMAs, 15 and 14 loads
+ * and reads, the last ones right after their MFMAs). */
 template <bool PREV, int MB = 8, int AB = QG_A_BYTES>
 __device__ __forceinline__ void qg_slice(const QgCtx &c, floatx4 (&acc)[8][8], bf16x8 (&pa)[8],
                                          bf16x8 (&pw)[8], const unsigned char *__restrict__ cur,
                                          unsigned char *__restrict__ nxt, uint32_t k_next) {
-    /* MB A blocks of 16 rows per wave (8: 256-row tiles, 7: 224-row
+    /* MB A blocks of 16 rows per wave (8, 7, 6: 256-, 224- and 192-row
      * tiles): 8 MB MFMAs per sub-step; MB + 8 direct loads (A, then W) and
      * fragment reads, those past the one-per-4-MFMAs slots right after */
     constexpr int NM = 8 * MB, NL = MB + 8;
@@ -667,8 +667,8 @@ __device__ __forceinline__ void qg_finish_wave(const qw_gemm_args &a, float *reg
             pld ? pld + poff : nullptr, npart, own);
 }
 
-/* The epilogue of the tile (MB = 8), 224-row tile (MB = 7) or half tile
- * (MB = 4) whose rows start at m0 and columns at n0: each wave's MB x 8
+/* The epilogue of the tile (MB = 8), 224- or 192-row tile (MB = 7, 6) or half
+ * tile (MB = 4) whose rows start at m0 and columns at n0: each wave's MB x 8
  * accumulator blocks. */
 template <int EPI, int INT8, int MB>
 __device__ __forceinline__ void qg_finish_at(const qw_gemm_args &a, unsigned char *lds,
@@ -740,7 +740,8 @@ __device__ __forceinline__ void qg_impl(const qw_gemm_args &a, unsigned char *ld
         qg_finish<EPI, INT8>(a, lds, lds_b, tm, tn, acc);
         return;
     }
-    /* piece of a split tile (k-range-major numbering, as gemm.h) */
+    /* piece of a split tile (numbered k-range-major: all tiles' first ranges,
+     * then all their second ones) */
     uint32_t &ticket = *(uint32_t *)(lds_b + QG_STAGE); /* reserved by QG_ENTRY */
     const uint32_t R = nt - ndp, S = a.split, np = R * S;
     uint32_t q = pid - ndp;
